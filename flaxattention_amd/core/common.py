@@ -12,6 +12,7 @@ and Python ints alike.
 """
 from __future__ import annotations
 
+import ctypes
 import inspect
 import math
 from enum import Enum
@@ -608,7 +609,7 @@ def dense_mask_on_device(fn: Callable, B: int, H: int, Q: int, KV: int, device,
     out-of-range gather yields under XLA.
 
     `b_range` / `h_range` / `q_range` restrict the evaluation to a slab (batches [b0,b1), heads [h0,h1), query
-    rows [q0,q1)); the result then covers that slab only."""
+    rows [q0,q1)); the result then covers that slab only (with `q_range`: expanded to it)."""
     b0, b1 = b_range or (0, B)
     h0, h1 = h_range or (0, H)
     q_lo, q_hi = q_range or (0, Q)
@@ -624,17 +625,9 @@ def dense_mask_on_device(fn: Callable, B: int, H: int, Q: int, KV: int, device,
 
     Qr, KVr = (Q, KV) if real is None else (min(real[0], Q), min(real[1], KV))
     if q_range is not None:
-        # a slab of rows: the same three regions, cut to [q_lo, q_hi)
-        clamp = not _index_arithmetic_only(fn)
-        m = torch.zeros((b1 - b0, h1 - h0, q_hi - q_lo, KV), dtype=torch.bool, device=device)
-        q_mid = min(max(Qr, q_lo), q_hi)   # rows [q_lo, q_mid) are real, [q_mid, q_hi) lie past the end
-        if q_mid > q_lo:
-            m[:, :, :q_mid - q_lo, :KVr] = grid(device, (q_lo, q_mid), (0, KVr))
-            if KVr < KV:
-                m[:, :, :q_mid - q_lo, KVr:] = grid(device, (q_lo, q_mid), (KVr, KV), clamp)
-        if q_hi > q_mid:
-            m[:, :, q_mid - q_lo:, :] = grid(device, (q_mid, q_hi), (0, KV), clamp)
-        return m
+        # one call for the whole slab: inside the real lengths a clamp changes no index
+        clamp = (q_hi > Qr or KV > KVr) and not _index_arithmetic_only(fn)
+        return torch.broadcast_to(grid(device, (q_lo, q_hi), (0, KV), clamp), (b1 - b0, h1 - h0, q_hi - q_lo, KV))
     core = grid(device, (0, Qr), (0, KVr))
     if Qr == Q and KVr == KV:
         return core
@@ -752,7 +745,7 @@ _mask_cache: dict = {}
 
 
 _SLAB_ELEMS = 1 << 24          # mask entries evaluated at a time (the callable's own temporaries scale with this)
-_FIT_ELEMS = 1 << 25           # entries of the first rows on which band parameters are fitted
+_ONE_PIECE_ELEMS = 1 << 25     # a grid of all (batch, head) up to this size is evaluated by one call of the callable
 _EAGER_T_BYTES = 64 << 20      # bitmaps up to this size get their query-packed copy right away
 
 
@@ -781,40 +774,97 @@ def _band_equals_bitmap(band: MaskMod, words: torch.Tensor, rows: int) -> bool:
     return True
 
 
+def _pack_slab(m: torch.Tensor, q0: int, at: int, bits: torch.Tensor, bits_t: Optional[torch.Tensor], blk: torch.Tensor) -> None:
+    """Write a slab of evaluated mask, bool [nb, nh, rows, KVp] (any strides), as rows q0 .. of the maps at, at + 1, ...
+    of bits [n, Qp, W], bits_t [n, KVp, Qp/32] (or None) and blk [n, Qp/32, W]."""
+    nb, nh, rows, KVp = m.shape
+    Qp = bits.shape[1]
+    if m.is_cuda:
+        with torch.cuda.device(m.device):
+            rc = _lib.lib().flexattn_pack_mask(
+                m.data_ptr(), (ctypes.c_int64 * 4)(*m.stride()), nb, nh, q0, rows, Qp, KVp, bits[at].data_ptr(),
+                bits_t[at].data_ptr() if bits_t is not None else None, blk[at].data_ptr(),
+                torch.cuda.current_stream(m.device).cuda_stream)
+        _lib.check(rc, "flexattn_pack_mask")
+        return
+    m = m.reshape(nb * nh, rows, KVp)
+    bits[at:at + nb * nh, q0:q0 + rows] = pack_bits(m)
+    blk[at:at + nb * nh, q0 // 32:(q0 + rows) // 32] = block_classes(m)
+    if bits_t is not None:
+        bits_t[at:at + nb * nh, :, q0 // 32:(q0 + rows) // 32] = pack_bits(m.transpose(1, 2).contiguous())
+
+
+def _fit_bitmaps(bits: torch.Tensor) -> Tuple[bool, Optional[MaskMod]]:
+    """(every map of bits [n, Qp, W] is the same, the band mask it then is or None)."""
+    n, Qp, W = bits.shape
+    if bits.is_cuda:
+        fit = torch.empty(6, dtype=torch.int32, device=bits.device)
+        with torch.cuda.device(bits.device):
+            rc = _lib.lib().flexattn_bitmap_fit(bits.data_ptr(), n, Qp, W * 32, fit.data_ptr(),
+                                                torch.cuda.current_stream(bits.device).cuda_stream)
+        _lib.check(rc, "flexattn_bitmap_fit")
+        lo, differs, d, kv, bad_sink, bad_plain = fit.tolist()
+        if differs:
+            return False, None
+        if lo == INT_MAX:
+            return True, MaskMod(INT_MAX, INT_MAX, -1)
+        if lo <= -(W * 32 - 1):
+            lo = INT_MIN
+        hi, sink = (INT_MAX, -1) if d == INT_MAX else (d - 1, kv - 1)
+        return True, MaskMod(lo, hi, sink) if not bad_sink else MaskMod(lo, hi, -1) if not bad_plain else None
+    if not bool((bits == bits[:1]).all()):
+        return False, None
+    band = _fit_band(unpack_bits(bits[0], W * 32))
+    return True, band if band is not None and _band_equals_bitmap(band, bits[0], Qp) else None
+
+
 def _lower_mask_callable(fn: Callable, B: int, H: int, Q: int, KV: int, Qp: int, KVp: int, device, real) -> MaskMod:
-    """Evaluate the callable over the padded index grid one (batch, head, rows) slab at a time -- the dense
-    [B,H,Q,KV] mask is never held -- and pack each slab straight into the bitmap words and the classes of its
-    32 x 32 blocks.  If every (batch, head) turns out to carry the same mask, it is fitted to the band form or kept
-    as one broadcast bitmap."""
+    """Evaluate the callable over the padded index grid and pack it into the bitmap words and the classes of its
+    32 x 32 blocks: in one piece where the grid of all (batch, head) is small, else slab by slab -- whole maps while
+    they are small, rows of one map otherwise -- so that the dense [B,H,Q,KV] mask is never held.  If every
+    (batch, head) turns out to carry the same mask, it is fitted to the band form, and every word checked against it, or
+    kept as one broadcast bitmap."""
     name = getattr(fn, "__name__", "mask_mod")
     real = real or (Q, KV)
-    Bm, Hm = _bh_extents(fn, B, H, device)
-    rows = max(128, min(Qp, (_SLAB_ELEMS // KVp) // 128 * 128))
+    device = torch.device(device)
     W = KVp // 32
-    bits = torch.empty((Bm, Hm, Qp, W), dtype=torch.int32, device=device)
-    blk = torch.empty((Bm, Hm, Qp // 32, KVp // 32), dtype=torch.int8, device=device)
-    same = True          # every (batch, head) seen so far equals (0, 0)
-    for b in range(Bm):
-        for h in range(Hm):
-            for q0 in range(0, Qp, rows):
-                q1 = min(q0 + rows, Qp)
-                m = dense_mask_on_device(fn, B, H, Qp, KVp, device, real=real, b_range=(b, b + 1), h_range=(h, h + 1),
-                                         q_range=(q0, q1))[0, 0]
-                bits[b, h, q0:q1] = pack_bits(m)
-                blk[b, h, q0 // 32:q1 // 32] = block_classes(m)
-                if same and (b or h):
-                    same = bool(torch.equal(bits[b, h, q0:q1], bits[0, 0, q0:q1]))
-    if same:
-        # the closed band form: parameters are fitted on the first rows (_FIT_ELEMS entries) and then
-        # checked against EVERY word of the bitmap, slab by slab; a band whose window is longer than the fitted rows
-        # fails that check and stays a bitmap
-        bits, blk = bits[:1, :1].contiguous(), blk[:1, :1].contiguous()   # (lets go of the per-(batch, head) arrays)
-        fit_rows = min(Qp, max(128, (_FIT_ELEMS // KVp) // 128 * 128))
-        band = _fit_band(unpack_bits(bits[0, 0, :fit_rows], KVp))
-        if band is not None and _band_equals_bitmap(band, bits[0, 0], rows):
-            band.__name__ = name
-            return band
-    spec = MaskMod(name=name, bits=bits, fn=fn, blk=blk)
+    whole = None
+    if B * H * Qp * KVp <= _ONE_PIECE_ELEMS:
+        # the result's own shape tells which extents it has; a probe of one position would cost ten launches more
+        whole = dense_mask_on_device(fn, B, H, Qp, KVp, device, real=real, b_range=(0, B), h_range=(0, H), q_range=(0, Qp))
+        Bm, Hm = (n if whole.stride(i) else 1 for i, n in enumerate((B, H)))
+    else:
+        Bm, Hm = _bh_extents(fn, B, H, device)
+    n_maps = Bm * Hm
+    bits = torch.empty((n_maps, Qp, W), dtype=torch.int32, device=device)
+    blk = torch.empty((n_maps, Qp // 32, W), dtype=torch.int8, device=device)
+    bits_t = None
     if bits.numel() * 4 <= _EAGER_T_BYTES:
+        bits_t = torch.empty((n_maps, KVp, Qp // 32), dtype=torch.int32, device=device)
+    if whole is not None:
+        _pack_slab(whole[:Bm, :Hm], 0, 0, bits, bits_t, blk)
+        del whole
+    else:
+        rows = max(128, min(Qp, (_SLAB_ELEMS // KVp) // 128 * 128))
+        heads = max(1, min(Hm, _SLAB_ELEMS // (Qp * KVp)))
+        for b in range(Bm):
+            for h in range(0, Hm, heads):
+                h1 = min(h + heads, Hm)
+                for q0 in range(0, Qp, rows):
+                    m = dense_mask_on_device(fn, B, H, Qp, KVp, device, real=real, b_range=(b, b + 1), h_range=(h, h1),
+                                             q_range=(q0, min(q0 + rows, Qp)))
+                    _pack_slab(m, q0, b * Hm + h, bits, bits_t, blk)
+    same, band = _fit_bitmaps(bits)
+    if band is not None:
+        band.__name__ = name
+        return band
+    if same:   # one broadcast bitmap (the copies let go of the per-(batch, head) arrays)
+        Bm = Hm = 1
+        if n_maps > 1:
+            bits, blk = bits[:1].clone(), blk[:1].clone()
+            bits_t = bits_t[:1].clone() if bits_t is not None else None
+    spec = MaskMod(name=name, bits=bits.view(Bm, Hm, Qp, W), fn=fn, blk=blk.view(Bm, Hm, Qp // 32, W),
+                   bits_t=bits_t.view(Bm, Hm, KVp, Qp // 32) if bits_t is not None else None)
+    if bits_t is None and bits.numel() * 4 <= _EAGER_T_BYTES:
         spec.ensure_transposed()
     return spec

@@ -7,6 +7,8 @@
 // stable partition (selected ids ascending, then the rest ascending -- the
 // order a stable descending argsort of a 0/1 row gives).  The dense mask is
 // never materialised.  All outputs are integers and bit-exact.
+#include <climits>
+
 #include "flex_common.cuh"
 
 namespace flex {
@@ -112,6 +114,130 @@ __global__ __launch_bounds__(256) void order_rows_kernel(OrderJobs jobs, long lo
   }
 }
 
+// ---- lowering of a mask given as evaluated booleans ----
+// A callable's mask arrives as one byte per position (any strides, 0 where it broadcasts) and leaves as what the
+// attention kernels read: words packed along the keys, words packed along the queries, and the class of every 32 x 32
+// block.  Bound by the read of the bytes: every byte is loaded once and serves all three outputs (a wave takes 32
+// rows x 64 keys; a row's 64 bytes become two words through one ballot, a lane collects its own key's column and the
+// columns' words give the classes).  It stands for some twenty elementwise and reduction launches per slab (two of
+// them reductions over innermost extents of 8 and 32, 38 us each at 3072 x 3072): [2,1,3072,3072] with both packings
+// and classes 10.4 us (18.9 MB read) against 0.42 ms of device time.
+constexpr int kPackRows = 32, kPackCols = 64;
+
+__global__ __launch_bounds__(256) void pack_mask_kernel(const uint8_t* __restrict__ mask, int64_t sb, int64_t sh, int64_t sq,
+                                                        int64_t skv, int nh, int q_lo, int Qp, int KVp,
+                                                        uint32_t* __restrict__ bits, uint32_t* __restrict__ bits_t,
+                                                        int8_t* __restrict__ blk) {
+  const int lane = threadIdx.x & 63;
+  const int kv0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * kPackCols;
+  if (kv0 >= KVp) return;
+  const int r0 = blockIdx.y * kPackRows, map = blockIdx.z;
+  const uint8_t* src = mask + (map / nh) * sb + (map % nh) * sh + (int64_t)r0 * sq + (int64_t)(kv0 + lane) * skv;
+  uint8_t seen[kPackRows];
+#pragma unroll
+  for (int r = 0; r < kPackRows; r++) seen[r] = src[(int64_t)r * sq];
+  uint32_t column = 0;           // this lane's key, bit r = row r0 + r
+  unsigned long long row = 0;    // lane r: the 64 keys of row r0 + r
+#pragma unroll
+  for (int r = 0; r < kPackRows; r++) {
+    const unsigned long long ballot = __ballot(seen[r] != 0);
+    column |= (seen[r] != 0 ? 1u : 0u) << r;
+    if (lane == r) row = ballot;
+  }
+  const int W = KVp >> 5, Wq = Qp >> 5, qb = (q_lo + r0) >> 5;
+  if (lane < kPackRows)
+    *(unsigned long long*)(bits + ((int64_t)map * Qp + q_lo + r0 + lane) * W + (kv0 >> 5)) = row;
+  if (bits_t) bits_t[((int64_t)map * KVp + kv0 + lane) * Wq + qb] = column;
+  const unsigned long long all = __ballot(column == 0xffffffffu), none = __ballot(column == 0);
+  if ((lane & 31) == 0) {
+    const uint32_t a = (uint32_t)(all >> lane), n = (uint32_t)(none >> lane);
+    blk[((int64_t)map * Wq + qb) * W + ((kv0 + lane) >> 5)] = a == 0xffffffffu ? 1 : n == 0xffffffffu ? 2 : 0;
+  }
+}
+
+// Band fit of packed maps: d = q - kv;  visible = (d >= lo) && (d <= hi || kv <= sink).  Three sweeps over the words, a
+// word at a time, each sweep's minima read by the next one on the device, so that the host waits once, for the verdict
+// (fitting and checking on the host's side of the stream took up to six waits):
+//   fit[0] lowest d of a visible entry (INT_MAX: none)   fit[1] 1 where some map differs from the first
+//   fit[2] lowest d, fit[3] lowest kv of a hidden entry with d >= lo (INT_MAX: none)
+//   fit[4] / fit[5] 1 where the band with sink = fit[3] - 1 / without sink fails to reproduce the first map
+__device__ __forceinline__ uint32_t bits_up_to(long long last, int kv0) {   // bits of the keys kv0 .. last
+  const long long n = last - kv0 + 1;
+  return n >= 32 ? 0xffffffffu : n <= 0 ? 0u : (1u << n) - 1u;
+}
+
+__device__ __forceinline__ int fit_lo(const int32_t* fit, int KVp) {
+  return fit[0] <= -(KVp - 1) ? INT_MIN : fit[0];   // hides nothing ahead of the row
+}
+
+// At most kFitBlocks workgroups, each ending in one atomic (or, for a flag, plain stores of the same 1): one per wave of
+// 1024 workgroups queued up on the one address and took 70 to 88 us a sweep at [2,3072,3072], against 17 us this way.
+constexpr int kFitThreads = 512, kFitBlocks = 256;
+
+__device__ __forceinline__ void block_min_to(int v, int32_t* out) {
+  __shared__ int wave_min[kFitThreads / 64];
+  for (int off = 32; off > 0; off >>= 1) v = min(v, __shfl_xor(v, off, 64));
+  __syncthreads();   // (an earlier use has been read)
+  if ((threadIdx.x & 63) == 0) wave_min[threadIdx.x >> 6] = v;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int w = 1; w < kFitThreads / 64; w++) v = min(v, wave_min[w]);
+    if (v != INT_MAX) atomicMin(out, v);
+  }
+}
+
+__global__ void fit_init_kernel(int32_t* fit) {
+  const int i = threadIdx.x;
+  if (i < 6) fit[i] = (i == 0 || i == 2 || i == 3) ? INT_MAX : 0;
+}
+
+__global__ __launch_bounds__(kFitThreads) void fit_visible_kernel(const uint32_t* __restrict__ bits, long long words, int W,
+                                                                  long long n_maps, int32_t* fit) {
+  int lo = INT_MAX;
+  bool differs = false;
+  for (long long i = (long long)blockIdx.x * kFitThreads + threadIdx.x; i < words; i += (long long)gridDim.x * kFitThreads) {
+    const uint32_t w = bits[i];
+    const int q = (int)(i / W), kv0 = (int)(i % W) * 32;
+    if (w) lo = min(lo, q - (kv0 + 31 - __clz((int)w)));
+    for (long long m = 1; m < n_maps; m++) differs |= bits[m * words + i] != w;
+  }
+  block_min_to(lo, fit);
+  if (differs) fit[1] = 1;
+}
+
+// (the sweeps below have nothing to answer once the maps are known to differ)
+__global__ __launch_bounds__(kFitThreads) void fit_hidden_kernel(const uint32_t* __restrict__ bits, long long words, int W, int32_t* fit) {
+  if (fit[1]) return;
+  const long long lo = fit_lo(fit, W * 32);
+  int d_min = INT_MAX, kv_min = INT_MAX;
+  for (long long i = (long long)blockIdx.x * kFitThreads + threadIdx.x; i < words; i += (long long)gridDim.x * kFitThreads) {
+    const int q = (int)(i / W), kv0 = (int)(i % W) * 32;
+    const uint32_t hidden = ~bits[i] & bits_up_to(q - lo, kv0);
+    if (hidden) {
+      d_min = min(d_min, q - (kv0 + 31 - __clz((int)hidden)));
+      kv_min = min(kv_min, kv0 + __ffs((int)hidden) - 1);
+    }
+  }
+  block_min_to(d_min, fit + 2);
+  block_min_to(kv_min, fit + 3);
+}
+
+__global__ __launch_bounds__(kFitThreads) void fit_check_kernel(const uint32_t* __restrict__ bits, long long words, int W, int32_t* fit) {
+  if (fit[1]) return;
+  const long long lo = fit_lo(fit, W * 32);
+  const bool gap = fit[2] != INT_MAX;
+  const long long hi = gap ? (long long)fit[2] - 1 : INT_MAX, sink = gap ? fit[3] - 1 : -1;
+  bool bad_sink = false, bad_plain = false;
+  for (long long i = (long long)blockIdx.x * kFitThreads + threadIdx.x; i < words; i += (long long)gridDim.x * kFitThreads) {
+    const int q = (int)(i / W), kv0 = (int)(i % W) * 32;
+    const uint32_t w = bits[i], ahead = bits_up_to(q - lo, kv0), near = ~bits_up_to(q - hi - 1, kv0);
+    bad_sink |= (ahead & (near | bits_up_to(sink, kv0))) != w;
+    bad_plain |= (ahead & near) != w;
+  }
+  if (bad_sink) fit[4] = 1;
+  if (bad_plain) fit[5] = 1;
+}
+
 }  // namespace flex
 
 using namespace flex;
@@ -170,5 +296,50 @@ extern "C" int flexattn_block_mask_build(const FlexMask* mask, int32_t B, int32_
   }
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) { flex_set_error("block_mask_build: launch failed: %s", hipGetErrorString(e)); return 2; }
+  return 0;
+}
+
+extern "C" int flexattn_pack_mask(const uint8_t* mask, const int64_t* strides, int32_t nb, int32_t nh, int32_t q_lo,
+                                  int32_t rows, int32_t Qp, int32_t KVp, int32_t* bits, int32_t* bits_t, int8_t* blk,
+                                  flexattn_stream_t stream_) {
+  hipStream_t stream = (hipStream_t)stream_;
+  if (!mask || !strides || !bits || !blk) { flex_set_error("pack_mask: null argument"); return 1; }
+  if (nb <= 0 || nh <= 0 || rows <= 0 || q_lo < 0 || Qp <= 0 || KVp <= 0 || Qp % 128 || KVp % 128 || q_lo % 32 || rows % 32 ||
+      (long long)q_lo + rows > Qp) {
+    flex_set_error("pack_mask: bad extents nb=%d nh=%d q_lo=%d rows=%d Qp=%d KVp=%d", nb, nh, q_lo, rows, Qp, KVp);
+    return 1;
+  }
+  const int most_rows = 65535 * kPackRows;   // blockIdx.y
+  if ((long long)nb * nh > 65535 || rows > most_rows) {
+    flex_set_error("pack_mask: grid too large (nb*nh=%lld, rows=%d)", (long long)nb * nh, rows);
+    return 1;
+  }
+  const int cols = 4 * kPackCols;
+  hipLaunchKernelGGL(pack_mask_kernel, dim3((KVp + cols - 1) / cols, rows / kPackRows, nb * nh), dim3(256), 0, stream, mask,
+                     strides[0], strides[1], strides[2], strides[3], nh, q_lo, Qp, KVp, (uint32_t*)bits, (uint32_t*)bits_t, blk);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) { flex_set_error("pack_mask: launch failed: %s", hipGetErrorString(e)); return 2; }
+  return 0;
+}
+
+extern "C" int flexattn_bitmap_fit(const int32_t* bits, int32_t n_maps, int32_t Qp, int32_t KVp, int32_t* fit,
+                                   flexattn_stream_t stream_) {
+  hipStream_t stream = (hipStream_t)stream_;
+  if (!bits || !fit) { flex_set_error("bitmap_fit: null argument"); return 1; }
+  if (n_maps <= 0 || Qp <= 0 || KVp <= 0 || KVp % 32) {
+    flex_set_error("bitmap_fit: bad extents n_maps=%d Qp=%d KVp=%d", n_maps, Qp, KVp);
+    return 1;
+  }
+  const int W = KVp / 32;
+  const long long words = (long long)Qp * W;
+  const long long want = (words + kFitThreads - 1) / kFitThreads;
+  const unsigned blocks = (unsigned)(want < kFitBlocks ? want : kFitBlocks);
+  const uint32_t* w = (const uint32_t*)bits;
+  hipLaunchKernelGGL(fit_init_kernel, dim3(1), dim3(64), 0, stream, fit);
+  hipLaunchKernelGGL(fit_visible_kernel, dim3(blocks), dim3(kFitThreads), 0, stream, w, words, W, (long long)n_maps, fit);
+  hipLaunchKernelGGL(fit_hidden_kernel, dim3(blocks), dim3(kFitThreads), 0, stream, w, words, W, fit);
+  hipLaunchKernelGGL(fit_check_kernel, dim3(blocks), dim3(kFitThreads), 0, stream, w, words, W, fit);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess) { flex_set_error("bitmap_fit: launch failed: %s", hipGetErrorString(e)); return 2; }
   return 0;
 }

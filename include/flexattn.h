@@ -204,6 +204,21 @@ int flexattn_block_mask_build(const FlexMask* mask, int32_t B, int32_t H,
                               int32_t* full_q_num, int32_t* full_q_idx,
                               void* workspace, flexattn_stream_t stream);
 
+/* Lowering of a mask that was evaluated to booleans (one byte per position, nonzero = visible): rows
+ * [q_lo, q_lo + rows) of nb x nh maps, byte (b, h, r, kv) at mask + b*strides[0] + h*strides[1] + r*strides[2] +
+ * kv*strides[3] (r counted from q_lo, kv < KVp; a stride may be 0), into FlexMask's arrays of the same nb*nh
+ * consecutive maps: bits [., Qp, KVp/32], bits_t [., KVp, Qp/32] (may be NULL), blk [., Qp/32, KVp/32].  Qp and KVp are
+ * multiples of 128, q_lo and rows of 32.  Stands for the dense mask the reference keeps
+ * (flaxattention/core/blockmask.py:277-322). */
+int flexattn_pack_mask(const uint8_t* mask, const int64_t* strides, int32_t nb, int32_t nh, int32_t q_lo, int32_t rows,
+                       int32_t Qp, int32_t KVp, int32_t* bits, int32_t* bits_t, int8_t* blk, flexattn_stream_t stream);
+
+/* Whether n_maps packed maps [n_maps, Qp, KVp/32] are one band mask: with d = q - kv, writes to fit (6 words on the
+ * device) the lowest d of a visible entry of the first map (INT32_MAX: none), whether another map differs from it, the
+ * lowest d and the lowest kv of its hidden entries with d >= lo (INT32_MAX: none), and whether the bands
+ * (lo, hi = fit[2] - 1, sink = fit[3] - 1) and (lo, hi, no sink) miss any entry of it. */
+int flexattn_bitmap_fit(const int32_t* bits, int32_t n_maps, int32_t Qp, int32_t KVp, int32_t* fit, flexattn_stream_t stream);
+
 /* Forward.  With FLEX_PARITY and lse2 == NULL the log-sum-exp that the second pass reads is kept
  * in `workspace` (flexattn_fwd_workspace_bytes); otherwise workspace may be NULL.  A workspace
  * of that size also lets the matrix-core kernels split calls with few query rows against many

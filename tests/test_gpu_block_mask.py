@@ -177,3 +177,60 @@ def test_head_and_batch_dependent_callable_at_config4_size(dev):
         for f in ("kv_num_blocks", "kv_indices", "full_kv_num_blocks", "full_kv_indices", "q_num_blocks", "q_indices",
                   "full_q_num_blocks", "full_q_indices"):
             assert (getattr(bm, f)[b0, h0].cpu().numpy() == ref[f][0, 0]).all(), (f, b0, h0)
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 128, 128), (2, 3, 128, 384), (1, 2, 384, 128), (3, 1, 256, 640)])
+def test_packed_bitmap_equals_torch_formulas(dev, shape):
+    """The packing kernel (words along the keys, words along the queries, 32 x 32 classes) against the torch formulas on
+    the CPU, bit for bit: slabs of rows, non-contiguous and broadcast inputs, all-set / all-clear / mixed blocks."""
+    from flaxattention_amd.core.common import _pack_slab, block_classes, pack_bits
+    nb, nh, Q, KV = shape
+    print("case pack", shape, flush=True)
+    g = torch.Generator().manual_seed(Q + KV)
+    m = torch.rand(shape, generator=g) < 0.3
+    m[..., :64, :96] = True
+    m[..., 32:64, 32:64] = False
+    m[..., 96:, 64:96] = False
+    forms = {"contiguous": m.to(dev), "transposed": m.transpose(2, 3).contiguous().to(dev).transpose(2, 3),
+             "every other": torch.stack([m, ~m], -1).reshape(nb, nh, Q, 2 * KV).to(dev)[..., ::2],
+             "rows broadcast": m[:, :, :1].to(dev).expand(shape), "maps broadcast": m[:1, :1].to(dev).expand(shape)}
+    for name, md in forms.items():
+        want = md.cpu().reshape(nb * nh, Q, KV)
+        for step in (Q, 128):
+            bits = torch.full((nb * nh + 1, Q, KV // 32), -7, dtype=torch.int32, device=dev)
+            bits_t = torch.full((nb * nh + 1, KV, Q // 32), -7, dtype=torch.int32, device=dev)
+            blk = torch.full((nb * nh + 1, Q // 32, KV // 32), -7, dtype=torch.int8, device=dev)
+            for q0 in range(0, Q, step):
+                _pack_slab(md[:, :, q0:q0 + step], q0, 1, bits, bits_t, blk)
+            assert torch.equal(bits[1:].cpu(), pack_bits(want)), name
+            assert torch.equal(bits_t[1:].cpu(), pack_bits(want.transpose(1, 2).contiguous())), name
+            assert torch.equal(blk[1:].cpu(), block_classes(want)), name
+            assert all(bool((t[0] == -7).all()) for t in (bits, bits_t, blk)), name   # nothing written ahead of its map
+
+
+@pytest.mark.parametrize("Q,KV", [(128, 128), (256, 384), (384, 128)])
+def test_band_fit_of_packed_bitmaps(dev, Q, KV):
+    """The fit on the device finds exactly the bands, on every entry: each verdict against the entries themselves."""
+    from flaxattention_amd.core.common import INT_MAX, INT_MIN, MaskMod, _fit_bitmaps, pack_bits
+    print("case fit", Q, KV, flush=True)
+    q, kv = torch.arange(Q, dtype=torch.int32).reshape(Q, 1), torch.arange(KV, dtype=torch.int32).reshape(1, KV)
+    zero = torch.zeros((), dtype=torch.int32)
+    bands = [(lo, hi, sink) for lo in (INT_MIN, -KV + 1, -5, 0, 31, Q - 1, Q, INT_MAX)
+             for hi, sink in ((INT_MAX, -1), (Q - 1, -1), (Q - 2, 0), (40, -1), (40, 3), (33, 32), (0, 64), (-3, 5))]
+    dense = lambda m: torch.broadcast_to(m(zero, zero, q, kv), (Q, KV))
+    for b in bands:
+        m = dense(MaskMod(*b))
+        same, got = _fit_bitmaps(pack_bits(m)[None].to(dev))
+        assert same and got is not None and torch.equal(dense(got), m), b
+    m = dense(MaskMod(0, 40, 3))
+    words = pack_bits(m)
+    for r, c in ((0, 0), (Q - 1, KV - 1), (Q // 2, 0), (Q // 2, KV - 1), (Q - 1, 7)):   # one entry off: no band any more
+        off = m.clone()
+        off[r, c] = ~off[r, c]
+        same, got = _fit_bitmaps(pack_bits(off)[None].to(dev))
+        assert same and (got is None or torch.equal(dense(got), off)), (r, c)
+        assert _fit_bitmaps(torch.stack([words, words, pack_bits(off)]).to(dev)) == (False, None), (r, c)
+    same, got = _fit_bitmaps(torch.stack([words, words]).to(dev))
+    assert same and torch.equal(dense(got), m)
+    g = torch.Generator().manual_seed(Q)
+    assert _fit_bitmaps(pack_bits(torch.rand(Q, KV, generator=g) < 0.5)[None].to(dev)) == (True, None)
