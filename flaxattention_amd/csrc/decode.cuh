@@ -10,21 +10,27 @@ constexpr int kStep = 32;  // KV rows per wave step
 // PASS selects the numerics, as in the forward kernel:
 //   kDecOnePass  online softmax; the unnormalised P is rounded to the input dtype for the P.V product
 //   kDecLse      first pass of the parity numerics: per split only (m, l), no V is read
-//   kDecNorm     second pass: P = 2^(x - lse2) with the merged log-sum-exp of the first pass is the normalised
-//                probability, rounded to the input dtype and multiplied into V; the splits' partial outputs simply
-//                add up (written with m = 0 and l = 1 for split 0, l = 0 for the others, so that the same combine
-//                kernel sums them)
-enum { kDecOnePass = 0, kDecLse = 1, kDecNorm = 2 };
+//   kDecNorm     second pass: P = 2^(x - lse2) with the log-sum-exp of the first pass (every workgroup merges the
+//                splits' (m, l) of its columns itself: the launch of a merge kernel in between cost 4.7 us) is the
+//                normalised probability, rounded to the input dtype and multiplied into V; the splits' partial outputs
+//                simply add up
+//   kDecLseKeep / kDecNormKept   the same two passes with the scores kept in between: S is rounded to the input dtype in
+//                these numerics, so 16 bits hold it exactly and the second pass reads 64 bytes per column and step
+//                where it would read the step's K rows again (64 * D bytes) and multiply them again.  Bound by HBM:
+//                a pass of K and a pass of V instead of K, K and V.
+enum { kDecOnePass = 0, kDecLse = 1, kDecNorm = 2, kDecLseKeep = 3, kDecNormKept = 4 };
 template <typename T, int D, int KIND, bool ROUND_S, int NB, int PASS = kDecOnePass>
 __global__ __launch_bounds__(256, D >= 192 ? 1 : NB == 1 ? (D == 64 ? 3 : 2) : (D == 64 ? 2 : 1)) void decode_split_kernel(FlexAttnParams p, const T* __restrict__ q,
                                                             const T* __restrict__ k, const T* __restrict__ v,
                                                             float* __restrict__ o_part, float* __restrict__ ml_part,
-                                                            int splits, const float* __restrict__ lse_in) {
+                                                            int splits, float* __restrict__ lse_out, T* __restrict__ kept) {
   typedef typename Frag<T>::vec8 vec8;
   // D = 256 serves one column block: the two V strips of the four waves are 128 KB of the 160 KB of LDS, which leaves
   // no room for a second block's Q fragments, and its registers (64 for Q, 64 for K, 128 for O) no room to keep them;
   // D = 192 likewise runs one wave per SIMD with one column block
   static_assert(D == 64 || D == 128 || ((D == 192 || D == 256) && NB == 1), "decode_split_kernel: head size / column blocks");
+  constexpr bool kLse = PASS == kDecLse || PASS == kDecLseKeep, kNorm = PASS == kDecNorm || PASS == kDecNormKept;
+  static_assert(NB == 1 || (PASS != kDecLseKeep && PASS != kDecNormKept), "scores are kept for one column block");
   constexpr int DS = D / 16, DB = D / 32, ROWE = D + 8, CPR = D / 8;
   // a strip is kStep * CPR chunks, 64 per wave-wide fetch instruction, laid down one after the other (at D = 192 an
   // instruction ends in the middle of a row)
@@ -124,6 +130,11 @@ __global__ __launch_bounds__(256, D >= 192 ? 1 : NB == 1 ? (D == 64 ? 3 : 2) : (
   // masked out and their P is 0, so what they hold does not matter as long as
   // it is finite.
   const int last = p.Lkv - 1;
+  // kept scores: [b, hk, step, column, lane half] x 16 values (the accumulator rows a lane holds)
+  const int kept_step = ncols * kStep;
+  T* kept_bh = nullptr;
+  if constexpr (PASS == kDecLseKeep || PASS == kDecNormKept)
+    kept_bh = kept + ((int64_t)b * p.Hkv + hk) * ((p.Lkv + kStep - 1) / kStep) * kept_step + (col_ok[0] ? i32 : 0) * kStep + 16 * g;
   vec8 kfA[DS], kfB[DS];  // two sets of K registers, named so that they stay in registers (kfB unused at DEPTH 1)
   T* Vw = reinterpret_cast<T*>(vs_red) + w * NSTG * kStripElems;
   // V first, K last: loads return in order, so once the K registers of a step have arrived (the
@@ -131,7 +142,7 @@ __global__ __launch_bounds__(256, D >= 192 ? 1 : NB == 1 ? (D == 64 ? 3 : 2) : (
   auto load_step = [&](vec8 (&kfr)[DS], int kv0, int stage) {
     const int lim = last - kv0;  // last valid row of this step, relative
     const T* vp = vbase + (int64_t)kv0 * vs2;
-    if constexpr (PASS != kDecLse) {
+    if constexpr (!kLse) {
 #pragma unroll
       for (int j = 0; j < NVI; j++) {
         const int c = 64 * j + lane, r = c / CPR;   // the strip row and position this lane fills
@@ -139,6 +150,13 @@ __global__ __launch_bounds__(256, D >= 192 ? 1 : NB == 1 ? (D == 64 ? 3 : 2) : (
         __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)vg,
                                          (__attribute__((address_space(3))) void*)(Vw + stage * kStripElems + 512 * j), 16, 0, 0);
       }
+    }
+    if constexpr (PASS == kDecNormKept) {
+      // in place of the K rows: this lane's 16 rounded scores of the step
+      const T* sp = kept_bh + (int64_t)(kv0 / kStep) * kept_step;
+      kfr[0] = *reinterpret_cast<const vec8*>(sp);
+      kfr[1] = *reinterpret_cast<const vec8*>(sp + 8);
+      return;
     }
     const T* kp = kbase + (int64_t)kv0 * ks2 + min(i32, lim) * (int)ks2 + 8 * g;
 #pragma unroll
@@ -165,9 +183,23 @@ __global__ __launch_bounds__(256, D >= 192 ? 1 : NB == 1 ? (D == 64 ? 3 : 2) : (
     sm[nb].init(p.score, p.scale, col_h[nb]);
     m_run[nb] = -INFINITY;
     l_run[nb] = 0.f;
-    if constexpr (PASS == kDecNorm) {
-      // the merged log-sum-exp of the first pass is the fixed reference; a column without visible keys gets +inf (P = 0)
-      const float l2 = lse_in[((int64_t)b * p.Hq + col_h[nb]) * p.Lq + col_q[nb]];
+    if constexpr (kNorm) {
+      // the log-sum-exp of the first pass is the fixed reference; a column without visible keys gets +inf (P = 0).
+      // The two lane halves of a column take alternate splits.
+      const int64_t all_rows = (int64_t)p.B * p.Hq * p.Lq, row = ((int64_t)b * p.Hq + col_h[nb]) * p.Lq + col_q[nb];
+      const float2* ml = reinterpret_cast<const float2*>(ml_part) + row;
+      float mm = -INFINITY, ll = 0.f;
+#pragma unroll 4
+      for (int sp = g; sp < splits; sp += 2) mm = fmaxf(mm, ml[sp * all_rows].x);
+      mm = xhalf_max(mm);
+#pragma unroll 4
+      for (int sp = g; sp < splits; sp += 2) {
+        const float2 part = ml[sp * all_rows];
+        ll += part.x == -INFINITY ? 0.f : part.y * fast_exp2(part.x - mm);
+      }
+      ll = xhalf_sum(ll);
+      const float l2 = ll > 0.f ? mm + log2f(ll) : -INFINITY;
+      if (lse_out && split == 0 && w == 0 && g == 0 && col_ok[nb]) lse_out[row] = l2;
       m_run[nb] = l2 == -INFINITY ? INFINITY : l2;
     }
 #pragma unroll
@@ -195,8 +227,14 @@ __global__ __launch_bounds__(256, D >= 192 ? 1 : NB == 1 ? (D == 64 ? 3 : 2) : (
     float16_t s_a, s_b;  // named (not an array) so that they stay in registers
 #pragma unroll
     for (int r = 0; r < 16; r++) { s_a[r] = 0.f; s_b[r] = 0.f; }
+    if constexpr (PASS == kDecNormKept) {
+      // everything in flight belongs to this step: its scores are copied out, its V strip may be read
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 #pragma unroll
-    for (int s = 0; s < DS; s++) {
+      for (int r = 0; r < 16; r++) s_a[r] = (float)kfr[r / 8][r % 8];
+    }
+#pragma unroll
+    for (int s = 0; s < (PASS == kDecNormKept ? 0 : DS); s++) {
       if (!kQInLds) {
         s_a = Frag<T>::mfma(kfr[s], qf[0][s], s_a);
         if (NB > 1) s_b = Frag<T>::mfma(kfr[s], qf[NB - 1][s], s_b);
@@ -213,6 +251,24 @@ __global__ __launch_bounds__(256, D >= 192 ? 1 : NB == 1 ? (D == 64 ? 3 : 2) : (
     kv_q1 = kv_q2;
     kv_q2 = kv_q3;
     if (st + 16 < st_end) kv_q3 = step_kv0(st + 16);
+    if constexpr (PASS == kDecLseKeep) {
+      vec8 lo, hi;
+#pragma unroll
+      for (int r = 0; r < 8; r++) {
+        lo[r] = (T)s_a[r];
+        hi[r] = (T)s_a[r + 8];
+      }
+      if (col_ok[0]) {
+        T* sp = kept_bh + (int64_t)(kv0 / kStep) * kept_step;
+        *reinterpret_cast<vec8*>(sp) = lo;
+        *reinterpret_cast<vec8*>(sp + 8) = hi;
+      }
+#pragma unroll
+      for (int r = 0; r < 8; r++) {
+        s_a[r] = (float)lo[r];
+        s_a[r + 8] = (float)hi[r];
+      }
+    }
     // steps that every row of the call sees completely need no mask evaluation: those from the list of fully
     // visible tiles, and under a one-range band mask those inside the range common to all rows
     const bool listed_full = full_idx && (st >> 1) < n_full;
@@ -223,12 +279,12 @@ __global__ __launch_bounds__(256, D >= 192 ? 1 : NB == 1 ? (D == 64 ? 3 : 2) : (
 #pragma unroll
     for (int nb = 0; nb < NB; nb++) {
       float16_t sacc = nb ? s_b : s_a;
-      const float m_use = (PASS != kDecNorm && m_run[nb] == -INFINITY) ? 0.f : m_run[nb];
+      const float m_use = (!kNorm && m_run[nb] == -INFINITY) ? 0.f : m_run[nb];
       sm[nb].tile(col_q[nb] + p.q_index_base, kv0 + 4 * g);
 #pragma unroll
       for (int r = 0; r < 16; r += 2) {
         float s0 = sacc[r], s1 = sacc[r + 1];
-        if (ROUND_S) round_pair<T>(s0, s1);
+        if (ROUND_S && PASS != kDecLseKeep && PASS != kDecNormKept) round_pair<T>(s0, s1);   // (kept scores are rounded)
         sacc[r] = sm[nb].apply_sub(s0, acc_row(r), m_use);
         sacc[r + 1] = sm[nb].apply_sub(s1, acc_row(r + 1), m_use);
       }
@@ -241,7 +297,7 @@ __global__ __launch_bounds__(256, D >= 192 ? 1 : NB == 1 ? (D == 64 ? 3 : 2) : (
         mask_block_q(sacc, p.mask, visible, q_opaque, kv_opaque, g, p.Lkv);
       }
       // online softmax; the reference max moves only when it is beaten by 2^kTau
-      if constexpr (PASS != kDecNorm) {
+      if constexpr (!kNorm) {
         const float m_rel = xhalf_max(block_max(sacc));
         const bool need = (m_rel > kTau) || (m_run[nb] == -INFINITY && m_rel > -INFINITY);
         if (__any(need)) {
@@ -259,7 +315,7 @@ __global__ __launch_bounds__(256, D >= 192 ? 1 : NB == 1 ? (D == 64 ? 3 : 2) : (
           }
         }
       }
-      if constexpr (PASS == kDecLse) {
+      if constexpr (kLse) {
         // only the row sums, in fp32 (the dense path sums the unrounded exponentials)
 #pragma unroll
         for (int r = 0; r < 16; r++) l_run[nb] += fast_exp2(sacc[r]);
@@ -278,7 +334,7 @@ __global__ __launch_bounds__(256, D >= 192 ? 1 : NB == 1 ? (D == 64 ? 3 : 2) : (
         }
       }
     }
-    if constexpr (PASS != kDecLse) {
+    if constexpr (!kLse) {
       // the V strips belong to this wave alone: no workgroup barrier is needed
       __builtin_amdgcn_wave_barrier();
 #pragma unroll
@@ -313,8 +369,8 @@ __global__ __launch_bounds__(256, D >= 192 ? 1 : NB == 1 ? (D == 64 ? 3 : 2) : (
   for (int nb = 0; nb < NB; nb++) {
     float mm = fmaxf(fmaxf(mbuf[0][nb][i32], mbuf[1][nb][i32]), fmaxf(mbuf[2][nb][i32], mbuf[3][nb][i32]));
     m_all[nb] = mm;
-    // kDecNorm: every wave used the same fixed reference (possibly +inf), the partial outputs just add up
-    const float sc = PASS == kDecNorm ? 1.f : ((m_run[nb] == -INFINITY) ? 0.f : fast_exp2(m_run[nb] - mm));
+    // second pass: every wave used the same fixed reference (possibly +inf), the partial outputs just add up
+    const float sc = kNorm ? 1.f : ((m_run[nb] == -INFINITY) ? 0.f : fast_exp2(m_run[nb] - mm));
     l_scaled[nb] = l_run[nb] * sc;
 #pragma unroll
     for (int db = 0; db < DB; db++)
@@ -331,13 +387,13 @@ __global__ __launch_bounds__(256, D >= 192 ? 1 : NB == 1 ? (D == 64 ? 3 : 2) : (
 #pragma unroll
   for (int nb = 0; nb < NB; nb++) {
     const int64_t row_id = ((int64_t)b * p.Hq + col_h[nb]) * p.Lq + col_q[nb];
-    if (w == 0 && g == 0 && col_ok[nb]) {
+    if (!kNorm && w == 0 && g == 0 && col_ok[nb]) {
       float lt = mbuf[0][nb][i32] + mbuf[1][nb][i32] + mbuf[2][nb][i32] + mbuf[3][nb][i32];
       float* ml = ml_part + ((int64_t)split * part_rows + row_id) * 2;
-      ml[0] = PASS == kDecNorm ? 0.f : m_all[nb];
-      ml[1] = PASS == kDecNorm ? (split == 0 ? 1.f : 0.f) : lt;
+      ml[0] = m_all[nb];
+      ml[1] = lt;
     }
-    if constexpr (PASS == kDecLse) continue;  // no partial output in the log-sum-exp pass
+    if constexpr (kLse) continue;  // no partial output in the log-sum-exp pass
 #pragma unroll
     for (int db = 0; db < DB; db++) {
       const int blk = nb * DB + db;
@@ -365,7 +421,7 @@ __global__ __launch_bounds__(256, D >= 192 ? 1 : NB == 1 ? (D == 64 ? 3 : 2) : (
 // one wave per output row: merge the splits, normalise, write O and lse2.
 // Lane s first takes split s's (m, l) so that the max and the weights come from
 // one round of loads; the partial outputs are then fetched with all loads in
-// flight together.
+// flight together.  Without ml_part the partial outputs are normalised already and just add up.
 template <typename T, int D>
 __global__ __launch_bounds__(256) void decode_combine_kernel(FlexAttnParams p, const float* __restrict__ o_part,
                                                               const float* __restrict__ ml_part, int splits,
@@ -375,7 +431,10 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(FlexAttnParams p, c
   const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= rows) return;
   float ms = -INFINITY, ls = 0.f;
-  if (lane < splits) {
+  if (!ml_part) {
+    ms = lane < splits ? 0.f : -INFINITY;
+    ls = lane == 0 ? 1.f : 0.f;
+  } else if (lane < splits) {
     const float2 ml = *reinterpret_cast<const float2*>(ml_part + (lane * rows + row) * 2);
     ms = ml.x;
     ls = ml.y;
@@ -431,9 +490,9 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(FlexAttnParams p, c
 struct DecodeArgs {
   const void *q, *k, *v;
   void* o;
-  float* lse2;      // output, may be null
-  float* lse_pass;  // parity numerics: where the first pass leaves the merged log-sum-exp (lse2 or workspace)
+  float* lse2;  // output, may be null
   float *o_part, *ml_part;
+  void* kept;   // parity numerics: room for the rounded scores between the passes, or null
   int splits;
   hipStream_t s;
 };
@@ -444,34 +503,38 @@ static void launch_nb(const FlexAttnParams& p, const DecodeArgs& a) {
   const int ncols = (p.Hq / p.Hkv) * p.Lq;
   if (ncols <= 32 || D >= 192) {  // the caller has checked that D = 192 / 256 come with at most 32 columns
     hipLaunchKernelGGL((decode_split_kernel<T, D, KIND, RS, 1, PASS>), grid, dim3(256), 0, a.s, p, (const T*)a.q, (const T*)a.k,
-                       (const T*)a.v, a.o_part, a.ml_part, a.splits, a.lse_pass);
-  } else if constexpr (D < 192) {
+                       (const T*)a.v, a.o_part, a.ml_part, a.splits, a.lse2, (T*)a.kept);
+  } else if constexpr (D < 192 && PASS != kDecLseKeep && PASS != kDecNormKept) {
     hipLaunchKernelGGL((decode_split_kernel<T, D, KIND, RS, 2, PASS>), grid, dim3(256), 0, a.s, p, (const T*)a.q, (const T*)a.k,
-                       (const T*)a.v, a.o_part, a.ml_part, a.splits, a.lse_pass);
+                       (const T*)a.v, a.o_part, a.ml_part, a.splits, a.lse2, (T*)a.kept);
   }
 }
 
 template <typename T, int D>
-static void launch_combine(const FlexAttnParams& p, const DecodeArgs& a, T* o, float* lse2) {
+static void launch_combine(const FlexAttnParams& p, const DecodeArgs& a, const float* ml_part, float* lse2) {
   const int64_t rows = (int64_t)p.B * p.Hq * p.Lq;
-  hipLaunchKernelGGL((decode_combine_kernel<T, D>), dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, a.s, p, a.o_part, a.ml_part,
-                     a.splits, o, lse2);
+  hipLaunchKernelGGL((decode_combine_kernel<T, D>), dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, a.s, p, a.o_part, ml_part,
+                     a.splits, (T*)a.o, lse2);
 }
 
 template <typename T, int D, int KIND>
 static void launch_rs(const FlexAttnParams& p, const DecodeArgs& a) {
   if (p.flags & FLEX_PARITY) {
-    // parity numerics: (m, l) per split and their merge into the log-sum-exp, then the pass that multiplies the
-    // normalised, rounded P into V and the sum of the splits' partial outputs
-    launch_nb<T, D, KIND, true, kDecLse>(p, a);
-    launch_combine<T, D>(p, a, nullptr, a.lse_pass);
-    launch_nb<T, D, KIND, true, kDecNorm>(p, a);
-    launch_combine<T, D>(p, a, (T*)a.o, nullptr);
+    // parity numerics: (m, l) per split, then the pass that multiplies the normalised, rounded P into V and the sum of
+    // the splits' partial outputs
+    if (a.kept) {
+      launch_nb<T, D, KIND, true, kDecLseKeep>(p, a);
+      launch_nb<T, D, KIND, true, kDecNormKept>(p, a);
+    } else {
+      launch_nb<T, D, KIND, true, kDecLse>(p, a);
+      launch_nb<T, D, KIND, true, kDecNorm>(p, a);
+    }
+    launch_combine<T, D>(p, a, nullptr, nullptr);
     return;
   }
   if (p.flags & FLEX_ROUND_S) launch_nb<T, D, KIND, true, kDecOnePass>(p, a);
   else launch_nb<T, D, KIND, false, kDecOnePass>(p, a);
-  launch_combine<T, D>(p, a, (T*)a.o, a.lse2);
+  launch_combine<T, D>(p, a, a.ml_part, a.lse2);
 }
 
 template <typename T, int D>

@@ -69,12 +69,20 @@ int flex_decode_default_splits(const FlexAttnParams& p) {
   return s;
 }
 
-// partial outputs and (m, l) per split; the parity numerics add one float per row for the merged log-sum-exp
-// that the second pass reads (used when the caller passes no lse2)
+// partial outputs and (m, l) per split
 size_t flex_decode_workspace(const FlexAttnParams& p, int splits) {
   const size_t rows = (size_t)p.B * p.Hq * p.Lq;
-  const size_t lse = (p.flags & FLEX_PARITY) ? rows : 0;
-  return ((rows * splits * (p.D + 2) + lse) * sizeof(float) + 255) / 256 * 256;
+  return (rows * splits * (p.D + 2) * sizeof(float) + 255) / 256 * 256;
+}
+
+// Bytes in which the parity numerics keep the rounded scores between their two passes, 0 where they read K twice
+// instead.  A step's scores are 64 bytes per column, written and read once, against 64 * D bytes of K: kept while that is
+// at most half (columns <= D / 4).  bf16 KV cache [16,8,6001,128], 4 columns:
+// 107.7 us with K read twice and a merge launch between the passes, 86.8 us with the scores kept.
+size_t flex_decode_kept_bytes(const FlexAttnParams& p) {
+  const int64_t ncols = (int64_t)(p.Hq / p.Hkv) * p.Lq;
+  if (!(p.flags & FLEX_PARITY) || ncols > p.D / 4 || ncols > 32) return 0;
+  return (size_t)p.B * p.Hkv * ((p.Lkv + kStep - 1) / kStep) * ncols * kStep * 2;
 }
 
 // Device address of this file's scratch array on the current device, looked up once per device
@@ -104,7 +112,7 @@ void* flex_decode_static_scratch(size_t* bytes) {
 }
 
 int flex_decode_launch(const FlexAttnParams& p, const void* q, const void* k, const void* v, void* o, float* lse2, int splits,
-                       void* workspace, hipStream_t s) {
+                       void* workspace, bool keep_scores, hipStream_t s) {
   if (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)workspace) & 15) {
     flex_set_error("decode needs 16-byte aligned tensors");
     return 1;
@@ -113,8 +121,8 @@ int flex_decode_launch(const FlexAttnParams& p, const void* q, const void* k, co
   const size_t rows = (size_t)p.B * p.Hq * p.Lq;
   float* o_part = (float*)workspace;
   float* ml_part = o_part + rows * splits * p.D;
-  float* lse_ws = ml_part + rows * splits * 2;
-  const DecodeArgs a = {q, k, v, o, lse2, lse2 ? lse2 : lse_ws, o_part, ml_part, splits, s};
+  void* kept = keep_scores ? (char*)workspace + flex_decode_workspace(p, splits) : nullptr;
+  const DecodeArgs a = {q, k, v, o, lse2, o_part, ml_part, kept, splits, s};
   int rc;
   if (p.dtype == FLEX_F16)
     rc = p.D == 64 ? flex_decode_f16_64(p, a) : p.D == 128 ? flex_decode_f16_128(p, a) : p.D == 192 ? flex_decode_f16_192(p, a) : flex_decode_f16_256(p, a);

@@ -55,7 +55,8 @@ bool flex_decode_supported(const FlexAttnParams& p);
 int flex_decode_default_splits(const FlexAttnParams& p);
 size_t flex_decode_workspace(const FlexAttnParams& p, int splits);
 int flex_decode_launch(const FlexAttnParams& p, const void* q, const void* k, const void* v, void* o, float* lse2, int splits,
-                       void* workspace, hipStream_t s);
+                       void* workspace, bool keep_scores, hipStream_t s);
+size_t flex_decode_kept_bytes(const FlexAttnParams& p);
 void* flex_decode_static_scratch(size_t* bytes);
 void flex_mfma_tiles(int dtype, int D, int Dv, int which, int* qb, int* kvb);
 bool flex_simple_supported(const FlexAttnParams& p, int which);
@@ -236,16 +237,16 @@ extern "C" int flexattn_bwd(const FlexAttnParams* p, const void* q, const void* 
 extern "C" size_t flexattn_decode_workspace_bytes(const FlexAttnParams* p, int32_t num_splits) {
   if (!p) return 0;
   if (num_splits <= 0) num_splits = flex_decode_default_splits(*p);
-  return flex_decode_workspace(*p, num_splits);
+  return flex_decode_workspace(*p, num_splits) + flex_decode_kept_bytes(*p);
 }
 
 static int decode_checked(const FlexAttnParams* p, const void* q, const void* k, const void* v, void* o, float* lse2,
-                          int32_t num_splits, void* workspace, flexattn_stream_t stream);
+                          int32_t num_splits, void* workspace, bool keep_scores, flexattn_stream_t stream);
 
 extern "C" int flexattn_decode(const FlexAttnParams* p, const void* q, const void* k, const void* v, void* o, float* lse2,
                                int32_t num_splits, void* workspace, flexattn_stream_t stream) {
   if (int rc = validate(p, "flexattn_decode")) return rc;
-  return decode_checked(p, q, k, v, o, lse2, num_splits, workspace, stream);
+  return decode_checked(p, q, k, v, o, lse2, num_splits, workspace, true, stream);
 }
 
 extern "C" int flexattn_decode_static(const FlexAttnParams* p, const void* q, const void* k, const void* v, void* o,
@@ -266,11 +267,12 @@ extern "C" int flexattn_decode_static(const FlexAttnParams* p, const void* q, co
                    need, p->B, p->Hq, p->Lq, p->D, num_splits, cap);
     return 1;
   }
-  return decode_checked(p, q, k, v, o, lse2, num_splits, ws, stream);
+  // the parity numerics keep their scores between the passes where those fit beside the partials
+  return decode_checked(p, q, k, v, o, lse2, num_splits, ws, need + flex_decode_kept_bytes(*p) <= cap, stream);
 }
 
 static int decode_checked(const FlexAttnParams* p, const void* q, const void* k, const void* v, void* o, float* lse2,
-                          int32_t num_splits, void* workspace, flexattn_stream_t stream) {
+                          int32_t num_splits, void* workspace, bool keep_scores, flexattn_stream_t stream) {
   if (p->flags & FLEX_UNROUNDED) { flex_set_error("flexattn_decode: FLEX_UNROUNDED is served by flexattn_fwd (the decode kernel carries P in one part)"); return 1; }
   if (p->q_index_base < 0) { flex_set_error("flexattn_decode: q_index_base must not be negative (got %d)", p->q_index_base); return 1; }
   if (!q || !k || !v || !o || !workspace) { flex_set_error("flexattn_decode: null pointer"); return 1; }
@@ -279,7 +281,8 @@ static int decode_checked(const FlexAttnParams* p, const void* q, const void* k,
     return 1;
   }
   if (num_splits <= 0) num_splits = flex_decode_default_splits(*p);
-  int rc = flex_decode_launch(*p, q, k, v, o, lse2, num_splits, workspace, (hipStream_t)stream);
+  int rc = flex_decode_launch(*p, q, k, v, o, lse2, num_splits, workspace,
+                              keep_scores && flex_decode_kept_bytes(*p) > 0, (hipStream_t)stream);
   if (rc) return rc;
   return check_launch("flexattn_decode");
 }

@@ -237,3 +237,43 @@ def test_decode_kv_cache_beyond_2_31_elements(dev, Lq):
                                    score_mod=generate_alibi_bias(1, -1.0), block_mask=bm, return_lse=True, kernel_options=opts)
     torch.cuda.synchronize()
     assert torch.equal(out[b:b + 1, h:h + 1], out1) and torch.equal(lse[b:b + 1, h:h + 1], lse1)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,Lq,Lkv,D,mask", [
+    (1, 64, 8, 4, 33000, 128, "none"),      # 32 columns: the widest call that keeps its scores at D = 128
+    (8, 64, 16, 4, 8200, 64, "causal"),     # 16 columns, the widest at D = 64; the last step ragged
+    (40, 32, 8, 2, 6200, 192, "window"),
+    (48, 32, 16, 1, 12001, 256, "window")])
+def test_parity_decode_with_and_without_kept_scores(dev, B, Hq, Hkv, Lq, Lkv, D, mask):
+    """The parity numerics keep their rounded scores between the two passes where the workspace has room: beyond
+    the 16 MiB of flexattn_decode_static the same call reads K twice instead.  Outputs and log-sum-exps are the same bits."""
+    from flaxattention_amd import _lib
+    from flaxattention_amd.core.attention import _Plan
+    from flaxattention_amd.core.common import IDENTITY, MaskMod
+    print("case kept scores", B, Hq, Hkv, Lq, Lkv, D, mask, flush=True)
+    g = torch.Generator(device=dev).manual_seed(3)
+    mk = lambda *s: torch.randn(*s, generator=g, device=dev).to(torch.bfloat16)
+    q, k, v = mk(B, Hq, Lq, D), mk(B, Hkv, Lkv, D), mk(B, Hkv, Lkv, D)
+    m = {"none": MaskMod(), "causal": MaskMod(0, q_offset=Lkv - Lq), "window": MaskMod(0, 700, 3, Lkv - Lq)}[mask]
+    got = []
+    L, s = _lib.lib(), torch.cuda.current_stream().cuda_stream
+    for static in (False, True):
+        o, lse = torch.empty_like(q), torch.empty((B, Hq, Lq), device=dev)
+        plan = _Plan(q, k, v, IDENTITY, m, None, D ** -0.5, _lib.FLAG_PARITY | _lib.FLAG_ROUND_S, True)
+        p = plan.params(q, k, v, o)
+        nbytes = L.flexattn_decode_workspace_bytes(p, 0)
+        assert nbytes > 16 << 20
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
+        args = (p, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(), 0)
+        _lib.check(L.flexattn_decode_static(*args, s) if static else L.flexattn_decode(*args, ws.data_ptr(), s), "decode")
+        torch.cuda.synchronize()
+        got.append((o, lse))
+    assert torch.isfinite(got[0][0].float()).all() and torch.isfinite(got[0][1]).all()
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    # and against the same formulas in float64 for one (batch, head): P rounds to 8 bits, so 2^-8 relative
+    qs, ks, vs = q[-1, -1].double(), k[-1, -1].double(), v[-1, -1].double()
+    i = torch.arange(Lq, device=dev).reshape(-1, 1)
+    x = (qs @ ks.T) * D ** -0.5
+    x = x.masked_fill(~m(None, None, i, torch.arange(Lkv, device=dev).reshape(1, -1)), -float("inf")) if mask != "none" else x
+    want = torch.softmax(x, -1) @ vs
+    assert ((got[0][0][-1, -1].double() - want).norm() / want.norm()).item() < 2 ** -6
