@@ -43,7 +43,8 @@ selects numerics here:
     {"decode_splits": n}  force the split-KV decode kernel with n splits
     {"split_kv": bool}    False: the forward kernel never splits a call over the keys
                           (by default it does when the query tiles alone are fewer
-                          workgroups than the GPU has compute units); the result of a
+                          workgroups than the GPU has compute units), and the backward
+                          never splits a key tile's queries; the result of a
                           (batch, head) pair then does not depend on how many pairs
                           the call has, bit for bit
     {"pad_head_dim": bool}  inputs whose head sizes are not among those of the matrix-core kernels
@@ -197,6 +198,8 @@ def _make_plan(q, k, v, score_mod, block_mask: Optional[BlockMask], mask_mod, sc
         flags |= _lib.FLAG_PARITY
     if numerics == "unrounded":
         flags = (flags & ~(_lib.FLAG_ROUND_S | _lib.FLAG_STRICT)) | _lib.FLAG_UNROUNDED
+    if not opts.get("split_kv", True):
+        flags |= _lib.FLAG_NO_SPLIT
     plan = _Plan(q, k, v, score, mask, block_mask, scale, flags, True, _decode_choice(q, k, v, score, flags, opts))
     plan.split_kv = bool(opts.get("split_kv", True))
     # tile lists at the fused kernels' granularity (skipped for a mask that hides nothing)

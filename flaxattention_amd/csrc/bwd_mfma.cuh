@@ -377,13 +377,17 @@ template <int D> struct DkvShape {
 // from the kBwdDelta sweep) is subtracted, and the scale is applied before dS is rounded.
 // HILO (the "unrounded" numerics, exclusive with PARITY, launched with ROUND_S = false): P and dS go into their
 // products as a high and a low part each (two matrix instructions per fragment); delta comes from the kBwdDeltaRaw sweep.
-template <typename T, int D, int KIND, bool ROUND_S, bool BITS, bool PARITY = false, bool HILO = false>
+// SPLIT: `parts` workgroups share a key tile -- each takes some of the group's query heads, or a stretch of every head's
+// tile list -- and leave float32 partial sums of dK and dV in `partial`, in the order their lanes hold them;
+// dkv_combine_kernel adds and converts them.  For calls with too few key tiles to fill the chip evenly (dkv_parts below).
+template <typename T, int D, int KIND, bool ROUND_S, bool BITS, bool PARITY = false, bool HILO = false, bool SPLIT = false>
 __global__ __launch_bounds__(DkvShape<D>::kThreads, D == 64 ? 2 : 1) void bwd_dkv_kernel(FlexAttnParams p, const T* __restrict__ q,
                                                                const T* __restrict__ k, const T* __restrict__ v,
                                                                const float* __restrict__ lse2,
                                                                const float* __restrict__ delta,
                                                                const T* __restrict__ d_o, T* __restrict__ dk,
-                                                               T* __restrict__ dv) {
+                                                               T* __restrict__ dv, int parts_g, int parts_t,
+                                                               float* __restrict__ partial) {
   typedef typename Frag<T>::vec8 vec8;
   constexpr int BM = kBM, BN = kListBN;
   constexpr int QBW = DkvShape<D>::kQBlocks;
@@ -401,7 +405,14 @@ __global__ __launch_bounds__(DkvShape<D>::kThreads, D == 64 ? 2 : 1) void bwd_dk
   const int wk = __builtin_amdgcn_readfirstlane(w);  // key block (32 rows) of this wave (wave-uniform)
   const int nkt = (p.Lkv + BN - 1) / BN;
   int kt, bh;  // early key tiles see the most queries under causal masks
-  xcd_tile_map(blockIdx.x, nkt, p.Hkv * p.B, kt, bh);
+  int wid = blockIdx.x, part = 0;
+  if constexpr (SPLIT) {
+    // the parts of a tile stay on one XCD (they read the same K and V) and next to each other in the order
+    const int parts = parts_g * parts_t, run = (p.Hkv * p.B) % 8 ? 1 : 8;
+    part = wid / run % parts;
+    wid = wid / (run * parts) * run + wid % run;
+  }
+  xcd_tile_map(wid, nkt, p.Hkv * p.B, kt, bh);
   const int hk = bh % p.Hkv, b = bh / p.Hkv, G = p.Hq / p.Hkv;
   const int kv_col = kt * BN + wk * 32 + i32;
   const int kv_ld = min(kv_col, p.Lkv - 1);
@@ -441,7 +452,7 @@ __global__ __launch_bounds__(DkvShape<D>::kThreads, D == 64 ? 2 : 1) void bwd_dk
   Score2<KIND> sm;
   float key_grad = 1.f;  // derivative of a score_mod that depends on the key only: applied to dK at the end
 
-  for (int gi = 0; gi < G; gi++) {
+  for (int gi = SPLIT ? part % parts_g : 0; gi < G; gi += SPLIT ? parts_g : 1) {
     const int h = hk * G + gi;
     sm.init(p.score, p.scale, h, b, p.Lq, p.Lkv);
     const int32_t* full_idx = nullptr;
@@ -458,7 +469,12 @@ __global__ __launch_bounds__(DkvShape<D>::kThreads, D == 64 ? 2 : 1) void bwd_dk
       n_full = (p.Lq + BM - 1) / BM;
       if (!mask_hides_nothing(p.mask)) { n_part = n_full; n_full = 0; }
     }
-    const int nt = n_full + n_part;
+    int it0 = 0, nt = n_full + n_part;   // this workgroup's stretch of the list
+    if constexpr (SPLIT) {
+      const int share = part / parts_g, all = nt;
+      it0 = all * share / parts_t;
+      nt = all * (share + 1) / parts_t;
+    }
     const T* qbase = q + b * p.q_stride[0] + h * p.q_stride[1];
     const int64_t rows0 = ((int64_t)b * p.Hq + h) * p.Lq;
     const T* dobase = d_o + rows0 * D;
@@ -497,8 +513,8 @@ __global__ __launch_bounds__(DkvShape<D>::kThreads, D == 64 ? 2 : 1) void bwd_dk
         if (lreg == -INFINITY) lreg = INFINITY;  // row without visible keys: P = 0
       }
     };
-    int t_cur = nt > 0 ? tile_at(0) : 0;
-    int t_nxt = nt > 1 ? tile_at(1) : 0;
+    int t_cur = nt > it0 ? tile_at(it0) : 0;
+    int t_nxt = nt > it0 + 1 ? tile_at(it0 + 1) : 0;
     auto store_tile = [&](int st) {
       T* Qw = stage_q(st);
       T* Ow = Qw + BM * ROWE;
@@ -509,15 +525,15 @@ __global__ __launch_bounds__(DkvShape<D>::kThreads, D == 64 ? 2 : 1) void bwd_dk
       }
     };
     __syncthreads();  // the stages may still be in use by the previous head of the group
-    if (nt > 0) {
-      issue_tile(0, t_cur * BM);
+    if (nt > it0) {
+      issue_tile(it0 & 1, t_cur * BM);
       load_tile(t_cur * BM);
-      store_tile(0);
+      store_tile(it0 & 1);
     }
-    if (nt > 1) load_tile(t_nxt * BM);
+    if (nt > it0 + 1) load_tile(t_nxt * BM);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    for (int it = 0; it < nt; it++) {
+    for (int it = it0; it < nt; it++) {
       const int q0 = t_cur * BM;
       const bool masked = (it >= n_full) || (q0 + BM > p.Lq) || (kt * BN + BN > p.Lkv);
       const T* Qs = stage_q(it & 1);
@@ -664,6 +680,26 @@ __global__ __launch_bounds__(DkvShape<D>::kThreads, D == 64 ? 2 : 1) void bwd_dk
     }
   }
 
+  if constexpr (SPLIT) {
+    // [part][tile][wave][dk | dv][register quad][lane]: every store instruction fills 1 KB
+    float4_t* out = reinterpret_cast<float4_t*>(partial) +
+                    ((((int64_t)part * p.B * p.Hkv + bh) * nkt + kt) * DkvShape<D>::kWaves + wk) * (2 * DB * 4 * 64) + lane;
+    const float dk_scale = PARITY ? 1.f : p.scale * key_grad;
+#pragma unroll
+    for (int db = 0; db < DB; db++)
+#pragma unroll
+      for (int rr = 0; rr < 4; rr++) {
+        float4_t a, c;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          a[e] = dkacc[db][4 * rr + e] * dk_scale;
+          c[e] = dvacc[db][4 * rr + e];
+        }
+        out[(db * 4 + rr) * 64] = a;
+        out[((DB + db) * 4 + rr) * 64] = c;
+      }
+    return;
+  }
   if (kv_col < p.Lkv) {
     const int64_t row_id = ((int64_t)b * p.Hkv + hk) * p.Lkv + kv_col;
     T* dkp = dk + row_id * D + 4 * g;
@@ -685,6 +721,28 @@ __global__ __launch_bounds__(DkvShape<D>::kThreads, D == 64 ? 2 : 1) void bwd_dk
   }
 }
 
+// adds the partial sums of a split dK/dV call: one workgroup per (key tile, wave of it), coalesced reads of every part
+template <typename T, int D>
+__global__ __launch_bounds__(256) void dkv_combine_kernel(const float* __restrict__ partial, int parts, int nkt, int Lkv,
+                                                          T* __restrict__ dk, T* __restrict__ dv) {
+  constexpr int DB = D / 32, kWaves = DkvShape<D>::kWaves, kQuads = 2 * DB * 4 * 64;
+  const int wk = blockIdx.x % kWaves, kt = blockIdx.x / kWaves % nkt, bh = blockIdx.x / (kWaves * nkt);
+  const float4_t* in = reinterpret_cast<const float4_t*>(partial) + (int64_t)blockIdx.x * kQuads;
+  const int64_t part_stride = (int64_t)gridDim.x * kQuads;
+  for (int i = threadIdx.x; i < kQuads; i += 256) {
+    float4_t sum = in[i];
+    for (int s = 1; s < parts; s++) sum += in[s * part_stride + i];
+    const int lane = i & 63, quad = i >> 6, db = quad / 4 % DB;
+    const int kv = kt * kListBN + wk * 32 + (lane & 31);
+    if (kv >= Lkv) continue;
+    union { T e[4]; uint2 u; } pk;
+#pragma unroll
+    for (int e = 0; e < 4; e++) pk.e[e] = (T)sum[e];
+    T* out = quad < DB * 4 ? dk : dv;
+    *reinterpret_cast<uint2*>(out + ((int64_t)bh * Lkv + kv) * D + 32 * db + 8 * (quad & 3) + 4 * (lane >> 5)) = pk.u;
+  }
+}
+
 // two stages of (Q tile, dO tile, lse, -delta)
 template <int D, typename T> constexpr size_t dkv_smem() {
   return 2 * ((size_t)2 * kBM * D * sizeof(T) + 2 * kBM * sizeof(float));
@@ -696,26 +754,38 @@ struct BwdArgs {
   const float* lse2;
   void *dq, *dk, *dv;
   float* delta;
+  float* partial;          // partial sums of a dK/dV call split into parts_g x parts_t
+  int parts_g, parts_t;
   hipStream_t s;
 };
 
 // (D = 192 and D = 256 have the dQ kernel only: the resident K / V fragments and the two accumulators of a dK/dV workgroup do not
 // fit a wave's registers; the caller runs the dK/dV kernel of the simple family)
+template <typename T, int D, int KIND, bool RS, bool BITS, bool PARITY, bool HILO, bool SPLIT>
+static int launch_dkv_form(const FlexAttnParams& p, const BwdArgs& a) {
+  constexpr size_t sm = dkv_smem<D, T>();
+  // set on every call: the attribute is per device, and a remembered "already set" would be neither
+  // per device nor safe between threads (the call is a host-side table update, no device work)
+  if (hipFuncSetAttribute(reinterpret_cast<const void*>(bwd_dkv_kernel<T, D, KIND, RS, BITS, PARITY, HILO, SPLIT>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm) != hipSuccess)
+    return 2;
+  const int nkt = (p.Lkv + kListBN - 1) / kListBN, tiles = nkt * p.Hkv * p.B, parts = SPLIT ? a.parts_g * a.parts_t : 1;
+  hipLaunchKernelGGL((bwd_dkv_kernel<T, D, KIND, RS, BITS, PARITY, HILO, SPLIT>), dim3(tiles * parts), dim3(DkvShape<D>::kThreads),
+                     sm, a.s, p, (const T*)a.q, (const T*)a.k, (const T*)a.v, a.lse2, a.delta, (const T*)a.d_o, (T*)a.dk,
+                     (T*)a.dv, a.parts_g, a.parts_t, a.partial);
+  if constexpr (SPLIT)
+    hipLaunchKernelGGL((dkv_combine_kernel<T, D>), dim3(tiles * DkvShape<D>::kWaves), dim3(256), 0, a.s, a.partial, parts, nkt,
+                       p.Lkv, (T*)a.dk, (T*)a.dv);
+  return 0;
+}
 template <typename T, int D, int KIND, bool RS, bool BITS, bool PARITY, bool HILO = false>
 static int launch_dkv_as(const FlexAttnParams& p, const BwdArgs& a) {
   if constexpr (D >= 192) {
     return 3;
   } else {
-  constexpr size_t sm = dkv_smem<D, T>();
-  // set on every call: the attribute is per device, and a remembered "already set" would be neither
-  // per device nor safe between threads (the call is a host-side table update, no device work)
-  if (hipFuncSetAttribute(reinterpret_cast<const void*>(bwd_dkv_kernel<T, D, KIND, RS, BITS, PARITY, HILO>),
-                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)sm) != hipSuccess)
-    return 2;
-  const int nkt = (p.Lkv + kListBN - 1) / kListBN;
-  hipLaunchKernelGGL((bwd_dkv_kernel<T, D, KIND, RS, BITS, PARITY, HILO>), dim3(nkt * p.Hkv * p.B), dim3(DkvShape<D>::kThreads), sm, a.s,
-                     p, (const T*)a.q, (const T*)a.k, (const T*)a.v, a.lse2, a.delta, (const T*)a.d_o, (T*)a.dk, (T*)a.dv);
-  return 0;
+    if constexpr (!HILO)
+      if (a.parts_g * a.parts_t > 1) return launch_dkv_form<T, D, KIND, RS, BITS, PARITY, HILO, true>(p, a);
+    return launch_dkv_form<T, D, KIND, RS, BITS, PARITY, HILO, false>(p, a);
   }
 }
 template <typename T, int D, int KIND, bool RS, bool PARITY>

@@ -1,9 +1,12 @@
 // Fused flash-attention backward for gfx950 (fp16 / bf16, D = Dv in {64, 128}; dQ also at 192 / 256): checks and dispatch.  The kernels are
 // in bwd_mfma.cuh, instantiated per (dtype, head size) by bwd_mfma_inst.hip.
+#include <cmath>
+
 #include "bwd_mfma.cuh"
 
 using namespace flex;
 void flex_set_error(const char* fmt, ...);
+int flex_cu_count();
 bool flex_mfma_shape_ok(const FlexAttnParams& p);
 int flex_mfma_bwd_f16_64(const FlexAttnParams& p, const BwdArgs& a);
 int flex_mfma_bwd_f16_128(const FlexAttnParams& p, const BwdArgs& a);
@@ -34,7 +37,51 @@ bool flex_mfma_bwd_supported(const FlexAttnParams& p) {
   return true;
 }
 
-size_t flex_mfma_bwd_workspace(const FlexAttnParams& p) { return 0; }  // delta is accounted for by the caller
+// How many workgroups share a key tile of the dK/dV kernel: parts_g over the query heads of the group times parts_t over
+// each head's list of query tiles.  A key tile's workgroup visits up to `visits` query tiles; under a mask the work of
+// the tiles differs (causal: the heaviest is twice the mean), so with no more tiles than compute units slots the
+// heaviest one is the call: bf16 [1,32->8,4096,128] causal, 256 tiles on 256 slots, 637 us against 398 + 14 us in two parts.
+// Counted in tile visits (about 5 us each), with what adding the partial sums costs in the same unit (4 us, and 27 us
+// for the 67 MB that twice the slots write and read); taken where it promises a fifth and 30 us
+// (less is lost again on the second launch where the host sets the pace: bf16 [1,4,881,64] causal 131 -> 145 us).
+struct DkvParts { int g, t; };
+static DkvParts dkv_parts(const FlexAttnParams& p) {
+  if ((p.D != 64 && p.D != 128) || (p.flags & (FLEX_UNROUNDED | FLEX_NO_SPLIT))) return {1, 1};
+  const double slots = (double)flex_cu_count() * (p.D == 64 ? 2 : 1);   // workgroups the chip holds at once
+  const double tiles = (double)((p.Lkv + kListBN - 1) / kListBN) * p.Hkv * p.B;
+  const int G = p.Hq / p.Hkv, nqt = (p.Lq + kBM - 1) / kBM;
+  // what a tile's list holds is on the device: bitmaps (documents) count as a quarter full, a window without sink keys
+  // by its width (bf16 [2,8,3000,64], 9 documents: in two parts 30 + 11 us against 33 us, so not split)
+  double listed = nqt;
+  if (p.mask.kind == FLEX_MASK_BITS) listed = fmax(1.0, 0.25 * nqt);
+  else if (p.mask.hi != INT32_MAX && p.mask.sink < 0 && p.mask.lo != INT32_MIN)
+    listed = fmin(nqt, fmax(0.0, (double)p.mask.hi - p.mask.lo) / kBM + 2);
+  const double visits = G * listed;
+  const bool uneven = p.tiles_bwd.kv_num || !mask_hides_nothing(p.mask);
+  auto cost = [&](int parts) {
+    const double each = visits / parts, rounds = ceil(tiles * parts / slots);
+    const double run = uneven ? fmax(each, 0.5 * visits * tiles / slots) : each * rounds;
+    return parts == 1 ? (uneven ? fmax(visits, 0.5 * visits * tiles / slots) : run) : run + 1 + 2.7 * tiles * parts / slots;
+  };
+  DkvParts best = {1, 1};
+  double least = fmin(0.8 * cost(1), cost(1) - 6);
+  for (int parts = 2; parts <= 16 && parts <= visits && tiles * parts <= 2 * slots; parts++) {
+    int g = parts < G ? parts : G;
+    while (G % g || parts % g) g--;   // whole heads first, stretches of the lists for the rest
+    if (parts / g > nqt || cost(parts) >= least) continue;
+    least = cost(parts);
+    best = {g, parts / g};
+  }
+  return best;
+}
+
+// beside delta, which the caller accounts for: the partial sums of a split dK/dV call
+size_t flex_mfma_bwd_workspace(const FlexAttnParams& p) {
+  const DkvParts n = dkv_parts(p);
+  if (n.g * n.t == 1) return 0;
+  const size_t rows = (size_t)((p.Lkv + kListBN - 1) / kListBN) * kListBN * p.Hkv * p.B;
+  return (size_t)n.g * n.t * rows * 2 * p.D * sizeof(float);
+}
 
 int flex_mfma_bwd(const FlexAttnParams& p, const void* q, const void* k, const void* v, const void* o, const float* lse2,
                   const void* d_o, void* dq, void* dk, void* dv, void* workspace, hipStream_t s) {
@@ -42,7 +89,9 @@ int flex_mfma_bwd(const FlexAttnParams& p, const void* q, const void* k, const v
     flex_set_error("fused backward needs 16-byte aligned tensors");
     return 1;
   }
-  const BwdArgs a = {q, k, v, o, d_o, lse2, dq, dk, dv, (float*)workspace, s};
+  const DkvParts n = dkv_parts(p);
+  const size_t delta_bytes = ((size_t)p.B * p.Hq * p.Lq * sizeof(float) + 255) / 256 * 256;
+  const BwdArgs a = {q, k, v, o, d_o, lse2, dq, dk, dv, (float*)workspace, (float*)((char*)workspace + delta_bytes), n.g, n.t, s};
   int rc;
   if (p.D >= 192 && !(p.flags & FLEX_BWD_ONLY_DQ)) {
     flex_set_error("fused backward: only the dQ kernel exists for 192- and 256-wide heads");

@@ -113,6 +113,9 @@ enum FlexFlags {
                             simplification removes the round trips of attention.py:27, 104-105.
                             Exclusive with FLEX_PARITY / FLEX_ROUND_S (it wins); the generic kernels
                             do the same when neither FLEX_STRICT nor FLEX_ROUND_S is set.  */
+  FLEX_NO_SPLIT = 128,   /* flexattn_bwd: one workgroup per key tile always sums all its queries.  Without it a call with
+                            few key tiles divides each over several workgroups (float32 partial sums in the
+                            workspace), so that the order of those sums depends on the number of tiles.  */
   /* profiling aids for flexattn_bwd: launch only one of the two fused backward
    * kernels.  The dK/dV kernel then reads the delta values a previous complete
    * call left in the same workspace. */

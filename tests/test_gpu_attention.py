@@ -1151,3 +1151,42 @@ def test_document_mask_equals_per_document_attention(dev):
     assert rel_l2(out.detach().float().cpu(), want.detach().cpu()) <= 1e-3
     for got, ref in ((q.grad, qf.grad), (k.grad, kf.grad), (v.grad, vf.grad)):
         assert rel_l2(got.float().cpu(), ref.cpu()) <= 2e-3
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("B,Hq,Hkv,Lq,Lkv,D,kind", [
+    (1, 8, 2, 1500, 1500, 128, "causal"),     # whole heads of the group per part, ragged tiles
+    (1, 6, 2, 900, 1100, 64, "causal"),       # a group of three heads
+    (1, 2, 2, 3000, 1000, 64, "none"),        # stretches of the list, no mask
+    (3, 1, 1, 2100, 130, 128, "none"),        # tile count not a multiple of the XCDs
+    (1, 4, 1, 1700, 1700, 64, "window"),
+    (2, 3, 1, 2000, 1300, 128, "bitmap")])
+def test_backward_split_over_the_queries(dev, dtype, B, Hq, Hkv, Lq, Lkv, D, kind):
+    """Calls with few key tiles divide each tile's queries over several workgroups of the dK/dV kernel; against the oracle,
+    and against the undivided call, whose float32 sums only run in another order (a result then moves by at most one
+    rounding of the dtype, and few of them do)."""
+    from flaxattention_amd import _lib
+    from flaxattention_amd.core.attention import _make_plan, _run_bwd, _run_fwd
+    print("case split backward", dtype, B, Hq, Hkv, Lq, Lkv, D, kind, flush=True)
+    mask, omask = {"causal": (causal_mask, o_causal_mask), "none": (None, None),
+                   "window": (generate_attention_sink(300, 3), o_attention_sink(300, 3)),
+                   "bitmap": ((lambda b, h, q, kv: (q * 7 + kv * 3 + b) % 5 != 0),) * 2}[kind]
+    q, k, v = seeded_qkv(B, Hq, Hkv, Lq, Lkv, D, dtype)
+    d_o = torch.randn(B, Hq, Lq, D, generator=torch.Generator().manual_seed(4)).to(dtype)
+    bm = fa.create_block_mask(mask, B if kind == "bitmap" else None, None, Lq, Lkv, device=dev) if mask is not None else None
+    qd, kd, vd, dod = (t.to(dev) for t in (q, k, v, d_o))
+    grads = {}
+    for split in (True, False):
+        plan = _make_plan(qd, kd, vd, None, bm, None, D ** -0.5, None if split else {"split_kv": False})
+        if split:
+            out, lse2 = _run_fwd(plan, qd, kd, vd)
+        delta = (B * Hq * Lq * 4 + 255) // 256 * 256
+        assert (_lib.lib().flexattn_bwd_workspace_bytes(plan.params(qd, kd, vd, out)) > delta) == split
+        grads[split] = _run_bwd(plan, qd, kd, vd, out, lse2, dod)
+    assert torch.equal(grads[True][0], grads[False][0])
+    want = ref_attention_bwd(q, k, v, d_o, None, omask, strict=True)
+    for name, a, b, w in zip(("dQ", "dK", "dV"), grads[True], grads[False], want):
+        close(a, w, dtype, name, scale_maxabs=True)
+        # one rounding of the result, and for entries that cancel the float32 sums' own error (2^-24 of what they add up)
+        eps = 2.0 ** (-7 if dtype == torch.bfloat16 else -10)
+        assert ((a.float() - b.float()).abs() <= eps * b.float().abs() + 1e-5 * b.float().abs().max()).all(), name
