@@ -13,6 +13,7 @@ and Python ints alike.
 from __future__ import annotations
 
 import ctypes
+import functools
 import inspect
 import math
 from enum import Enum
@@ -132,13 +133,32 @@ def _identity(score, batch, head, token_q, token_kv):
 IDENTITY = ScoreMod(_lib.SCORE_IDENTITY, name="identity")
 
 
+_CORNER_SCORES = (-1.75, -0.5, 0.0, 0.625, 2.5)
+_TABLE_SCORES = (0.0, 8.0, -8.0, 0.625, -1.75, 3.25)   # what flexattn_affine_tables takes
+
+
+@functools.lru_cache(maxsize=None)
+def _scores_on(scores: tuple, device: torch.device) -> torch.Tensor:
+    return torch.tensor(scores, dtype=torch.float32, device=device).reshape(-1, 1, 1, 1, 1)
+
+
+def _grid5(scores: tuple, extents: Tuple[int, int, int, int], where):
+    """score [n,1,1,1,1] and b, h, q, kv index tensors that broadcast against it, made on `where` (a copy of the scores:
+    a callable may write into its argument)."""
+    idx = []
+    for i, n in enumerate(extents):
+        idx.append(torch.arange(n, dtype=torch.int32, device=where).reshape([-1 if j == i + 1 else 1 for j in range(5)]))
+    return (_scores_on(scores, torch.device(where)).clone(), *idx)
+
+
 def _probe_score_mod(fn: Callable, H: int, shape: Optional[Tuple[int, int, int, int]] = None,
-                     device=None) -> Optional[ScoreMod]:
+                     device=None, corner: Optional[list] = None) -> Optional[ScoreMod]:
     """Recognise an untagged Python score_mod as one of the functor families by
     evaluating it on a small grid and checking every family exactly.  A callable that may look
     positions up in captured tensors is only probed inside the real index ranges of `shape`
     (an out-of-range index into a device tensor stops the process), and on the device when it
-    cannot take CPU tensors."""
+    cannot take CPU tensors or holds device tensors.  The values on the grid, [scores, b, h, q, kv] on the CPU, are
+    appended to `corner`."""
     Pq, Pkv, nb = 7, 9, 2
     Hn = max(int(H), 1)
     shape_in = shape
@@ -146,24 +166,31 @@ def _probe_score_mod(fn: Callable, H: int, shape: Optional[Tuple[int, int, int, 
         if shape is None:
             return None
         nb, Pq, Pkv = min(nb, shape[0]), min(Pq, shape[2]), min(Pkv, shape[3])
-    s = torch.tensor([-1.75, -0.5, 0.0, 0.625, 2.5], dtype=torch.float32).reshape(5, 1, 1, 1, 1)
-    b = torch.arange(nb, dtype=torch.int32).reshape(1, nb, 1, 1, 1)
-    h = torch.arange(Hn, dtype=torch.int32).reshape(1, 1, Hn, 1, 1)
-    q = torch.arange(Pq, dtype=torch.int32).reshape(1, 1, 1, Pq, 1)
-    kv = torch.arange(Pkv, dtype=torch.int32).reshape(1, 1, 1, 1, Pkv)
     shape5 = (5, nb, Hn, Pq, Pkv)
     out = None
-    for where in ("cpu",) + ((device,) if device is not None else ()):
+    captured: list = []
+    _scan_captures(fn, captured)
+    on_device = device is not None and any(t.is_cuda for t in captured)
+    for where in (("cpu",) if not on_device else ()) + ((device,) if device is not None else ()):
         try:
-            res = fn(s.to(where).expand(shape5), b.to(where), h.to(where), q.to(where), kv.to(where))
+            s, b, h, q, kv = _grid5(_CORNER_SCORES, shape5[1:], where)
+            res = fn(s.expand(shape5), b, h, q, kv)
             if not torch.is_tensor(res):
                 return None
             out = torch.broadcast_to(res.to(torch.float32), shape5).cpu()
-            s, b, h, q, kv = (t.to(where) for t in (s, b, h, q, kv))
             break
         except Exception:
             continue
+    if out is not None and corner is not None:
+        corner.append(out)
     if out is None or Pkv < 2:
+        return None
+    # a family is only compared where its exact zeros allow it: identity, checkerboard and soft-cap give 0 at score 0, the
+    # position biases (at score 0) 0 where kv_idx == q_idx; `same` below allows 1e-6
+    at_zero = out[2].abs() > 1e-6
+    scaling = not bool(at_zero.any())
+    biasing = not bool(at_zero.diagonal(dim1=-2, dim2=-1).any())
+    if not scaling and not biasing:
         return None
     shape = shape5
 
@@ -171,11 +198,11 @@ def _probe_score_mod(fn: Callable, H: int, shape: Optional[Tuple[int, int, int, 
         ref = torch.broadcast_to(_f32(c(s.expand(shape), b, h, q, kv)), shape).cpu()
         return bool(torch.allclose(out, ref, rtol=1e-6, atol=1e-6))
 
-    cands = [IDENTITY]
+    cands = [IDENTITY] if scaling else []
     # multiplicative checkerboards: read both factors off two grid points
     with torch.no_grad():
         one = out[4] / 2.5  # score 2.5
-        for i0 in (0, 1):
+        for i0 in (0, 1) if scaling else ():
             f_even = one[0, 0, 0, 0].item()
             f_odd = one[0, 0, 0, 1].item()
             cands.append(ScoreMod(_lib.SCORE_CHECKERBOARD, f_even, f_odd, i0, name=getattr(fn, "__name__", "checkerboard")))
@@ -185,6 +212,8 @@ def _probe_score_mod(fn: Callable, H: int, shape: Optional[Tuple[int, int, int, 
         cands.append(ScoreMod(_lib.SCORE_REL_BIAS, bias[0, 0, 0, 1].item(), name=getattr(fn, "__name__", "rel_bias")))
         # tanh soft-cap: cap from the saturated value
         try:
+            if not scaling:
+                raise ValueError("not a soft-cap")
             big = fn(torch.full((1, 1, 1, 1, 1), 1e9, device=s.device), b[:, :1], h[:, :, :1], q[..., :1, :], kv[..., :1])
             cap = float(torch.as_tensor(big).reshape(-1)[0])
             if math.isfinite(cap) and cap > 0:
@@ -226,13 +255,18 @@ def _same_on_full_range(fn: Callable, cand: "ScoreMod", shape: Tuple[int, int, i
     return True
 
 
-def affine_score_mod(fn: Callable, B: int, H: int, Lq: int, Lkv: int, device) -> Optional[ScoreMod]:
+def affine_score_mod(fn: Callable, B: int, H: int, Lq: int, Lkv: int, device, corner: Optional[torch.Tensor] = None
+                     ) -> Optional[ScoreMod]:
     """Lower a score_mod that is affine in the score, mod(s) = mul[b,h,q,kv] * s + add[b,h,q,kv], to dense
     fp32 tables read off the callable on the device (what attention.py:59-63 evaluates per element;
     captured tensors such as bias tables, attention.py:22-23, are simply part of the callable).
+    `corner`: the callable's values on a corner of the index space if they are known (_probe_score_mod).
     Returns None when the callable is not affine in the score."""
     # affinity, on a small CPU grid: five score values must lie on one line per (b, h, q, kv)
     P = 5
+    near = (min(B, 2), H, min(Lq, P), min(Lkv, P + 2))
+    if corner is not None and all(have >= want for have, want in zip(corner.shape[1:], near)):
+        return _affine_tables(fn, B, H, Lq, Lkv, device, corner[:, :near[0], :near[1], :near[2], :near[3]])
     s = torch.tensor([-1.75, -0.5, 0.0, 0.625, 2.5], dtype=torch.float32).reshape(5, 1, 1, 1, 1)
     b = torch.arange(min(B, 2), dtype=torch.int32).reshape(1, -1, 1, 1, 1)
     h = torch.arange(H, dtype=torch.int32).reshape(1, 1, H, 1, 1)
@@ -249,9 +283,32 @@ def affine_score_mod(fn: Callable, B: int, H: int, Lq: int, Lkv: int, device) ->
             continue
     if out is None:
         return None
+    return _affine_tables(fn, B, H, Lq, Lkv, device, out)
+
+
+def _affine_tables(fn: Callable, B: int, H: int, Lq: int, Lkv: int, device, out: torch.Tensor) -> Optional[ScoreMod]:
+    """affine_score_mod past its corner grid, whose values are `out` [scores, b, h, q, kv]."""
+    s = torch.tensor(_CORNER_SCORES).reshape(5, 1, 1, 1, 1)
     a0, c0 = (out[4] - out[2]) / 2.5, out[2]
     if not torch.isfinite(out).all() or not torch.allclose(out, a0 * s + c0, rtol=1e-5, atol=1e-5):
         return None
+    name = getattr(fn, "__name__", "affine_score_mod")
+    # One call of the callable at all six scores, one kernel that makes the tables and checks them on every position, one
+    # wait -- as long as six planes are small (a corner that does not vary over the batch counts as one that has no batch
+    # extent); larger problems are read off and checked piece by piece below.
+    planes = (1 if bool((out == out[:, :1]).all()) else B) * H * Lq * Lkv
+    if torch.device(device).type == "cuda" and planes <= _SIX_PLANES_ELEMS:
+        try:
+            y = torch.as_tensor(fn(*_grid5(_TABLE_SCORES, (B, H, Lq, Lkv), device))).to(torch.float32)
+            y = y.reshape((1,) * (5 - y.dim()) + tuple(y.shape))
+            extents = tuple(y.shape[1:4])
+            if y.shape[0] not in (1, 6) or y.shape[4] not in (1, Lkv) or any(e not in (1, n) for e, n in zip(extents, (B, H, Lq))):
+                y = None
+        except Exception:   # (what a callable raises on five-dimensional tensors it may not raise on four)
+            y = None
+        if y is not None:
+            y = torch.broadcast_to(y, (6, *extents, Lkv)).contiguous()
+            return _tables_of_planes(fn, name, y, Lq)
     # the tables, on the device; a [1,1,1,1] score keeps every extent the callable does not use at 1
     bi = torch.arange(B, dtype=torch.int32, device=device).reshape(B, 1, 1, 1)
     hi = torch.arange(H, dtype=torch.int32, device=device).reshape(1, H, 1, 1)
@@ -291,7 +348,7 @@ def affine_score_mod(fn: Callable, B: int, H: int, Lq: int, Lkv: int, device) ->
     mul = None if bool(((mul - 1).abs() <= 1e-6).all()) else torch.broadcast_to(mul, shp).contiguous()
     if add is None and mul is None:
         return IDENTITY
-    spec = ScoreMod(_lib.SCORE_AFFINE, name=getattr(fn, "__name__", "affine_score_mod"), mul=mul, add=add, fn=fn)
+    spec = ScoreMod(_lib.SCORE_AFFINE, name=name, mul=mul, add=add, fn=fn)
     if (mul is None and add.shape[2] == Lq and Lq > 1 and Lkv > 1
             and bool(torch.equal(add[:, :, 1:, 1:], add[:, :, :-1, :-1]))):
         # constant along every diagonal: first column upwards (kv - q = -(Lq-1) .. 0), then first row (1 .. Lkv-1)
@@ -300,6 +357,30 @@ def affine_score_mod(fn: Callable, B: int, H: int, Lq: int, Lkv: int, device) ->
     return spec
 
 
+def _tables_of_planes(fn: Callable, name: str, y: torch.Tensor, Lq: int) -> Optional[ScoreMod]:
+    """The tables of a callable whose values at _TABLE_SCORES are the planes y [6, b', h', q', Lkv], or None where they do
+    not reproduce them."""
+    _, b, h, rows, Lkv = y.shape
+    add, mul = torch.empty_like(y[0]), torch.empty_like(y[0])
+    diag = torch.empty((b, h, rows + Lkv - 1), dtype=torch.float32, device=y.device) if rows == Lq > 1 and Lkv > 1 else None
+    flags = torch.zeros(4, dtype=torch.int32, device=y.device)
+    with torch.cuda.device(y.device):
+        rc = _lib.lib().flexattn_affine_tables(y.data_ptr(), b * h, rows, Lkv, add.data_ptr(), mul.data_ptr(),
+                                               diag.data_ptr() if diag is not None else None, flags.data_ptr(),
+                                               torch.cuda.current_stream(y.device).cuda_stream)
+    _lib.check(rc, "flexattn_affine_tables")
+    bad, adds, scales, bends = flags.tolist()
+    if bad:
+        return None
+    if not adds and not scales:
+        return IDENTITY
+    spec = ScoreMod(_lib.SCORE_AFFINE, name=name, mul=mul if scales else None, add=add if adds else None, fn=fn)
+    if adds and not scales and diag is not None and not bends:
+        spec.add, spec.diag_zero = diag, Lq - 1
+    return spec
+
+
+_SIX_PLANES_ELEMS = 1 << 26    # positions up to which a callable is evaluated at six scores in one call (1.6 GB)
 _score_cache: dict = {}
 
 
@@ -325,8 +406,9 @@ def resolve_score_mod(fn: Optional[Callable], H: int, shape: Optional[Tuple[int,
         hit = None
     if hit is not None and hit[1] is not None:
         return hit[1]
+    corner: list = []
     if hit is None:   # (a cached None says: probed before, not one of the families)
-        spec = _probe_score_mod(fn, H, shape, device)
+        spec = _probe_score_mod(fn, H, shape, device, corner)
         if stamp is not None:
             if len(_score_cache) > 64:
                 _score_cache.clear()
@@ -338,7 +420,7 @@ def resolve_score_mod(fn: Optional[Callable], H: int, shape: Optional[Tuple[int,
         hit = _score_cache.get(key)
         if hit is not None and _same_callable(hit[0], fn) and stamp is not None and _stamp_valid(hit[2], stamp):
             return hit[1]
-        spec = affine_score_mod(fn, *shape, device)
+        spec = affine_score_mod(fn, *shape, device, corner[0] if corner else None)
         if spec is not None:
             if len(_score_cache) > 64:
                 _score_cache.clear()

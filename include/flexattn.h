@@ -222,6 +222,15 @@ int flexattn_pack_mask(const uint8_t* mask, const int64_t* strides, int32_t nb, 
  * (lo, hi = fit[2] - 1, sink = fit[3] - 1) and (lo, hi, no sink) miss any entry of it. */
 int flexattn_bitmap_fit(const int32_t* bits, int32_t n_maps, int32_t Qp, int32_t KVp, int32_t* fit, flexattn_stream_t stream);
 
+/* Lowering of a score_mod that is affine in the score: `values` [6, maps, rows, cols] holds the callable at the scores 0,
+ * 8, -8, 0.625, -1.75 and 3.25.  Writes add = values at 0 and mul = (values at 8 - values at -8) / 16 ([maps, rows, cols]) and
+ * sets (never clears) flags[0] where the tables are not finite or do not reproduce the other three scores to 1e-5,
+ * flags[1] where add has a nonzero, flags[2] where mul differs from 1 by more than 1e-6 and, with diag ([maps,
+ * rows + cols - 1], may be NULL), flags[3] where add is not constant along its diagonals; diag[kv - q + rows - 1] is the
+ * value of a diagonal.  Replaces the element-wise mod of flaxattention/core/attention.py:59-63. */
+int flexattn_affine_tables(const float* values, int64_t maps, int32_t rows, int32_t cols, float* add, float* mul, float* diag,
+                           int32_t* flags, flexattn_stream_t stream);
+
 /* Forward.  With FLEX_PARITY and lse2 == NULL the log-sum-exp that the second pass reads is kept
  * in `workspace` (flexattn_fwd_workspace_bytes); otherwise workspace may be NULL.  A workspace
  * of that size also lets the matrix-core kernels split calls with few query rows against many

@@ -1190,3 +1190,42 @@ def test_backward_split_over_the_queries(dev, dtype, B, Hq, Hkv, Lq, Lkv, D, kin
         # one rounding of the result, and for entries that cancel the float32 sums' own error (2^-24 of what they add up)
         eps = 2.0 ** (-7 if dtype == torch.bfloat16 else -10)
         assert ((a.float() - b.float()).abs() <= eps * b.float().abs() + 1e-5 * b.float().abs().max()).all(), name
+
+
+@pytest.mark.parametrize("B,H,Lq,Lkv", [(2, 3, 70, 90), (1, 1, 1, 300), (3, 2, 257, 2), (1, 4, 33, 1)])
+def test_affine_lowering_in_one_call_equals_the_general_path(dev, B, H, Lq, Lkv, monkeypatch):
+    """A score_mod that captures tables is read off by one call at six scores and one kernel while the problem is small,
+    piece by piece where it is not: the same verdict, the same tables, the same diagonal form."""
+    from flaxattention_amd.core import common
+    print("case affine lowering", B, H, Lq, Lkv, flush=True)
+    g = torch.Generator(device=dev).manual_seed(6)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev)
+    rel, dense, row, per_b, gain = rnd(H, Lq + Lkv), rnd(H, Lq, Lkv), rnd(Lq), rnd(B), rnd(H, Lkv)
+    hole = dense.clone()
+    hole[-1, -1, -1] = float("inf")
+    mods = {
+        "diagonal": lambda s, b, h, q, kv: s + rel[h, kv - q + Lq - 1],
+        "dense": lambda s, b, h, q, kv: s + dense[h, q, kv],
+        "rows": lambda s, b, h, q, kv: s + row[q],
+        "batch": lambda s, b, h, q, kv: s * 1.5 + per_b[b],
+        "gain": lambda s, b, h, q, kv: s * gain[h, kv],
+        "both": lambda s, b, h, q, kv: s * gain[h, kv] + dense[h, q, kv],
+        "constant": lambda s, b, h, q, kv: s * 0.0 + rel[0, 0],
+        "nothing": lambda s, b, h, q, kv: s + 0.0 * rel[h, 0],
+        "not finite": lambda s, b, h, q, kv: s + hole[h, q, kv],
+        "bends": lambda s, b, h, q, kv: torch.where(q + kv == Lq + Lkv - 2, s * s, s) + rel[h, kv],
+        "half": lambda s, b, h, q, kv: (s + dense[h, q, kv]).to(torch.bfloat16),
+    }
+    for name, fn in mods.items():
+        fast = common.affine_score_mod(fn, B, H, Lq, Lkv, dev)
+        monkeypatch.setattr(common, "_SIX_PLANES_ELEMS", 0)
+        slow = common.affine_score_mod(fn, B, H, Lq, Lkv, dev)
+        monkeypatch.undo()
+        assert (fast is None) == (slow is None), name
+        if fast is None:
+            continue
+        assert fast.kind == slow.kind and fast.diag_zero == slow.diag_zero, name
+        for a, b_ in ((fast.mul, slow.mul), (fast.add, slow.add)):
+            assert (a is None) == (b_ is None), name
+            assert a is None or torch.equal(a.expand(b_.shape), b_), name
+    assert common.affine_score_mod(mods["not finite"], B, H, Lq, Lkv, dev) is None
