@@ -406,12 +406,7 @@ __global__ __launch_bounds__(DkvShape<D>::kThreads, D == 64 ? 2 : 1) void bwd_dk
   const int nkt = (p.Lkv + BN - 1) / BN;
   int kt, bh;  // early key tiles see the most queries under causal masks
   int wid = blockIdx.x, part = 0;
-  if constexpr (SPLIT) {
-    // the parts of a tile stay on one XCD (they read the same K and V) and next to each other in the order
-    const int parts = parts_g * parts_t, run = (p.Hkv * p.B) % 8 ? 1 : 8;
-    part = wid / run % parts;
-    wid = wid / (run * parts) * run + wid % run;
-  }
+  if constexpr (SPLIT) dkv_part_map(p.Hkv * p.B, parts_g * parts_t, wid, part);
   xcd_tile_map(wid, nkt, p.Hkv * p.B, kt, bh);
   const int hk = bh % p.Hkv, b = bh / p.Hkv, G = p.Hq / p.Hkv;
   const int kv_col = kt * BN + wk * 32 + i32;
@@ -681,23 +676,7 @@ __global__ __launch_bounds__(DkvShape<D>::kThreads, D == 64 ? 2 : 1) void bwd_dk
   }
 
   if constexpr (SPLIT) {
-    // [part][tile][wave][dk | dv][register quad][lane]: every store instruction fills 1 KB
-    float4_t* out = reinterpret_cast<float4_t*>(partial) +
-                    ((((int64_t)part * p.B * p.Hkv + bh) * nkt + kt) * DkvShape<D>::kWaves + wk) * (2 * DB * 4 * 64) + lane;
-    const float dk_scale = PARITY ? 1.f : p.scale * key_grad;
-#pragma unroll
-    for (int db = 0; db < DB; db++)
-#pragma unroll
-      for (int rr = 0; rr < 4; rr++) {
-        float4_t a, c;
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          a[e] = dkacc[db][4 * rr + e] * dk_scale;
-          c[e] = dvacc[db][4 * rr + e];
-        }
-        out[(db * 4 + rr) * 64] = a;
-        out[((DB + db) * 4 + rr) * 64] = c;
-      }
+    store_dkv_part<DB>(partial, ((int64_t)part * p.B * p.Hkv + bh) * nkt + kt, wk, lane, dkacc, dvacc, PARITY ? 1.f : p.scale * key_grad);
     return;
   }
   if (kv_col < p.Lkv) {
@@ -718,28 +697,6 @@ __global__ __launch_bounds__(DkvShape<D>::kThreads, D == 64 ? 2 : 1) void bwd_dk
         *reinterpret_cast<uint2*>(dkp + 32 * db + 8 * rr) = pk.u;
         *reinterpret_cast<uint2*>(dvp + 32 * db + 8 * rr) = pv.u;
       }
-  }
-}
-
-// adds the partial sums of a split dK/dV call: one workgroup per (key tile, wave of it), coalesced reads of every part
-template <typename T, int D>
-__global__ __launch_bounds__(256) void dkv_combine_kernel(const float* __restrict__ partial, int parts, int nkt, int Lkv,
-                                                          T* __restrict__ dk, T* __restrict__ dv) {
-  constexpr int DB = D / 32, kWaves = DkvShape<D>::kWaves, kQuads = 2 * DB * 4 * 64;
-  const int wk = blockIdx.x % kWaves, kt = blockIdx.x / kWaves % nkt, bh = blockIdx.x / (kWaves * nkt);
-  const float4_t* in = reinterpret_cast<const float4_t*>(partial) + (int64_t)blockIdx.x * kQuads;
-  const int64_t part_stride = (int64_t)gridDim.x * kQuads;
-  for (int i = threadIdx.x; i < kQuads; i += 256) {
-    float4_t sum = in[i];
-    for (int s = 1; s < parts; s++) sum += in[s * part_stride + i];
-    const int lane = i & 63, quad = i >> 6, db = quad / 4 % DB;
-    const int kv = kt * kListBN + wk * 32 + (lane & 31);
-    if (kv >= Lkv) continue;
-    union { T e[4]; uint2 u; } pk;
-#pragma unroll
-    for (int e = 0; e < 4; e++) pk.e[e] = (T)sum[e];
-    T* out = quad < DB * 4 ? dk : dv;
-    *reinterpret_cast<uint2*>(out + ((int64_t)bh * Lkv + kv) * D + 32 * db + 8 * (quad & 3) + 4 * (lane >> 5)) = pk.u;
   }
 }
 
@@ -774,7 +731,7 @@ static int launch_dkv_form(const FlexAttnParams& p, const BwdArgs& a) {
                      sm, a.s, p, (const T*)a.q, (const T*)a.k, (const T*)a.v, a.lse2, a.delta, (const T*)a.d_o, (T*)a.dk,
                      (T*)a.dv, a.parts_g, a.parts_t, a.partial);
   if constexpr (SPLIT)
-    hipLaunchKernelGGL((dkv_combine_kernel<T, D>), dim3(tiles * DkvShape<D>::kWaves), dim3(256), 0, a.s, a.partial, parts, nkt,
+    hipLaunchKernelGGL((dkv_combine_kernel<T, D>), dim3(tiles * 4), dim3(256), 0, a.s, a.partial, parts, nkt,
                        p.Lkv, (T*)a.dk, (T*)a.dv);
   return 0;
 }

@@ -37,17 +37,16 @@ bool flex_mfma_bwd_supported(const FlexAttnParams& p) {
   return true;
 }
 
-// How many workgroups share a key tile of the dK/dV kernel: parts_g over the query heads of the group times parts_t over
-// each head's list of query tiles.  A key tile's workgroup visits up to `visits` query tiles; under a mask the work of
-// the tiles differs (causal: the heaviest is twice the mean), so with no more tiles than compute units slots the
-// heaviest one is the call: bf16 [1,32->8,4096,128] causal, 256 tiles on 256 slots, 637 us against 398 + 14 us in two parts.
-// Counted in tile visits (about 5 us each), with what adding the partial sums costs in the same unit (4 us, and 27 us
-// for the 67 MB that twice the slots write and read); taken where it promises a fifth and 30 us
+// How many workgroups share a key tile of a dK/dV kernel of which the chip holds `slots` at once: n.g over the query heads
+// of the group times n.t over each head's list of query tiles.  A key tile's workgroup visits up to `visits` query tiles
+// of visit_us each; under a mask the work of the tiles differs (causal: the heaviest is twice the mean), so with no more
+// tiles than slots the heaviest one is the call: bf16 [1,32->8,4096,128] causal, 256 tiles on 256 slots, 637 us against
+// 398 + 14 us in two parts; f16 [2,8,2048,256] causal 214 us against
+// 148 + 27 us.  What adding the partial sums costs: a launch, and their
+// bytes twice (27 us for twice 256 slots at D = 128, about half of it hidden).  Taken where it promises a fifth and 30 us
 // (less is lost again on the second launch where the host sets the pace: bf16 [1,4,881,64] causal 131 -> 145 us).
-struct DkvParts { int g, t; };
-static DkvParts dkv_parts(const FlexAttnParams& p) {
-  if ((p.D != 64 && p.D != 128) || (p.flags & (FLEX_UNROUNDED | FLEX_NO_SPLIT))) return {1, 1};
-  const double slots = (double)flex_cu_count() * (p.D == 64 ? 2 : 1);   // workgroups the chip holds at once
+DkvParts flex_dkv_parts(const FlexAttnParams& p, double slots, double visit_us) {
+  if (p.flags & (FLEX_UNROUNDED | FLEX_NO_SPLIT)) return {1, 1};
   const double tiles = (double)((p.Lkv + kListBN - 1) / kListBN) * p.Hkv * p.B;
   const int G = p.Hq / p.Hkv, nqt = (p.Lq + kBM - 1) / kBM;
   // what a tile's list holds is on the device: bitmaps (documents) count as a quarter full, a window without sink keys
@@ -56,15 +55,15 @@ static DkvParts dkv_parts(const FlexAttnParams& p) {
   if (p.mask.kind == FLEX_MASK_BITS) listed = fmax(1.0, 0.25 * nqt);
   else if (p.mask.hi != INT32_MAX && p.mask.sink < 0 && p.mask.lo != INT32_MIN)
     listed = fmin(nqt, fmax(0.0, (double)p.mask.hi - p.mask.lo) / kBM + 2);
-  const double visits = G * listed;
+  const double visits = G * listed, part_us = 2. * kListBN * 2 * p.D * sizeof(float) / 5e6;
   const bool uneven = p.tiles_bwd.kv_num || !mask_hides_nothing(p.mask);
   auto cost = [&](int parts) {
-    const double each = visits / parts, rounds = ceil(tiles * parts / slots);
-    const double run = uneven ? fmax(each, 0.5 * visits * tiles / slots) : each * rounds;
-    return parts == 1 ? (uneven ? fmax(visits, 0.5 * visits * tiles / slots) : run) : run + 1 + 2.7 * tiles * parts / slots;
+    const double rounds = ceil(tiles * parts / slots);
+    const double run = uneven ? fmax(visits / parts, 0.5 * visits * tiles / slots) : visits / parts * rounds;
+    return run * visit_us + (parts > 1 ? 4 + tiles * parts * part_us : 0);
   };
   DkvParts best = {1, 1};
-  double least = fmin(0.8 * cost(1), cost(1) - 6);
+  double least = fmin(0.8 * cost(1), cost(1) - 30);
   for (int parts = 2; parts <= 16 && parts <= visits && tiles * parts <= 2 * slots; parts++) {
     int g = parts < G ? parts : G;
     while (G % g || parts % g) g--;   // whole heads first, stretches of the lists for the rest
@@ -74,14 +73,20 @@ static DkvParts dkv_parts(const FlexAttnParams& p) {
   }
   return best;
 }
-
-// beside delta, which the caller accounts for: the partial sums of a split dK/dV call
-size_t flex_mfma_bwd_workspace(const FlexAttnParams& p) {
-  const DkvParts n = dkv_parts(p);
+size_t flex_dkv_partial_bytes(const FlexAttnParams& p, DkvParts n) {
   if (n.g * n.t == 1) return 0;
   const size_t rows = (size_t)((p.Lkv + kListBN - 1) / kListBN) * kListBN * p.Hkv * p.B;
   return (size_t)n.g * n.t * rows * 2 * p.D * sizeof(float);
 }
+
+// two workgroups share a compute unit at D = 64, one has it at D = 128 (and 192 / 256 go to the simple kernel)
+static DkvParts dkv_parts(const FlexAttnParams& p) {
+  if (p.D != 64 && p.D != 128) return {1, 1};
+  return flex_dkv_parts(p, flex_cu_count() * (p.D == 64 ? 2 : 1), 5.);
+}
+
+// beside delta, which the caller accounts for: the partial sums of a divided dK/dV call
+size_t flex_mfma_bwd_workspace(const FlexAttnParams& p) { return flex_dkv_partial_bytes(p, dkv_parts(p)); }
 
 int flex_mfma_bwd(const FlexAttnParams& p, const void* q, const void* k, const void* v, const void* o, const float* lse2,
                   const void* d_o, void* dq, void* dk, void* dv, void* workspace, hipStream_t s) {

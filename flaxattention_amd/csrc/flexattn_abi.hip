@@ -64,6 +64,7 @@ int flex_simple_fwd_splits(const FlexAttnParams& p);
 size_t flex_simple_fwd_partial_bytes(const FlexAttnParams& p, int splits);
 int flex_simple_fwd(const FlexAttnParams& p, const void* q, const void* k, const void* v, void* o, float* lse2, int splits,
                     void* partials, hipStream_t s);
+size_t flex_simple_bwd_workspace(const FlexAttnParams& p);
 int flex_simple_bwd(const FlexAttnParams& p, const void* q, const void* k, const void* v, const void* o, const float* lse2,
                     const void* d_o, void* dq, void* dk, void* dv, void* workspace, hipStream_t s);
 
@@ -201,7 +202,8 @@ static size_t delta_bytes(const FlexAttnParams* p) { return ((size_t)p->B * p->H
 extern "C" size_t flexattn_bwd_workspace_bytes(const FlexAttnParams* p) {
   if (!p) return 0;
   size_t n = delta_bytes(p);
-  if (!(p->flags & (FLEX_FORCE_GENERIC | FLEX_STRICT)) && flex_mfma_bwd_supported(*p)) n += flex_mfma_bwd_workspace(*p);
+  if (wants_fused(p) && flex_simple_supported(*p, 1)) n += flex_simple_bwd_workspace(*p);
+  else if (wants_fused(p) && flex_mfma_bwd_supported(*p)) n += flex_mfma_bwd_workspace(*p);
   return n;
 }
 

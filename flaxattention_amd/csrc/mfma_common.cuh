@@ -554,4 +554,59 @@ __device__ __forceinline__ void xcd_tile_map(int wid, int ntile, int nbh, int& r
   }
 }
 
+// ---- dK/dV calls divided over the queries ----
+// `parts` workgroups share a tile of 128 keys (four waves of 32) and leave float32 partial sums of dK and dV.
+struct DkvParts { int g, t; };   // parts: over the query heads of the group, and over each head's list of query tiles
+
+// workgroup id -> (tile's id, part): the parts of a tile stay on one XCD (they read the same K and V) and next to each
+// other in the order
+__device__ __forceinline__ void dkv_part_map(int nbh, int parts, int& wid, int& part) {
+  const int run = nbh % 8 ? 1 : 8;
+  part = wid / run % parts;
+  wid = wid / (run * parts) * run + wid % run;
+}
+
+// [part and tile][wave][dk | dv][register quad][lane]: every store instruction fills 1 KB
+template <int DB>
+__device__ __forceinline__ void store_dkv_part(float* partial, int64_t tile, int wave, int lane, const float16_t (&dk)[DB],
+                                               const float16_t (&dv)[DB], float dk_scale) {
+  float4_t* out = reinterpret_cast<float4_t*>(partial) + (tile * 4 + wave) * (2 * DB * 4 * 64) + lane;
+#pragma unroll
+  for (int db = 0; db < DB; db++)
+#pragma unroll
+    for (int rr = 0; rr < 4; rr++) {
+      float4_t a, c;
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        a[e] = dk[db][4 * rr + e] * dk_scale;
+        c[e] = dv[db][4 * rr + e];
+      }
+      out[(db * 4 + rr) * 64] = a;
+      out[((DB + db) * 4 + rr) * 64] = c;
+    }
+}
+
+// adds the partial sums: one workgroup per (key tile, wave of it), coalesced reads of every part
+template <typename T, int D>
+__global__ __launch_bounds__(256) void dkv_combine_kernel(const float* __restrict__ partial, int parts, int nkt, int Lkv,
+                                                          T* __restrict__ dk, T* __restrict__ dv) {
+  constexpr int DB = D / 32, kQuads = 2 * DB * 4 * 64;
+  struct alignas(4 * sizeof(T)) Quad { T e[4]; };
+  const int wk = blockIdx.x % 4, kt = blockIdx.x / 4 % nkt, bh = blockIdx.x / (4 * nkt);
+  const float4_t* in = reinterpret_cast<const float4_t*>(partial) + (int64_t)blockIdx.x * kQuads;
+  const int64_t part_stride = (int64_t)gridDim.x * kQuads;
+  for (int i = threadIdx.x; i < kQuads; i += 256) {
+    float4_t sum = in[i];
+    for (int s = 1; s < parts; s++) sum += in[s * part_stride + i];
+    const int lane = i & 63, quad = i >> 6, db = quad / 4 % DB;
+    const int kv = kt * 128 + wk * 32 + (lane & 31);
+    if (kv >= Lkv) continue;
+    Quad pk;
+#pragma unroll
+    for (int e = 0; e < 4; e++) pk.e[e] = (T)sum[e];
+    T* out = quad < DB * 4 ? dk : dv;
+    *reinterpret_cast<Quad*>(out + ((int64_t)bh * Lkv + kv) * D + 32 * db + 8 * (quad & 3) + 4 * (lane >> 5)) = pk;
+  }
+}
+
 }  // namespace flex

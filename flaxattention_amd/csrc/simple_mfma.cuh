@@ -499,12 +499,15 @@ __global__ __launch_bounds__(256) void simple_dq_kernel(FlexAttnParams p, const 
 // dV = P^T.dO and dK = scale * (P o (dP - delta) o g)^T . Q for the 128 keys of a workgroup (one 32-key block per
 // wave, a lane owns one key), summed over the query heads of the key head's group.  PARITY: dP is rounded through T
 // before delta is subtracted and the scale is applied before dS is rounded.
+// With parts_g * parts_t > 1 that many workgroups share a key tile and leave partial sums (dkv_combine_kernel), as in the
+// tuned kernel.
 template <typename T, int D, int KIND, bool PARITY>
 __global__ __launch_bounds__(256) void simple_dkv_kernel(FlexAttnParams p, const T* __restrict__ q,
                                                          const T* __restrict__ k, const T* __restrict__ v,
                                                          const float* __restrict__ lse2, const float* __restrict__ delta,
                                                          const T* __restrict__ d_o, T* __restrict__ dk,
-                                                         T* __restrict__ dv) {
+                                                         T* __restrict__ dv, int parts_g, int parts_t,
+                                                         float* __restrict__ partial) {
   typedef SimpleOps<T, D> Ops;
   constexpr int DB = D / 32, ROWE = Ops::ROWE;
   __shared__ __align__(16) T Qs[kSimpleStep * ROWE];
@@ -517,7 +520,9 @@ __global__ __launch_bounds__(256) void simple_dkv_kernel(FlexAttnParams p, const
   const int i32 = lane & 31, g = lane >> 5;
   const int nkt = (p.Lkv + kSimpleKvTile - 1) / kSimpleKvTile;
   int kt, bh;  // early key tiles see the most queries under causal masks
-  xcd_tile_map(blockIdx.x, nkt, p.Hkv * p.B, kt, bh);
+  int wid = blockIdx.x, part = 0;
+  if (partial) dkv_part_map(p.Hkv * p.B, parts_g * parts_t, wid, part);
+  xcd_tile_map(wid, nkt, p.Hkv * p.B, kt, bh);
   const int hk = bh % p.Hkv, b = bh / p.Hkv, G = p.Hq / p.Hkv;
   const int kv_col = kt * kSimpleKvTile + w * 32 + i32;
   const int kv_ld = min(kv_col, p.Lkv - 1);
@@ -534,14 +539,15 @@ __global__ __launch_bounds__(256) void simple_dkv_kernel(FlexAttnParams p, const
 
   const FlexTileLists& tl = p.tiles_bwd;
   Score2<KIND> sm;
-  for (int gi = 0; gi < G; gi++) {
+  for (int gi = part % parts_g; gi < G; gi += parts_g) {
     const int h = hk * G + gi;
     sm.init(p.score, p.scale, h, b, p.Lq, p.Lkv);
     const Mask2 visible(p.mask, b, h, p.Lkv);
     SimpleSteps st;
     st.init(tl.q_num, tl.q_idx, tl.full_q_num, tl.full_q_idx,
             (b * tl.stride_b + h * tl.stride_h) * tl.n_kv_blocks + kt, tl.n_q_blocks, tl.q_block, p.Lq, p.mask);
-    const int nt = st.count(), n_full_t = st.full_steps();
+    const int n_full_t = st.full_steps(), share = part / parts_g;
+    const int it0 = (int)((int64_t)st.count() * share / parts_t), nt = (int)((int64_t)st.count() * (share + 1) / parts_t);
     const T* qbase = q + b * p.q_stride[0] + h * p.q_stride[1];
     const int64_t rows0 = ((int64_t)b * p.Hq + h) * p.Lq;
     const T* dobase = d_o + rows0 * D;
@@ -558,9 +564,9 @@ __global__ __launch_bounds__(256) void simple_dkv_kernel(FlexAttnParams p, const
         dreg = delta[rows0 + q0 + tid];
       }
     };
-    int s_cur = nt > 0 ? st.at(0) : 0;
-    if (nt > 0) load_step(s_cur * kSimpleStep);
-    for (int it = 0; it < nt; it++) {
+    int s_cur = nt > it0 ? st.at(it0) : 0;
+    if (nt > it0) load_step(s_cur * kSimpleStep);
+    for (int it = it0; it < nt; it++) {
       const int q0 = s_cur * kSimpleStep;
       __syncthreads();  // the previous step's (or head's) reads are done
       qt.store(Qs, tid);
@@ -623,6 +629,10 @@ __global__ __launch_bounds__(256) void simple_dkv_kernel(FlexAttnParams p, const
   }
 
   const float out_scale = PARITY ? 1.f : p.scale;
+  if (partial) {
+    store_dkv_part<DB>(partial, ((int64_t)part * p.B * p.Hkv + bh) * nkt + kt, w, lane, dkacc, dvacc, out_scale);
+    return;
+  }
   if (kv_col < p.Lkv) {
     const int64_t row_id = ((int64_t)b * p.Hkv + hk) * p.Lkv + kv_col;
     T* dkp = dk + row_id * D + 4 * g;
@@ -650,6 +660,9 @@ struct SimpleArgs {
   // forward over split key ranges: shares per query tile (1 = none) and where their partial (O, m, l) go
   int splits;
   float *o_part, *ml_part;
+  // dK/dV divided over the queries: parts per key tile and where their partial sums go (null: none)
+  DkvParts parts;
+  float* dkv_partial;
 };
 
 template <typename T, int D, int KIND> void simple_launch_fwd(const FlexAttnParams& p, const SimpleArgs& a) {
@@ -680,7 +693,14 @@ template <typename T, int D, int KIND> void simple_launch_fwd(const FlexAttnPara
 }
 template <typename T, int D, int KIND> void simple_launch_bwd(const FlexAttnParams& p, const SimpleArgs& a) {
   const dim3 qgrid((p.Lq + kSimpleQTile - 1) / kSimpleQTile * p.Hq * p.B);
-  const dim3 kgrid((p.Lkv + kSimpleKvTile - 1) / kSimpleKvTile * p.Hkv * p.B), block(256);
+  const int nkt = (p.Lkv + kSimpleKvTile - 1) / kSimpleKvTile, tiles = nkt * p.Hkv * p.B;
+  const int parts = a.dkv_partial ? a.parts.g * a.parts.t : 1;
+  const dim3 kgrid(tiles * parts), block(256);
+  auto merge = [&] {
+    if (parts > 1)
+      hipLaunchKernelGGL((dkv_combine_kernel<T, D>), dim3(tiles * 4), block, 0, a.s, a.dkv_partial, parts, nkt, p.Lkv, (T*)a.dk,
+                         (T*)a.dv);
+  };
   const T *q = (const T*)a.q, *k = (const T*)a.k, *v = (const T*)a.v, *o = (const T*)a.o, *d_o = (const T*)a.d_o;
   if constexpr (SimpleOps<T, D>::kRounds) {  // the parity numerics exist where something is rounded
     if (p.flags & FLEX_PARITY) {
@@ -690,18 +710,22 @@ template <typename T, int D, int KIND> void simple_launch_bwd(const FlexAttnPara
         hipLaunchKernelGGL((simple_dq_kernel<T, D, KIND, kSimpleBwdParity>), qgrid, block, 0, a.s, p, q, k, v, o, a.lse2_in,
                            d_o, (T*)a.dq, a.delta);
       }
-      if (!(p.flags & FLEX_BWD_ONLY_DQ))
+      if (!(p.flags & FLEX_BWD_ONLY_DQ)) {
         hipLaunchKernelGGL((simple_dkv_kernel<T, D, KIND, true>), kgrid, block, 0, a.s, p, q, k, v, a.lse2_in, a.delta, d_o,
-                           (T*)a.dk, (T*)a.dv);
+                           (T*)a.dk, (T*)a.dv, a.parts.g, a.parts.t, a.dkv_partial);
+        merge();
+      }
       return;
     }
   }
   if (!(p.flags & FLEX_BWD_ONLY_DKV))
     hipLaunchKernelGGL((simple_dq_kernel<T, D, KIND, kSimpleBwdFast>), qgrid, block, 0, a.s, p, q, k, v, o, a.lse2_in, d_o,
                        (T*)a.dq, a.delta);
-  if (!(p.flags & FLEX_BWD_ONLY_DQ))
+  if (!(p.flags & FLEX_BWD_ONLY_DQ)) {
     hipLaunchKernelGGL((simple_dkv_kernel<T, D, KIND, false>), kgrid, block, 0, a.s, p, q, k, v, a.lse2_in, a.delta, d_o,
-                       (T*)a.dk, (T*)a.dv);
+                       (T*)a.dk, (T*)a.dv, a.parts.g, a.parts.t, a.dkv_partial);
+    merge();
+  }
 }
 template <typename T, int D, int KIND> void simple_launch(const FlexAttnParams& p, const SimpleArgs& a) {
   if (a.bwd) simple_launch_bwd<T, D, KIND>(p, a);
