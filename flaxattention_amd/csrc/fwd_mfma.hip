@@ -54,12 +54,22 @@ bool flex_mfma_fwd_supported(const FlexAttnParams& p) {
 // Shares of the key tiles a forward call is split into (1 = none): calls whose query tiles alone would leave most
 // compute units without a workgroup, or with one where two fit (at most one per compute unit) -- few rows against a
 // long key sequence -- are split until there are about two workgroups per compute unit, with at least 8 tiles of 64
-// keys each.
+// keys each.  A causal call with up to as many query tiles as fit at once waits for its heaviest tile, twice the mean:
+// such a call is halved where half of that tile's visits outweighs the merge of the partial outputs (a launch, and
+// their bytes twice at 5 TB/s) with a margin: f16 [2,8,2048,256] causal 126 -> 113 us, bf16 [1,8,4096,256] 273 -> 202,
+// [2,8,2048,192] 120 -> 110.  Where two workgroups share a compute unit the heaviest one has it to itself in the end, and
+// a key tile less saves little: [1,8,8192,128] 342 -> 301 us, but [2,16,2048,128] 99 -> 124, [1,16,4096,64] 126 -> 136 (so
+// not split), and nothing at D = 64.
 int flex_mfma_fwd_splits(const FlexAttnParams& p) {
   const int64_t wgs = (int64_t)((p.Lq + kFwdBM - 1) / kFwdBM) * p.Hq * p.B;
   const int slots = (p.D >= 192 ? 1 : 2) * flex_cu_count();  // 192- and 256-wide heads run one workgroup per compute unit
-  if (wgs > slots / 2) return 1;
   const int tiles = (p.Lkv + kFwdBN - 1) / kFwdBN;
+  if (wgs > slots / 2) {
+    const bool causal = p.mask.kind == FLEX_MASK_BAND && p.mask.lo != INT32_MIN && p.mask.hi == INT32_MAX && p.Lq > p.Lkv / 2;
+    const double visit_us = p.D >= 192 ? 4. : p.D == 128 ? 1.2 : 0.;   // what a key tile less of the heaviest workgroup saves
+    const double merge_us = 4 + (double)p.B * p.Hq * p.Lq * 2 * p.D * sizeof(float) * 2 / 5e6;
+    return causal && wgs <= slots && 0.5 * tiles * visit_us > 1.5 * merge_us ? 2 : 1;
+  }
   int s = (int)(slots / wgs);
   if (s > tiles / 8) s = tiles / 8;
   if (s > 64) s = 64;  // the merge kernel takes one split per lane

@@ -1232,3 +1232,27 @@ def test_affine_lowering_in_one_call_equals_the_general_path(dev, B, H, Lq, Lkv,
             assert (a is None) == (b_ is None), name
             assert a is None or torch.equal(a.expand(b_.shape), b_), name
     assert common.affine_score_mod(mods["not finite"], B, H, Lq, Lkv, dev) is None
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("B,H,Lq,Lkv,D,halved", [(2, 8, 2001, 2048, 256, True), (3, 5, 2048, 2000, 192, True),
+                                                 (1, 8, 7777, 8150, 128, True), (1, 16, 4096, 4096, 64, False)])
+def test_forward_with_uneven_tiles_is_halved(dev, dtype, B, H, Lq, Lkv, D, halved):
+    """A causal call with about as many query tiles as compute units hold is split in two over the keys: against the
+    undivided call, which rounds the same P (parity) or sums in another order: one rounding of the result."""
+    from flaxattention_amd import _lib
+    from flaxattention_amd.core.attention import _make_plan
+    print("case halved forward", dtype, B, H, Lq, Lkv, D, flush=True)
+    q, k, v = (t.to(dev) for t in seeded_qkv(B, H, H, Lq, Lkv, D, dtype))
+    bm = fa.create_block_mask(causal_mask, None, None, Lq, Lkv, device=dev)
+    plan = _make_plan(q, k, v, None, bm, None, D ** -0.5, None)
+    lse_part = (B * H * Lq * 4 + 255) // 256 * 256 if dtype == torch.bfloat16 else 0
+    rows = (B * H * Lq * 2 * (D + 2) * 4 + 255) // 256 * 256
+    assert _lib.lib().flexattn_fwd_workspace_bytes(plan.params(q, k, v, q)) - lse_part == (rows if halved else 0)
+    a, la = fa.flax_attention(q, k, v, block_mask=bm, return_lse=True)
+    b, lb = fa.flax_attention(q, k, v, block_mask=bm, return_lse=True, kernel_options={"split_kv": False})
+    assert (la - lb).abs().max().item() <= 1e-5   # float32 sums of up to 8150 terms in another order
+    # P is rounded to the dtype before its product: up to half a unit of it in every term, relative to the largest value
+    eps = torch.finfo(dtype).eps
+    assert ((a.float() - b.float()).abs() <= eps * (b.float().abs() + 0.5 * v.float().abs().max())).all()
+    assert rel_l2(a.float().cpu(), b.float().cpu()) <= eps / 2
