@@ -362,6 +362,149 @@ __global__ __launch_bounds__(256) void simple_fwd_kernel(FlexAttnParams p, const
   }
 }
 
+// The float32 forward of calls whose 128-row query tiles would leave compute units without a workgroup.  Bound there by a
+// wave's chain of matrix instructions (64 instructions of 64 cycles per 32 x 32 block at D = 64), so a workgroup takes 32 query rows
+// and its four waves take the key steps in turn, each with a softmax of its own, merged through LDS at the end: a quarter of
+// the chain on four times the workgroups.  Both operands come straight from global memory (a lane's half key row in 16-byte
+// pieces, V as whole 128-byte row segments), the next step's under the products of this one: no LDS and no barrier
+// in the loop.  [1,4,512,64] causal 48 -> 19 us, [1,4,256,128] 43 -> 19 us a call.
+template <typename T, int D, int KIND>
+__global__ __launch_bounds__(256) void simple_fwd_short_kernel(FlexAttnParams p, const T* __restrict__ q,
+                                                               const T* __restrict__ k, const T* __restrict__ v,
+                                                               T* __restrict__ o, float* __restrict__ lse2) {
+  typedef SimpleOps<T, D> Ops;
+  static_assert(!Ops::kRounds, "float32");
+  constexpr int DB = D / 32;
+  __shared__ float part_o[4][DB * 16][64];
+  __shared__ float part_m[4][32], part_l[4][32];
+
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int i32 = lane & 31, g = lane >> 5;
+  const int nqt = (p.Lq + 31) / 32;
+  int rank, bh;
+  xcd_tile_map(blockIdx.x, nqt, p.Hq * p.B, rank, bh);
+  const int qt = nqt - 1 - rank;  // late query rows see the most keys under causal masks
+  const int h = bh % p.Hq, b = bh / p.Hq, hk = h / (p.Hq / p.Hkv);
+  const int q_row = qt * 32 + i32;
+  const int64_t row_id = ((int64_t)b * p.Hq + h) * p.Lq + min(q_row, p.Lq - 1);
+
+  typename Ops::Resident qf;
+  Ops::load_resident(qf, q + b * p.q_stride[0] + h * p.q_stride[1] + (int64_t)min(q_row, p.Lq - 1) * p.q_stride[2], g);
+
+  SimpleSteps st;
+  const FlexTileLists& tl = p.tiles;
+  st.init(tl.kv_num, tl.kv_idx, tl.full_kv_num, tl.full_kv_idx,
+          (b * tl.stride_b + h * tl.stride_h) * tl.n_q_blocks + qt / (kSimpleQTile / 32), tl.n_kv_blocks, tl.kv_block, p.Lkv, p.mask);
+  const int nt = st.count(), n_full_t = st.full_steps();
+
+  const T* kbase = k + b * p.k_stride[0] + hk * p.k_stride[1];
+  const T* vbase = v + b * p.v_stride[0] + hk * p.v_stride[1];
+  Score2<KIND> sm;
+  sm.init(p.score, p.scale, h, b, p.Lq, p.Lkv);
+  const Mask2 visible(p.mask, b, h, p.Lkv);
+
+  float16_t oacc[DB];
+#pragma unroll
+  for (int db = 0; db < DB; db++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) oacc[db][r] = 0.f;
+  float m_run = -INFINITY, l_run = 0.f;
+
+  struct Step {
+    typename Ops::Resident kf;
+    float vf[16][DB];
+    int kv0, cls;
+  };
+  // rows past the end are clamped to the last one (finite filler, masked out); a step that is entirely hidden from
+  // these 32 rows is not fetched
+  auto load = [&](Step& s, int it) {
+    s.kv0 = st.at(it) * kSimpleStep;
+    const bool masked = (it >= n_full_t) || (s.kv0 + kSimpleStep > p.Lkv);
+    s.cls = masked ? block_class(p.mask, visible, qt * 32, s.kv0, 0x7fffffff, p.Lkv) : (int)kBlockAll;
+    if (s.cls == kBlockNone) return;
+    Ops::load_resident(s.kf, kbase + (int64_t)min(s.kv0 + i32, p.Lkv - 1) * p.k_stride[2], g);
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      const T* row = vbase + (int64_t)min(s.kv0 + acc_row(r) + 4 * g, p.Lkv - 1) * p.v_stride[2] + i32;
+#pragma unroll
+      for (int db = 0; db < DB; db++) s.vf[r][db] = row[32 * db];
+    }
+  };
+  auto visit = [&](const Step& s) {
+    if (s.cls == kBlockNone) return;
+    float16_t x;
+#pragma unroll
+    for (int r = 0; r < 16; r++) x[r] = 0.f;
+#pragma unroll
+    for (int j = 0; j < D / 2; j++) x = Ops::mfma(s.kf.v[j], qf.v[j], x);  // S^T: rows = keys, the lane's column = its query row
+    sm.tile(q_row, s.kv0 + 4 * g);
+#pragma unroll
+    for (int r = 0; r < 16; r++) x[r] = sm.apply(x[r], acc_row(r));
+    if (s.cls == kBlockMixed) mask_block_q(x, p.mask, visible, q_row, s.kv0, g, p.Lkv);
+    const float m_new = fmaxf(m_run, xhalf_max(block_max(x)));
+    const float m_use = m_new == -INFINITY ? 0.f : m_new;  // nothing visible so far: P = 0 against any reference
+    const float alpha = fast_exp2(m_run - m_use);
+    float l_blk = 0.f;
+#pragma unroll
+    for (int r = 0; r < 16; r++) {
+      x[r] = fast_exp2(x[r] - m_use);
+      l_blk += x[r];
+    }
+    l_run = fmaf(l_run, alpha, l_blk);
+    m_run = m_new;
+#pragma unroll
+    for (int db = 0; db < DB; db++)
+#pragma unroll
+      for (int r = 0; r < 16; r++) oacc[db][r] *= alpha;
+#pragma unroll
+    for (int r = 0; r < 16; r++)
+#pragma unroll
+      for (int db = 0; db < DB; db++) oacc[db] = Ops::mfma(s.vf[r][db], x[r], oacc[db]);  // O^T += V^T.P^T
+  };
+  Step sa, sb;
+  if (w < nt) load(sa, w);
+  for (int it = w; it < nt; it += 8) {
+    if (it + 4 < nt) load(sb, it + 4);
+    visit(sa);
+    if (it + 4 < nt) {
+      if (it + 8 < nt) load(sa, it + 8);
+      visit(sb);
+    }
+  }
+
+  // ---- merge the four waves: wave w writes the quad w of every 32-column block ----
+  const float l_wave = xhalf_sum(l_run);
+  if (g == 0) { part_m[w][i32] = m_run; part_l[w][i32] = l_wave; }
+#pragma unroll
+  for (int db = 0; db < DB; db++)
+#pragma unroll
+    for (int r = 0; r < 16; r++) part_o[w][db * 16 + r][lane] = oacc[db][r];
+  __syncthreads();
+  const float m = fmaxf(fmaxf(part_m[0][i32], part_m[1][i32]), fmaxf(part_m[2][i32], part_m[3][i32]));
+  float sc[4], l_tot = 0.f;
+#pragma unroll
+  for (int u = 0; u < 4; u++) {
+    sc[u] = part_m[u][i32] == -INFINITY ? 0.f : fast_exp2(part_m[u][i32] - m);
+    l_tot = fmaf(part_l[u][i32], sc[u], l_tot);
+  }
+  if (q_row >= p.Lq) return;
+  const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+  T* op = o + b * p.o_stride[0] + h * p.o_stride[1] + (int64_t)q_row * p.o_stride[2] + 4 * g + 8 * w;
+#pragma unroll
+  for (int db = 0; db < DB; db++) {
+    float out[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      out[e] = 0.f;
+#pragma unroll
+      for (int u = 0; u < 4; u++) out[e] = fmaf(part_o[u][db * 16 + 4 * w + e][lane], sc[u], out[e]);
+    }
+    Ops::store4(op + 32 * db, out[0] * inv, out[1] * inv, out[2] * inv, out[3] * inv);
+  }
+  if (lse2 && w == 0 && g == 0) lse2[row_id] = l_tot > 0.f ? m + log2f(l_tot) : -INFINITY;
+}
+
 // MODE, as in the tuned dQ kernel:
 //   kSimpleBwdFast    delta_i = sum_d O_id dO_id - log2(e) d_lse2_i (written to delta_out for the dK/dV kernel),
 //                     dQ = scale * (P o (dP - delta) o g) . K
@@ -660,6 +803,7 @@ struct SimpleArgs {
   // forward over split key ranges: shares per query tile (1 = none) and where their partial (O, m, l) go
   int splits;
   float *o_part, *ml_part;
+  bool short_rows;  // forward of few query tiles: 32 rows per workgroup, the key steps divided over its waves
   // dK/dV divided over the queries: parts per key tile and where their partial sums go (null: none)
   DkvParts parts;
   float* dkv_partial;
@@ -684,6 +828,13 @@ template <typename T, int D, int KIND> void simple_launch_fwd(const FlexAttnPara
       hipLaunchKernelGGL((simple_fwd_kernel<T, D, KIND, kSimpleNorm>), grid, block, 0, a.s, p, q, k, v, (T*)a.out, a.lse2_out,
                          a.o_part, a.ml_part);
       merge((T*)a.out, nullptr);
+      return;
+    }
+  }
+  if constexpr (!SimpleOps<T, D>::kRounds) {
+    if (splits == 1 && a.short_rows) {
+      hipLaunchKernelGGL((simple_fwd_short_kernel<T, D, KIND>), dim3((p.Lq + 31) / 32 * p.Hq * p.B), block, 0, a.s, p, q, k, v,
+                         (T*)a.out, a.lse2_out);
       return;
     }
   }

@@ -53,7 +53,7 @@ static int dispatch(const FlexAttnParams& p, const SimpleArgs& a) {
 // Shares of the key steps a forward call is split into (1 = none): calls whose query tiles alone would leave most
 // compute units without a workgroup -- few rows against a long key sequence -- are split until there is about one
 // workgroup per compute unit, with at least 16 steps of 32 keys each.
-int flex_simple_fwd_splits(const FlexAttnParams& p) {
+static int splits_over_keys(const FlexAttnParams& p) {
   const int64_t wgs = (int64_t)((p.Lq + kSimpleQTile - 1) / kSimpleQTile) * p.Hq * p.B;
   const int cus = flex_cu_count();
   if (wgs > cus / 2) return 1;
@@ -63,6 +63,27 @@ int flex_simple_fwd_splits(const FlexAttnParams& p) {
   if (s > 64) s = 64;  // the merge kernel takes one split per lane
   return s < 2 ? 1 : s;
 }
+// Float32 forwards of few query tiles: 32 rows per workgroup with the key steps divided over its waves
+// (simple_fwd_short_kernel) instead of 128 rows.  Four times the workgroups with a quarter of the chain, so it wins while those
+// fit the chip about twice (causal: while the 128-row ones fit once, their tiles being uneven), and loses beyond, where
+// it only reads K and V four times as often.  us, 128 rows / 32 rows, D = 64 and 128: 8 tiles [1,4,256] causal 27 / 17
+// and 43 / 19; 16 tiles [1,4,512] 48 / 19 and 80 / 31; 128 tiles [4,8,512] dense 48 / 35 and 82 / 63; 192 tiles [8,8,384]
+// causal 38 / 30 and 63 / 53, dense 37 / 40; 256 tiles [8,16,256] causal 28 / 32, [4,8,1024] causal 92 / 73.  Against the split
+// over workgroups below, by their chains: 32 tiles [1,4,1024] 52 / 33, 128 tiles [2,8,1024] causal 60 / 39 but dense
+// 97 / 112 at D = 128.
+static bool short_rows(const FlexAttnParams& p) {
+  if (p.dtype != FLEX_F32 || (p.flags & FLEX_NO_SPLIT)) return false;
+  const int64_t wgs = (int64_t)((p.Lq + kSimpleQTile - 1) / kSimpleQTile) * p.Hq * p.B;
+  const int cus = flex_cu_count(), steps = (p.Lkv + kSimpleStep - 1) / kSimpleStep, splits = splits_over_keys(p);
+  const bool causal = p.mask.kind == FLEX_MASK_BAND && p.mask.lo != INT32_MIN && p.Lq > p.Lkv / 2;
+  if (wgs > cus / 2) return causal && wgs <= cus && steps >= 12;
+  if (splits == 1) return true;
+  double rounds = 4. * wgs / cus * (causal ? 0.5 : 1.);
+  if (rounds < 1) rounds = 1;
+  return 1.1 * rounds * steps / 4 <= (double)steps / splits;
+}
+int flex_simple_fwd_splits(const FlexAttnParams& p) { return short_rows(p) ? 1 : splits_over_keys(p); }
+
 // bytes of the partial (O, m, l) of a split forward
 size_t flex_simple_fwd_partial_bytes(const FlexAttnParams& p, int splits) {
   if (splits <= 1) return 0;
@@ -83,6 +104,7 @@ int flex_simple_fwd(const FlexAttnParams& p, const void* q, const void* k, const
   SimpleArgs a = {};
   a.q = q; a.k = k; a.v = v; a.out = o; a.lse2_out = lse2; a.s = s; a.bwd = false;
   a.splits = 1;
+  a.short_rows = short_rows(p);
   if (splits > 1 && partials) {
     if ((uintptr_t)partials & 15) {
       flex_set_error("matrix-core forward needs a 16-byte aligned workspace");

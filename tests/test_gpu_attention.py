@@ -1256,3 +1256,28 @@ def test_forward_with_uneven_tiles_is_halved(dev, dtype, B, H, Lq, Lkv, D, halve
     eps = torch.finfo(dtype).eps
     assert ((a.float() - b.float()).abs() <= eps * (b.float().abs() + 0.5 * v.float().abs().max())).all()
     assert rel_l2(a.float().cpu(), b.float().cpu()) <= eps / 2
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("B,Hq,Hkv,Lq,Lkv,kind", [
+    (1, 4, 4, 256, 256, "causal"), (1, 2, 1, 1, 33, "none"), (2, 3, 1, 31, 700, "causal"), (1, 8, 2, 97, 129, "window"),
+    (1, 1, 1, 640, 1000, "bitmap"), (8, 8, 8, 400, 400, "causal"), (2, 4, 4, 160, 1, "none"), (1, 4, 4, 300, 290, "hidden")])
+def test_short_float32_forward(dev, B, Hq, Hkv, Lq, Lkv, D, kind):
+    """Float32 forwards of few query tiles divide the key steps over the waves of a workgroup: against the oracle, with
+    rows that see nothing, ragged ends, fewer steps than waves, and with and without tile lists."""
+    print("case short f32", B, Hq, Hkv, Lq, Lkv, D, kind, flush=True)
+    hidden = lambda b, h, q, kv: (q >= 40) & (kv >= 7) & (q - kv < 100) & (q >= kv)   # noqa: E731
+    bitmap = lambda b, h, q, kv: (q * 7 + kv * 3) % 5 != 0                              # noqa: E731
+    mask, omask = {"causal": (causal_mask, o_causal_mask), "none": (None, None), "hidden": (hidden, hidden),
+                   "window": (generate_attention_sink(40, 3), o_attention_sink(40, 3)), "bitmap": (bitmap, bitmap)}[kind]
+    q, k, v = seeded_qkv(B, Hq, Hkv, Lq, Lkv, D, torch.float32)
+    bm = fa.create_block_mask(mask, None, None, Lq, Lkv, device=dev) if mask is not None else None
+    want, want_lse = ref_attention(q, k, v, o_alibi(Hq), omask, return_lse=True)
+    qd, kd, vd = (t.to(dev) for t in (q, k, v))
+    for opts in (None, {"tile_lists": False}, {"split_kv": False}):
+        out, lse = fa.flax_attention(qd, kd, vd, score_mod=generate_alibi_bias(Hq, 1.0), block_mask=bm, enable_gqa=Hq != Hkv,
+                                     return_lse=True, kernel_options=opts)
+        close(out, want, torch.float32, f"O {opts}")
+        dead = torch.isneginf(want_lse)
+        assert torch.equal(torch.isneginf(lse.cpu()), dead)
+        assert max_abs(lse.cpu()[~dead], want_lse[~dead]) <= 1e-4
