@@ -1281,3 +1281,24 @@ def test_short_float32_forward(dev, B, Hq, Hkv, Lq, Lkv, D, kind):
         dead = torch.isneginf(want_lse)
         assert torch.equal(torch.isneginf(lse.cpu()), dead)
         assert max_abs(lse.cpu()[~dead], want_lse[~dead]) <= 1e-4
+
+
+@pytest.mark.parametrize("gain", [0.5, 1.0, 3.0, 12.0])
+@pytest.mark.parametrize("D,cap", [(64, 50.0), (128, 50.0), (128, 7.0), (256, 20.0)])
+def test_softcap_polynomial_against_64_bits(dev, D, cap, gain):
+    """Blocks whose scores lie well below the cap take a polynomial for the tanh, others the exponential: gains that put
+    all, some and none of the blocks on either side.  The unrounded numerics carry float32 up to the results, so the
+    log-sum-exp shows the scores' own error: 2^-24 per operation on scores of up to cap, doubled for the sum over D."""
+    print("case softcap polynomial", D, cap, gain, flush=True)
+    B, H, L = 1, 2, 500
+    q, k, v = seeded_qkv(B, H, H, L, L, D, torch.float16)
+    q = (q.float() * gain).half()
+    bm = fa.create_block_mask(causal_mask, None, None, L, L, device=dev)
+    out, lse = fa.flax_attention(q.to(dev), k.to(dev), v.to(dev), score_mod=generate_tanh_softcap(cap), block_mask=bm,
+                                 return_lse=True, kernel_options={"numerics": "unrounded"})
+    x = cap * torch.tanh(q.double() @ k.double().transpose(-1, -2) * D ** -0.5 / cap)
+    x = x.masked_fill(~torch.ones(L, L, dtype=torch.bool).tril(), -float("inf"))
+    err = (lse.cpu().double() - torch.logsumexp(x, -1)).abs().max().item()
+    rel = rel_l2(out.float().cpu(), (torch.softmax(x, -1) @ v.double()).float())
+    print(f"  lse error {err:.2e}, O rel-L2 {rel:.2e}", flush=True)
+    assert err <= 8 * cap * 2 ** -24 + 4e-6 and rel <= 2 ** -11
