@@ -73,20 +73,31 @@ DkvParts flex_dkv_parts(const FlexAttnParams& p, double slots, double visit_us) 
   }
   return best;
 }
-size_t flex_dkv_partial_bytes(const FlexAttnParams& p, DkvParts n) {
-  if (n.g * n.t == 1) return 0;
-  const size_t rows = (size_t)((p.Lkv + kListBN - 1) / kListBN) * kListBN * p.Hkv * p.B;
-  return (size_t)n.g * n.t * rows * 2 * p.D * sizeof(float);
+// Bytes of the partial sums for the most parts any mask and lists can get: a workspace is sized by the shape alone.
+size_t flex_dkv_partial_bytes(const FlexAttnParams& p, double slots, double visit_us) {
+  if (p.flags & (FLEX_UNROUNDED | FLEX_NO_SPLIT)) return 0;
+  const int64_t tiles = (int64_t)((p.Lkv + kListBN - 1) / kListBN) * p.Hkv * p.B;
+  const int64_t visits = (int64_t)(p.Hq / p.Hkv) * ((p.Lq + kBM - 1) / kBM);
+  int64_t parts = (int64_t)(2 * slots) / tiles;
+  if (parts > 16) parts = 16;
+  if (parts > visits) parts = visits;
+  // (a call that cannot save 30 us is never divided; even tiles take more rounds than `visits` only beyond the slots)
+  if (parts < 2 || (double)visits * visit_us * fmax(1.0, ceil(tiles / slots)) <= 30) return 0;
+  return (size_t)parts * tiles * kListBN * 2 * p.D * sizeof(float);
 }
 
 // two workgroups share a compute unit at D = 64, one has it at D = 128 (and 192 / 256 go to the simple kernel)
+static double dkv_slots(const FlexAttnParams& p) { return flex_cu_count() * (p.D == 64 ? 2. : 1.); }
+constexpr double kVisitUs = 5.;
 static DkvParts dkv_parts(const FlexAttnParams& p) {
   if (p.D != 64 && p.D != 128) return {1, 1};
-  return flex_dkv_parts(p, flex_cu_count() * (p.D == 64 ? 2 : 1), 5.);
+  return flex_dkv_parts(p, dkv_slots(p), kVisitUs);
 }
 
 // beside delta, which the caller accounts for: the partial sums of a divided dK/dV call
-size_t flex_mfma_bwd_workspace(const FlexAttnParams& p) { return flex_dkv_partial_bytes(p, dkv_parts(p)); }
+size_t flex_mfma_bwd_workspace(const FlexAttnParams& p) {
+  return p.D == 64 || p.D == 128 ? flex_dkv_partial_bytes(p, dkv_slots(p), kVisitUs) : 0;
+}
 
 int flex_mfma_bwd(const FlexAttnParams& p, const void* q, const void* k, const void* v, const void* o, const float* lse2,
                   const void* d_o, void* dq, void* dk, void* dv, void* workspace, hipStream_t s) {

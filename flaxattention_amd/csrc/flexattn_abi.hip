@@ -42,7 +42,7 @@ int flex_generic_fwd(const FlexAttnParams& p, const void* q, const void* k, cons
 int flex_generic_bwd(const FlexAttnParams& p, const void* q, const void* k, const void* v, const float* lse2, const void* d_o,
                      void* dq, void* dk, void* dv, float* delta, hipStream_t s);
 bool flex_mfma_fwd_supported(const FlexAttnParams& p);
-int flex_mfma_fwd_splits(const FlexAttnParams& p);
+int flex_mfma_fwd_splits(const FlexAttnParams& p, bool any_mask);
 size_t flex_mfma_fwd_partial_bytes(const FlexAttnParams& p, int splits);
 int flex_mfma_fwd(const FlexAttnParams& p, const void* q, const void* k, const void* v, void* o, float* lse2, int splits,
                   void* partials, hipStream_t s);
@@ -60,7 +60,7 @@ size_t flex_decode_kept_bytes(const FlexAttnParams& p);
 void* flex_decode_static_scratch(size_t* bytes);
 void flex_mfma_tiles(int dtype, int D, int Dv, int which, int* qb, int* kvb);
 bool flex_simple_supported(const FlexAttnParams& p, int which);
-int flex_simple_fwd_splits(const FlexAttnParams& p);
+int flex_simple_fwd_splits(const FlexAttnParams& p, bool any_mask);
 size_t flex_simple_fwd_partial_bytes(const FlexAttnParams& p, int splits);
 int flex_simple_fwd(const FlexAttnParams& p, const void* q, const void* k, const void* v, void* o, float* lse2, int splits,
                     void* partials, hipStream_t s);
@@ -153,8 +153,8 @@ extern "C" size_t flexattn_fwd_workspace_bytes(const FlexAttnParams* p) {
   size_t n = fwd_lse_bytes(p);
   // the matrix-core forward kernels split the keys of a call with few query tiles over several workgroups, whose
   // partial results live here
-  if (wants_fused(p) && flex_mfma_fwd_supported(*p)) n += flex_mfma_fwd_partial_bytes(*p, flex_mfma_fwd_splits(*p));
-  else if (wants_fused(p) && flex_simple_supported(*p, 0)) n += flex_simple_fwd_partial_bytes(*p, flex_simple_fwd_splits(*p));
+  if (wants_fused(p) && flex_mfma_fwd_supported(*p)) n += flex_mfma_fwd_partial_bytes(*p, flex_mfma_fwd_splits(*p, true));
+  else if (wants_fused(p) && flex_simple_supported(*p, 0)) n += flex_simple_fwd_partial_bytes(*p, flex_simple_fwd_splits(*p, true));
   return n;
 }
 
@@ -174,7 +174,7 @@ extern "C" int flexattn_fwd(const FlexAttnParams* p, const void* q, const void* 
       lse2 = (float*)workspace;
     }
     // with a workspace, a call with few query tiles is split over the keys (the partials follow the log-sum-exp space)
-    const int splits = workspace ? flex_simple_fwd_splits(ps) : 1;
+    const int splits = workspace ? flex_simple_fwd_splits(ps, false) : 1;
     void* partials = splits > 1 ? (char*)workspace + fwd_lse_bytes(p) : nullptr;
     if (int rcs = flex_simple_fwd(ps, q, k, v, o, lse2, splits, partials, s)) return rcs;
     return check_launch("flexattn_fwd");
@@ -187,7 +187,7 @@ extern "C" int flexattn_fwd(const FlexAttnParams* p, const void* q, const void* 
       lse2 = (float*)workspace;
     }
     // with a workspace, a call with few query tiles is split over the keys (the partials follow the log-sum-exp space)
-    const int splits = workspace ? flex_mfma_fwd_splits(pr) : 1;
+    const int splits = workspace ? flex_mfma_fwd_splits(pr, false) : 1;
     void* partials = splits > 1 ? (char*)workspace + fwd_lse_bytes(p) : nullptr;
     rc = flex_mfma_fwd(pr, q, k, v, o, lse2, splits, partials, s);
   } else {

@@ -60,7 +60,8 @@ bool flex_mfma_fwd_supported(const FlexAttnParams& p) {
 // [2,8,2048,192] 120 -> 110.  Where two workgroups share a compute unit the heaviest one has it to itself in the end, and
 // a key tile less saves little: [1,8,8192,128] 342 -> 301 us, but [2,16,2048,128] 99 -> 124, [1,16,4096,64] 126 -> 136 (so
 // not split), and nothing at D = 64.
-int flex_mfma_fwd_splits(const FlexAttnParams& p) {
+// any_mask: the most shares any mask gets (a workspace is sized by the shape alone).
+int flex_mfma_fwd_splits(const FlexAttnParams& p, bool any_mask) {
   const int64_t wgs = (int64_t)((p.Lq + kFwdBM - 1) / kFwdBM) * p.Hq * p.B;
   const int slots = (p.D >= 192 ? 1 : 2) * flex_cu_count();  // 192- and 256-wide heads run one workgroup per compute unit
   const int tiles = (p.Lkv + kFwdBN - 1) / kFwdBN;
@@ -68,7 +69,7 @@ int flex_mfma_fwd_splits(const FlexAttnParams& p) {
     const bool causal = p.mask.kind == FLEX_MASK_BAND && p.mask.lo != INT32_MIN && p.mask.hi == INT32_MAX && p.Lq > p.Lkv / 2;
     const double visit_us = p.D >= 192 ? 4. : p.D == 128 ? 1.2 : 0.;   // what a key tile less of the heaviest workgroup saves
     const double merge_us = 4 + (double)p.B * p.Hq * p.Lq * 2 * p.D * sizeof(float) * 2 / 5e6;
-    return causal && wgs <= slots && 0.5 * tiles * visit_us > 1.5 * merge_us ? 2 : 1;
+    return (causal || any_mask) && wgs <= slots && 0.5 * tiles * visit_us > 1.5 * merge_us ? 2 : 1;
   }
   int s = (int)(slots / wgs);
   if (s > tiles / 8) s = tiles / 8;

@@ -6,7 +6,7 @@ using namespace flex;
 void flex_set_error(const char* fmt, ...);
 int flex_cu_count();
 DkvParts flex_dkv_parts(const FlexAttnParams& p, double slots, double visit_us);
-size_t flex_dkv_partial_bytes(const FlexAttnParams& p, DkvParts n);
+size_t flex_dkv_partial_bytes(const FlexAttnParams& p, double slots, double visit_us);
 int flex_simple_f32_64(const FlexAttnParams& p, const SimpleArgs& a);
 int flex_simple_f32_128(const FlexAttnParams& p, const SimpleArgs& a);
 int flex_simple_f16_192(const FlexAttnParams& p, const SimpleArgs& a);
@@ -82,7 +82,10 @@ static bool short_rows(const FlexAttnParams& p) {
   if (rounds < 1) rounds = 1;
   return 1.1 * rounds * steps / 4 <= (double)steps / splits;
 }
-int flex_simple_fwd_splits(const FlexAttnParams& p) { return short_rows(p) ? 1 : splits_over_keys(p); }
+// any_mask: the most any mask gets (a workspace is sized by the shape alone)
+int flex_simple_fwd_splits(const FlexAttnParams& p, bool any_mask) {
+  return !any_mask && short_rows(p) ? 1 : splits_over_keys(p);
+}
 
 // bytes of the partial (O, m, l) of a split forward
 size_t flex_simple_fwd_partial_bytes(const FlexAttnParams& p, int splits) {
@@ -119,10 +122,11 @@ int flex_simple_fwd(const FlexAttnParams& p, const void* q, const void* k, const
 
 // The dK/dV kernel divided over the queries as the tuned one is (flex_dkv_parts).  A visit of a 128-row query tile takes about
 // 13 us at D = 192 / 256 in 16 bits and 18 / 36 us at D = 64 / 128 in float32; one workgroup per compute unit.
-static DkvParts simple_dkv_parts(const FlexAttnParams& p) {
-  return flex_dkv_parts(p, flex_cu_count(), p.dtype != FLEX_F32 ? 13. : p.D == 64 ? 18. : 36.);
+static double simple_visit_us(const FlexAttnParams& p) { return p.dtype != FLEX_F32 ? 13. : p.D == 64 ? 18. : 36.; }
+static DkvParts simple_dkv_parts(const FlexAttnParams& p) { return flex_dkv_parts(p, flex_cu_count(), simple_visit_us(p)); }
+size_t flex_simple_bwd_workspace(const FlexAttnParams& p) {
+  return flex_dkv_partial_bytes(p, flex_cu_count(), simple_visit_us(p));
 }
-size_t flex_simple_bwd_workspace(const FlexAttnParams& p) { return flex_dkv_partial_bytes(p, simple_dkv_parts(p)); }
 
 int flex_simple_bwd(const FlexAttnParams& p, const void* q, const void* k, const void* v, const void* o, const float* lse2,
                     const void* d_o, void* dq, void* dk, void* dv, void* workspace, hipStream_t s) {

@@ -462,3 +462,26 @@ def test_block_classes_of_a_bitmap():
                 want = 1 if bool(blk.all()) else (2 if not bool(blk.any()) else 0)
                 assert int(cls[b, 0, i, j]) == want
     assert int(cls[0, 0, 1, 2]) == 1 and int(cls[1, 0, 0, 0]) == 2 and int(cls[1, 0, 2, 3]) == 0
+
+
+@pytest.mark.parametrize("dtype,D", [(_lib.FLEX_F16, 64), (_lib.FLEX_BF16, 128), (_lib.FLEX_F16, 256), (_lib.FLEX_F32, 64), (_lib.FLEX_F32, 128)])
+def test_workspace_sizes_do_not_depend_on_the_mask(dtype, D):
+    """A workspace may be sized once for a shape, before masks and tile lists exist, and serve every call of it."""
+    L = _lib.lib()
+    for B, Hq, Hkv, Lq, Lkv in ((1, 8, 2, 2048, 2048), (2, 8, 8, 2048, 2048), (1, 2, 1, 130, 5000), (1, 1, 1, 128, 128),
+                                (1, 8, 8, 8192, 8192), (16, 16, 16, 4096, 4096)):
+        sizes = set()
+        for kind, lo, hi, sink in ((0, -2**31, 2**31 - 1, -1), (0, 0, 2**31 - 1, -1), (0, 0, 500, -1), (0, 0, 500, 3), (1, 0, 0, 0)):
+            for lists in (False, True):
+                p = _lib.FlexAttnParams()
+                p.dtype, p.B, p.Hq, p.Hkv, p.Lq, p.Lkv, p.D, p.Dv = dtype, B, Hq, Hkv, Lq, Lkv, D, D
+                for name, H, n in (("q_stride", Hq, Lq), ("k_stride", Hkv, Lkv), ("v_stride", Hkv, Lkv), ("o_stride", Hq, Lq)):
+                    getattr(p, name)[:] = [H * n * D, n * D, D]
+                p.mask.kind, p.mask.lo, p.mask.hi, p.mask.sink = kind, lo, hi, sink
+                if lists:   # (only whether they are there is looked at)
+                    for t, kvb in ((p.tiles, 64), (p.tiles_bwd, 128)):
+                        t.kv_num = t.kv_idx = t.full_kv_num = t.full_kv_idx = 256
+                        t.q_num = t.q_idx = t.full_q_num = t.full_q_idx = 256
+                        t.q_block, t.kv_block = 128, kvb
+                sizes.add((L.flexattn_fwd_workspace_bytes(p), L.flexattn_bwd_workspace_bytes(p), L.flexattn_decode_workspace_bytes(p, 4)))
+        assert len(sizes) == 1, (B, Hq, Hkv, Lq, Lkv, sizes)
