@@ -285,33 +285,12 @@ __global__ __launch_bounds__(256, D >= 192 ? 1 : 2) void fwd_mfma_kernel(FlexAtt
         const int q_row = q_row0 + 32 * a;
         // ---- score_mod relative to the reference, tile mask where needed ----
         const float m_use = m_run[a];
-        bool near = false;
-        if constexpr (KIND == FLEX_SCORE_TANH_SOFTCAP) {
-          // a block whose scores all lie well below the cap (under a cap of 50: below 9) takes the polynomial: bf16
-          // [4,16,8192,128], window 1024, cap 50: 667 -> 633 us, and the log-sum-exp's error against 64 bits falls
-          // from 4e-6 to 1e-6
-          float far = 0.f;
 #pragma unroll
-          for (int r = 0; r < 16; r++) far = fmaxf(far, fabsf(sacc[a][r]));
-          near = __all(far < sm.near_s);
-          if (near) {
-#pragma unroll
-            for (int r = 0; r < 16; r += 2) {
-              float s0 = sacc[a][r], s1 = sacc[a][r + 1];
-              if (ROUND_S) round_pair<T>(s0, s1);
-              sacc[a][r] = sm.apply_sub_near(s0, m_use);
-              sacc[a][r + 1] = sm.apply_sub_near(s1, m_use);
-            }
-          }
-        }
-        if (!near) {
-#pragma unroll
-          for (int r = 0; r < 16; r += 2) {
-            float s0 = sacc[a][r], s1 = sacc[a][r + 1];
-            if (ROUND_S) round_pair<T>(s0, s1);
-            sacc[a][r] = sm.apply_sub(s0, acc_row(r), m_use);
-            sacc[a][r + 1] = sm.apply_sub(s1, acc_row(r + 1), m_use);
-          }
+        for (int r = 0; r < 16; r += 2) {
+          float s0 = sacc[a][r], s1 = sacc[a][r + 1];
+          if (ROUND_S) round_pair<T>(s0, s1);
+          sacc[a][r] = sm.apply_sub(s0, acc_row(r), m_use);
+          sacc[a][r + 1] = sm.apply_sub(s1, acc_row(r + 1), m_use);
         }
         if (cls == kBlockMixed) {
           // a real branch: every input of the mask arithmetic passes through this asm, so that

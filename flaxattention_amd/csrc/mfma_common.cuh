@@ -184,21 +184,8 @@ template <> struct Score2<FLEX_SCORE_REL_BIAS> {
 template <> struct Score2<FLEX_SCORE_TANH_SOFTCAP> {
   static constexpr bool kGradOne = false;  // d score_mod / d score == 1 everywhere
   float a, cap2, sc;  // a = 2*log2e*scale/cap, cap2 = cap*log2e
-  float near_s, k1, k3, k5;
   __device__ __forceinline__ void init(const FlexScoreMod& m, float scale, int h, int b = 0, int Lq = 0, int Lkv = 0) {
     a = 2.f * kLog2e * scale * m.p1; cap2 = m.p0 * kLog2e; sc = scale;
-    const float z = scale * m.p1;
-    near_s = 0.18f / fabsf(z);
-    k1 = 0.99999994375f * cap2 * z;
-    k3 = -0.33330206128f * cap2 * z * (z * z);
-    k5 = 0.13074870575f * cap2 * z * (z * z) * (z * z);
-  }
-  // tanh t for |t| <= 0.18 as t (c1 + c3 t^2 + c5 t^4): the interpolation of tanh(t) / t at the Chebyshev nodes of
-  // t^2 in [0, 0.18^2], relative error 5.6e-8 -- less than what the exponential and reciprocal below leave there (their 1 - 2r
-  // cancels).  Four full-rate instructions against three and two transcendentals of twice their cycles.
-  __device__ __forceinline__ float apply_sub_near(float s, float m) const {
-    const float u = s * s;
-    return fmaf(s, fmaf(u, fmaf(u, k5, k3), k1), -m);
   }
   __device__ __forceinline__ void tile(int q, int kvb) {}
   __device__ __forceinline__ void tileT(int qb, int kv) {}

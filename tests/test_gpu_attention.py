@@ -1285,11 +1285,10 @@ def test_short_float32_forward(dev, B, Hq, Hkv, Lq, Lkv, D, kind):
 
 @pytest.mark.parametrize("gain", [0.5, 1.0, 3.0, 12.0])
 @pytest.mark.parametrize("D,cap", [(64, 50.0), (128, 50.0), (128, 7.0), (256, 20.0)])
-def test_softcap_polynomial_against_64_bits(dev, D, cap, gain):
-    """Blocks whose scores lie well below the cap take a polynomial for the tanh, others the exponential: gains that put
-    all, some and none of the blocks on either side.  The unrounded numerics carry float32 up to the results, so the
+def test_softcap_against_64_bits(dev, D, cap, gain):
+    """The tanh on scores far below the cap, around it and beyond it.  The unrounded numerics carry float32 up to the results, so the
     log-sum-exp shows the scores' own error: 2^-24 per operation on scores of up to cap, doubled for the sum over D."""
-    print("case softcap polynomial", D, cap, gain, flush=True)
+    print("case softcap 64 bits", D, cap, gain, flush=True)
     B, H, L = 1, 2, 500
     q, k, v = seeded_qkv(B, H, H, L, L, D, torch.float16)
     q = (q.float() * gain).half()
@@ -1302,3 +1301,30 @@ def test_softcap_polynomial_against_64_bits(dev, D, cap, gain):
     rel = rel_l2(out.float().cpu(), (torch.softmax(x, -1) @ v.double()).float())
     print(f"  lse error {err:.2e}, O rel-L2 {rel:.2e}", flush=True)
     assert err <= 8 * cap * 2 ** -24 + 4e-6 and rel <= 2 ** -11
+
+
+@pytest.mark.parametrize("dtype,numerics", [(torch.float16, "fast"), (torch.bfloat16, "parity"), (torch.float16, "unrounded")])
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_softcap_rows_do_not_depend_on_what_they_cannot_see(dev, dtype, numerics, D):
+    """How a soft-capped score is computed must not depend on its neighbours in a block: hidden keys and other query rows
+    that score near the cap leave the rows that cannot see them at the same bits, and a cap far below the scores' scale
+    still gives 0 at score 0."""
+    print("case softcap rows", dtype, numerics, D, flush=True)
+    B, H, L = 1, 2, 320
+    opts = {"numerics": numerics}
+    q, k, v = (t.to(dev) for t in seeded_qkv(B, H, H, L, L, D, dtype))
+    bm = fa.create_block_mask(causal_mask, None, None, L, L, device=dev)
+    attend = lambda q, k, cap: fa.flax_attention(q, k, v, score_mod=generate_tanh_softcap(cap), block_mask=bm,   # noqa: E731
+                                                 return_lse=True, kernel_options=opts)
+    out, lse = attend(q, k, 50.0)
+    k2, q2 = k.clone(), q.clone()
+    k2[:, :, L - 16:] *= 40       # seen by the last 16 rows only
+    q2[:, :, L - 16:] *= 40
+    for qx, kx in ((q, k2), (q2, k)):
+        o2, l2 = attend(qx, kx, 50.0)
+        assert torch.equal(o2[:, :, :L - 16], out[:, :, :L - 16]) and torch.equal(l2[:, :, :L - 16], lse[:, :, :L - 16])
+        assert not torch.equal(o2[:, :, L - 16:], out[:, :, L - 16:])
+    zero, lse0 = attend(torch.zeros_like(q), k, 1e-12)   # scores of 0: every row is the mean of what it sees
+    want = v.double().cumsum(2) / torch.arange(1, L + 1, device=dev, dtype=torch.float64).reshape(-1, 1)
+    assert ((zero.double() - want).norm() / want.norm()).item() <= 1.5 * torch.finfo(dtype).eps
+    assert (lse0[0, 0].double() - torch.arange(1, L + 1, device=dev, dtype=torch.float64).log()).abs().max().item() <= 1e-5
