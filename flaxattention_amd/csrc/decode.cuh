@@ -130,7 +130,9 @@ __global__ __launch_bounds__(256, D >= 192 ? 1 : NB == 1 ? (D == 64 ? 3 : 2) : (
   // masked out and their P is 0, so what they hold does not matter as long as
   // it is finite.
   const int last = p.Lkv - 1;
-  // kept scores: [b, hk, step, column, lane half] x 16 values (the accumulator rows a lane holds)
+  // kept scores: [b, hk, step, column, lane half] x 16 values (the accumulator rows a lane holds), for the steps that
+  // hold a key.  A listed 64-key tile whose second half lies past the end still schedules that half as a step: it stores
+  // nothing and reads the last slot, and every entry is then masked.
   const int kept_step = ncols * kStep;
   T* kept_bh = nullptr;
   if constexpr (PASS == kDecLseKeep || PASS == kDecNormKept)
@@ -153,7 +155,7 @@ __global__ __launch_bounds__(256, D >= 192 ? 1 : NB == 1 ? (D == 64 ? 3 : 2) : (
     }
     if constexpr (PASS == kDecNormKept) {
       // in place of the K rows: this lane's 16 rounded scores of the step
-      const T* sp = kept_bh + (int64_t)(kv0 / kStep) * kept_step;
+      const T* sp = kept_bh + (int64_t)(min(kv0, last) / kStep) * kept_step;
       kfr[0] = *reinterpret_cast<const vec8*>(sp);
       kfr[1] = *reinterpret_cast<const vec8*>(sp + 8);
       return;
@@ -258,7 +260,7 @@ __global__ __launch_bounds__(256, D >= 192 ? 1 : NB == 1 ? (D == 64 ? 3 : 2) : (
         lo[r] = (T)s_a[r];
         hi[r] = (T)s_a[r + 8];
       }
-      if (col_ok[0]) {
+      if (col_ok[0] && kv0 <= last) {
         T* sp = kept_bh + (int64_t)(kv0 / kStep) * kept_step;
         *reinterpret_cast<vec8*>(sp) = lo;
         *reinterpret_cast<vec8*>(sp + 8) = hi;

@@ -1,4 +1,6 @@
 """Split-KV decode kernel vs the CPU oracle, and vs the prefill kernel."""
+import math
+
 import pytest
 import torch
 
@@ -277,3 +279,49 @@ def test_parity_decode_with_and_without_kept_scores(dev, B, Hq, Hkv, Lq, Lkv, D,
     x = x.masked_fill(~m(None, None, i, torch.arange(Lkv, device=dev).reshape(1, -1)), -float("inf")) if mask != "none" else x
     want = torch.softmax(x, -1) @ vs
     assert ((got[0][0][-1, -1].double() - want).norm() / want.norm()).item() < 2 ** -6
+
+
+@pytest.mark.parametrize("B,H,Lq,Lkv,D,mask", [
+    (16, 16, 4, 8200, 64, "lengths"),      # 16.8 MB of scores: the static variant reads K twice, for the same bits
+    (2, 3, 1, 8200, 128, "lengths"), (2, 3, 16, 2080, 64, "sink"), (1, 5, 32, 4097, 128, "sink"),
+    (3, 2, 2, 1025, 256, "lengths"), (2, 2, 1, 1056, 192, "sink"), (2, 3, 1, 640, 64, "lengths")])
+def test_kept_scores_of_a_listed_tile_that_ends_past_the_last_key(dev, B, H, Lq, Lkv, D, mask):
+    """Steps that come from tile lists are halves of 64-key tiles, so the last one may hold no key at all: its scores have
+    no slot.  Nothing is written past the workspace or into a neighbour's scores, every (batch, head) against float64."""
+    from flaxattention_amd import _lib
+    from flaxattention_amd.core.attention import _make_plan
+    from flaxattention_amd.core.common import MaskMod
+    print("case kept scores, listed tail", B, H, Lq, Lkv, D, mask, flush=True)
+    g = torch.Generator(device=dev).manual_seed(5)
+    mk = lambda *s: torch.randn(*s, generator=g, device=dev).to(torch.bfloat16)
+    q, k, v = mk(B, H, Lq, D), mk(B, H, Lkv, D), mk(B, H, Lkv, D)
+    lens = torch.tensor([Lkv - 3 * b for b in range(B)], device=dev)
+    mod = (lambda b, h, q_idx, kv_idx: kv_idx < lens[b]) if mask == "lengths" else MaskMod(0, 700, 3, Lkv - Lq)
+    bm = fa.create_block_mask(mod, B, None, Lq, Lkv, device=dev)
+    plan = _make_plan(q, k, v, None, bm, None, D ** -0.5, None)
+    assert plan.decode_splits != 0 and plan.lists is not None and plan.flags & _lib.FLAG_PARITY
+    o, lse = torch.empty_like(q), torch.empty((B, H, Lq), device=dev)
+    L, s = _lib.lib(), torch.cuda.current_stream().cuda_stream
+    p = plan.params(q, k, v, o)
+    nbytes = L.flexattn_decode_workspace_bytes(p, 0)
+    ws = torch.full((nbytes + (1 << 20),), 0x5A, dtype=torch.uint8, device=dev)
+    args = (p, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(), 0)
+    _lib.check(L.flexattn_decode(*args, ws.data_ptr(), s), "decode")
+    torch.cuda.synchronize()
+    assert bool((ws[nbytes:] == 0x5A).all())
+    i = torch.arange(Lq, device=dev).reshape(-1, 1)
+    kv = torch.arange(Lkv, device=dev).reshape(1, -1)
+    for b in range(B):
+        vis = torch.broadcast_to(mod(b, None, i, kv), (Lq, Lkv))
+        x = ((q[b].double() @ k[b].double().transpose(-1, -2)) * D ** -0.5).masked_fill(~vis, -float("inf"))
+        want = torch.softmax(x, -1) @ v[b].double()
+        rel = (o[b].double() - want).norm(dim=(1, 2)) / want.norm(dim=(1, 2))
+        assert rel.max().item() < 2 ** -6, b     # scores and P round to 8 bits: 2^-8 relative
+        # (the scores are rounded: 2^-9 of up to 5, and the log-sum-exp averages them)
+        assert (lse[b].double() * math.log(2) - torch.logsumexp(x, -1)).abs().max().item() < 1e-2, b
+    if nbytes > 16 << 20:
+        o2, lse2 = torch.empty_like(o), torch.empty_like(lse)
+        args = (p, q.data_ptr(), k.data_ptr(), v.data_ptr(), o2.data_ptr(), lse2.data_ptr(), 0)
+        _lib.check(L.flexattn_decode_static(*args, s), "decode_static")
+        torch.cuda.synchronize()
+        assert torch.equal(o, o2) and torch.equal(lse, lse2)
