@@ -76,13 +76,17 @@ size_t flex_decode_workspace(const FlexAttnParams& p, int splits) {
 }
 
 // Bytes in which the parity numerics keep the rounded scores between their two passes, 0 where they read K twice
-// instead.  A step's scores are 64 bytes per column, written and read once, against 64 * D bytes of K: kept while that is
-// at most half (columns <= D / 4).  bf16 KV cache [16,8,6001,128], 4 columns:
-// 107.7 us with K read twice and a merge launch between the passes, 86.8 us with the scores kept.
+// instead (the same bits either way).  A step's scores are 64 bytes per column, written and read once, against 64 * D bytes of
+// K: at most half of that (columns <= D / 4).  Cold KV caches, bf16, us with K read twice / scores kept:
+//   [16,8,6016,128]  1 column 104.5 / 81.9, 4: 104.8 / 85.9, 8: 104.9 / 90.0, 16: 105.8 / 98.2, 32: 106.5 / 105.9
+//   [1,8,32768,128]  1 column 48.9 / 43.1, 32: 49.8 / 48.1;   [16,8,6016,256]  1 column 207 / 149, 32: 213 / 189
+// The room is bounded, so that a cache that nearly fills the card still fits: beyond kMaxKeptBytes K is read twice.
+constexpr size_t kMaxKeptBytes = (size_t)256 << 20;
 size_t flex_decode_kept_bytes(const FlexAttnParams& p) {
-  const int64_t ncols = (int64_t)(p.Hq / p.Hkv) * p.Lq;
+  const int64_t ncols = (int64_t)(p.Hq / p.Hkv) * p.Lq, heads = (int64_t)p.B * p.Hkv;
   if (!(p.flags & FLEX_PARITY) || ncols > p.D / 4 || ncols > 32) return 0;
-  return (size_t)p.B * p.Hkv * ((p.Lkv + kStep - 1) / kStep) * ncols * kStep * 2;
+  const size_t bytes = (size_t)heads * ((p.Lkv + kStep - 1) / kStep) * ncols * kStep * 2;
+  return bytes <= kMaxKeptBytes ? bytes : 0;
 }
 
 // Device address of this file's scratch array on the current device, looked up once per device

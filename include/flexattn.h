@@ -271,8 +271,8 @@ int flexattn_decode(const FlexAttnParams* p, const void* q, const void* k, const
  * FLEXATTN_DECODE_STATIC_BYTES that is part of the library image on every GPU it runs on (held
  * until the process ends); the call makes no hipMalloc / hipFree and no other allocating call.
  * Problems whose split-KV partials exceed that size are refused with an error; use
- * flexattn_decode for those.  (Under FLEX_PARITY flexattn_decode_workspace_bytes adds room for the rounded scores, which
- * here are kept only where they fit as well; the results are the same bits.)  All calls on one GPU share the buffer, whose
+ * flexattn_decode for those.  (Under FLEX_PARITY flexattn_decode_workspace_bytes adds room for the rounded scores, at most
+ * 256 MiB; here they are kept only where they fit as well.  The results are the same bits.)  All calls on one GPU share the buffer, whose
  * contents do not carry over between calls (every call overwrites what it reads): calls that
  * overlap on one GPU -- two streams, two threads -- race.  Results are bit-identical to
  * flexattn_decode with the same num_splits.  */

@@ -325,3 +325,26 @@ def test_kept_scores_of_a_listed_tile_that_ends_past_the_last_key(dev, B, H, Lq,
         _lib.check(L.flexattn_decode_static(*args, s), "decode_static")
         torch.cuda.synchronize()
         assert torch.equal(o, o2) and torch.equal(lse, lse2)
+
+
+def test_parity_decode_beyond_the_bound_of_kept_scores(dev):
+    """A call whose scores would take more than the stated bound reads K twice: the same bits as its batch elements in
+    calls that keep theirs."""
+    from flaxattention_amd import _lib
+    from flaxattention_amd.core.attention import _make_plan
+    B, G, Hkv, Lkv, D, part = 40, 32, 16, 8300, 128, 8
+    print("case beyond the bound", flush=True)
+    g = torch.Generator(device=dev).manual_seed(6)
+    mk = lambda *s: torch.randn(*s, generator=g, device=dev).to(torch.bfloat16)
+    q, k, v = mk(B, G * Hkv, 1, D), mk(B, Hkv, Lkv, D), mk(B, Hkv, Lkv, D)
+    kept = []
+    for n in (B, part):
+        plan = _make_plan(q[:n], k[:n], v[:n], None, None, None, D ** -0.5, None)
+        p = plan.params(q[:n], k[:n], v[:n], q[:n])
+        kept.append(_lib.lib().flexattn_decode_workspace_bytes(p, 2) - (n * G * Hkv * 2 * (D + 2) * 4 + 255) // 256 * 256)
+    assert kept == [0, part * Hkv * ((Lkv + 31) // 32) * G * 64]
+    opts = {"decode_splits": 2}
+    out, lse = fa.flax_attention(q, k, v, enable_gqa=True, return_lse=True, kernel_options=opts)
+    for b in range(0, B, part):
+        o, l = fa.flax_attention(q[b:b + part], k[b:b + part], v[b:b + part], enable_gqa=True, return_lse=True, kernel_options=opts)
+        assert torch.equal(o, out[b:b + part]) and torch.equal(l, lse[b:b + part]), b

@@ -485,3 +485,21 @@ def test_workspace_sizes_do_not_depend_on_the_mask(dtype, D):
                         t.q_block, t.kv_block = 128, kvb
                 sizes.add((L.flexattn_fwd_workspace_bytes(p), L.flexattn_bwd_workspace_bytes(p), L.flexattn_decode_workspace_bytes(p, 4)))
         assert len(sizes) == 1, (B, Hq, Hkv, Lq, Lkv, sizes)
+
+
+@pytest.mark.parametrize("D", [64, 128, 192, 256])
+def test_kept_scores_of_a_parity_decode_are_bounded(D):
+    """The room in which a parity decode keeps its scores has a fixed bound, whatever the KV cache."""
+    L = _lib.lib()
+    for B, Hkv, G, Lq, Lkv in ((1, 1, 1, 1, 512), (16, 8, 4, 1, 6001), (64, 8, 8, 1, 8192), (64, 8, 16, 1, 131072),
+                               (512, 16, 1, 1, 65536), (1, 8, 1, 1, 1 << 24), (2, 3, 4, 3, 2047)):
+        p = _lib.FlexAttnParams()
+        p.dtype, p.B, p.Hq, p.Hkv, p.Lq, p.Lkv, p.D, p.Dv = _lib.FLEX_BF16, B, Hkv * G, Hkv, Lq, Lkv, D, D
+        for splits in (1, 2, 64):
+            p.flags = 0
+            plain = L.flexattn_decode_workspace_bytes(p, splits)
+            p.flags = _lib.FLAG_PARITY | _lib.FLAG_ROUND_S
+            kept = L.flexattn_decode_workspace_bytes(p, splits) - plain
+            room = B * Hkv * ((Lkv + 31) // 32) * G * Lq * 64
+            want = G * Lq <= min(D // 4, 32) and room <= 256 << 20
+            assert kept == (room if want else 0), (B, Hkv, G, Lq, Lkv, splits, kept)
