@@ -56,7 +56,7 @@ int flex_decode_default_splits(const FlexAttnParams& p);
 size_t flex_decode_workspace(const FlexAttnParams& p, int splits);
 int flex_decode_launch(const FlexAttnParams& p, const void* q, const void* k, const void* v, void* o, float* lse2, int splits,
                        void* workspace, bool keep_scores, hipStream_t s);
-size_t flex_decode_kept_bytes(const FlexAttnParams& p);
+size_t flex_decode_kept_bytes(const FlexAttnParams& p, int splits);
 void* flex_decode_static_scratch(size_t* bytes);
 void flex_mfma_tiles(int dtype, int D, int Dv, int which, int* qb, int* kvb);
 bool flex_simple_supported(const FlexAttnParams& p, int which);
@@ -239,7 +239,7 @@ extern "C" int flexattn_bwd(const FlexAttnParams* p, const void* q, const void* 
 extern "C" size_t flexattn_decode_workspace_bytes(const FlexAttnParams* p, int32_t num_splits) {
   if (!p) return 0;
   if (num_splits <= 0) num_splits = flex_decode_default_splits(*p);
-  return flex_decode_workspace(*p, num_splits) + flex_decode_kept_bytes(*p);
+  return flex_decode_workspace(*p, num_splits) + flex_decode_kept_bytes(*p, num_splits);
 }
 
 static int decode_checked(const FlexAttnParams* p, const void* q, const void* k, const void* v, void* o, float* lse2,
@@ -270,7 +270,7 @@ extern "C" int flexattn_decode_static(const FlexAttnParams* p, const void* q, co
     return 1;
   }
   // the parity numerics keep their scores between the passes where those fit beside the partials
-  return decode_checked(p, q, k, v, o, lse2, num_splits, ws, need + flex_decode_kept_bytes(*p) <= cap, stream);
+  return decode_checked(p, q, k, v, o, lse2, num_splits, ws, need + flex_decode_kept_bytes(*p, num_splits) <= cap, stream);
 }
 
 static int decode_checked(const FlexAttnParams* p, const void* q, const void* k, const void* v, void* o, float* lse2,
@@ -284,7 +284,7 @@ static int decode_checked(const FlexAttnParams* p, const void* q, const void* k,
   }
   if (num_splits <= 0) num_splits = flex_decode_default_splits(*p);
   int rc = flex_decode_launch(*p, q, k, v, o, lse2, num_splits, workspace,
-                              keep_scores && flex_decode_kept_bytes(*p) > 0, (hipStream_t)stream);
+                              keep_scores && flex_decode_kept_bytes(*p, num_splits) > 0, (hipStream_t)stream);
   if (rc) return rc;
   return check_launch("flexattn_decode");
 }

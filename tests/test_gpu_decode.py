@@ -243,7 +243,7 @@ def test_decode_kv_cache_beyond_2_31_elements(dev, Lq):
 
 @pytest.mark.parametrize("B,Hq,Hkv,Lq,Lkv,D,mask", [
     (1, 64, 8, 4, 33000, 128, "none"),      # 32 columns: the widest call that keeps its scores at D = 128
-    (8, 64, 16, 4, 8200, 64, "causal"),     # 16 columns, the widest at D = 64; the last step ragged
+    (32, 64, 16, 4, 8200, 64, "causal"),    # 16 columns, the widest at D = 64; the last step ragged
     (40, 32, 8, 2, 6200, 192, "window"),
     (48, 32, 16, 1, 12001, 256, "window")])
 def test_parity_decode_with_and_without_kept_scores(dev, B, Hq, Hkv, Lq, Lkv, D, mask):
@@ -281,11 +281,11 @@ def test_parity_decode_with_and_without_kept_scores(dev, B, Hq, Hkv, Lq, Lkv, D,
     assert ((got[0][0][-1, -1].double() - want).norm() / want.norm()).item() < 2 ** -6
 
 
-@pytest.mark.parametrize("B,H,Lq,Lkv,D,mask", [
-    (16, 16, 4, 8200, 64, "lengths"),      # 16.8 MB of scores: the static variant reads K twice, for the same bits
-    (2, 3, 1, 8200, 128, "lengths"), (2, 3, 16, 2080, 64, "sink"), (1, 5, 32, 4097, 128, "sink"),
-    (3, 2, 2, 1025, 256, "lengths"), (2, 2, 1, 1056, 192, "sink"), (2, 3, 1, 640, 64, "lengths")])
-def test_kept_scores_of_a_listed_tile_that_ends_past_the_last_key(dev, B, H, Lq, Lkv, D, mask):
+@pytest.mark.parametrize("B,H,Lq,Lkv,D,mask,splits", [
+    (16, 32, 4, 8200, 64, "lengths", 0),   # 34 MB of scores: the static variant reads K twice, for the same bits
+    (2, 3, 1, 8200, 128, "lengths", 0), (12, 8, 16, 2080, 64, "sink", 6), (1, 5, 32, 4097, 128, "sink", 0),
+    (3, 2, 2, 1025, 256, "lengths", 0), (2, 2, 1, 1056, 192, "sink", 3), (2, 3, 1, 640, 128, "lengths", 0)])
+def test_kept_scores_of_a_listed_tile_that_ends_past_the_last_key(dev, B, H, Lq, Lkv, D, mask, splits):
     """Steps that come from tile lists are halves of 64-key tiles, so the last one may hold no key at all: its scores have
     no slot.  Nothing is written past the workspace or into a neighbour's scores, every (batch, head) against float64."""
     from flaxattention_amd import _lib
@@ -303,9 +303,10 @@ def test_kept_scores_of_a_listed_tile_that_ends_past_the_last_key(dev, B, H, Lq,
     o, lse = torch.empty_like(q), torch.empty((B, H, Lq), device=dev)
     L, s = _lib.lib(), torch.cuda.current_stream().cuda_stream
     p = plan.params(q, k, v, o)
-    nbytes = L.flexattn_decode_workspace_bytes(p, 0)
+    nbytes = L.flexattn_decode_workspace_bytes(p, splits)
+    assert nbytes > B * H * ((Lkv + 31) // 32) * Lq * 64     # the scores are kept
     ws = torch.full((nbytes + (1 << 20),), 0x5A, dtype=torch.uint8, device=dev)
-    args = (p, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(), 0)
+    args = (p, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(), splits)
     _lib.check(L.flexattn_decode(*args, ws.data_ptr(), s), "decode")
     torch.cuda.synchronize()
     assert bool((ws[nbytes:] == 0x5A).all())
@@ -321,7 +322,7 @@ def test_kept_scores_of_a_listed_tile_that_ends_past_the_last_key(dev, B, H, Lq,
         assert (lse[b].double() * math.log(2) - torch.logsumexp(x, -1)).abs().max().item() < 1e-2, b
     if nbytes > 16 << 20:
         o2, lse2 = torch.empty_like(o), torch.empty_like(lse)
-        args = (p, q.data_ptr(), k.data_ptr(), v.data_ptr(), o2.data_ptr(), lse2.data_ptr(), 0)
+        args = (p, q.data_ptr(), k.data_ptr(), v.data_ptr(), o2.data_ptr(), lse2.data_ptr(), splits)
         _lib.check(L.flexattn_decode_static(*args, s), "decode_static")
         torch.cuda.synchronize()
         assert torch.equal(o, o2) and torch.equal(lse, lse2)

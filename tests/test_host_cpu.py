@@ -489,7 +489,8 @@ def test_workspace_sizes_do_not_depend_on_the_mask(dtype, D):
 
 @pytest.mark.parametrize("D", [64, 128, 192, 256])
 def test_kept_scores_of_a_parity_decode_are_bounded(D):
-    """The room in which a parity decode keeps its scores has a fixed bound, whatever the KV cache."""
+    """The room in which a parity decode keeps its scores has a fixed bound, whatever the KV cache; at D = 64 it is only
+    asked for where two workgroups share a compute unit (256 on a machine without a device)."""
     L = _lib.lib()
     for B, Hkv, G, Lq, Lkv in ((1, 1, 1, 1, 512), (16, 8, 4, 1, 6001), (64, 8, 8, 1, 8192), (64, 8, 16, 1, 131072),
                                (512, 16, 1, 1, 65536), (1, 8, 1, 1, 1 << 24), (2, 3, 4, 3, 2047)):
@@ -501,5 +502,5 @@ def test_kept_scores_of_a_parity_decode_are_bounded(D):
             p.flags = _lib.FLAG_PARITY | _lib.FLAG_ROUND_S
             kept = L.flexattn_decode_workspace_bytes(p, splits) - plain
             room = B * Hkv * ((Lkv + 31) // 32) * G * Lq * 64
-            want = G * Lq <= min(D // 4, 32) and room <= 256 << 20
+            want = G * Lq <= min(D // 4, 32) and room <= 256 << 20 and (D > 64 or B * Hkv * splits >= 512)
             assert kept == (room if want else 0), (B, Hkv, G, Lq, Lkv, splits, kept)
