@@ -642,9 +642,10 @@ __global__ __launch_bounds__(256) void simple_dq_kernel(FlexAttnParams p, const 
 // dV = P^T.dO and dK = scale * (P o (dP - delta) o g)^T . Q for the 128 keys of a workgroup (one 32-key block per
 // wave, a lane owns one key), summed over the query heads of the key head's group.  PARITY: dP is rounded through T
 // before delta is subtracted and the scale is applied before dS is rounded.
-// With parts_g * parts_t > 1 that many workgroups share a key tile and leave partial sums (dkv_combine_kernel), as in the
-// tuned kernel.
-template <typename T, int D, int KIND, bool PARITY>
+// SPLIT: parts_g * parts_t workgroups share a key tile and leave partial sums (dkv_combine_kernel), as in the tuned kernel.  A
+// template parameter, because the accumulators leave no registers for the parts' numbers: as run-time arguments they took the
+// undivided kernel at D = 256 from 45 to 77 spilled registers (parity numerics, identity), next to the tile loop.
+template <typename T, int D, int KIND, bool PARITY, bool SPLIT = false>
 __global__ __launch_bounds__(256) void simple_dkv_kernel(FlexAttnParams p, const T* __restrict__ q,
                                                          const T* __restrict__ k, const T* __restrict__ v,
                                                          const float* __restrict__ lse2, const float* __restrict__ delta,
@@ -664,7 +665,7 @@ __global__ __launch_bounds__(256) void simple_dkv_kernel(FlexAttnParams p, const
   const int nkt = (p.Lkv + kSimpleKvTile - 1) / kSimpleKvTile;
   int kt, bh;  // early key tiles see the most queries under causal masks
   int wid = blockIdx.x, part = 0;
-  if (partial) dkv_part_map(p.Hkv * p.B, parts_g * parts_t, wid, part);
+  if constexpr (SPLIT) dkv_part_map(p.Hkv * p.B, parts_g * parts_t, wid, part);
   xcd_tile_map(wid, nkt, p.Hkv * p.B, kt, bh);
   const int hk = bh % p.Hkv, b = bh / p.Hkv, G = p.Hq / p.Hkv;
   const int kv_col = kt * kSimpleKvTile + w * 32 + i32;
@@ -682,15 +683,21 @@ __global__ __launch_bounds__(256) void simple_dkv_kernel(FlexAttnParams p, const
 
   const FlexTileLists& tl = p.tiles_bwd;
   Score2<KIND> sm;
-  for (int gi = part % parts_g; gi < G; gi += parts_g) {
+  for (int gi = SPLIT ? part % parts_g : 0; gi < G; gi += SPLIT ? parts_g : 1) {
     const int h = hk * G + gi;
     sm.init(p.score, p.scale, h, b, p.Lq, p.Lkv);
     const Mask2 visible(p.mask, b, h, p.Lkv);
     SimpleSteps st;
     st.init(tl.q_num, tl.q_idx, tl.full_q_num, tl.full_q_idx,
             (b * tl.stride_b + h * tl.stride_h) * tl.n_kv_blocks + kt, tl.n_q_blocks, tl.q_block, p.Lq, p.mask);
-    const int n_full_t = st.full_steps(), share = part / parts_g;
-    const int it0 = (int)((int64_t)st.count() * share / parts_t), nt = (int)((int64_t)st.count() * (share + 1) / parts_t);
+    const int n_full_t = st.full_steps();
+    int it0 = 0, nt = st.count();   // this workgroup's stretch of the list
+    if constexpr (SPLIT) {
+      const int share = part / parts_g;
+      const int64_t all = nt;
+      it0 = (int)(all * share / parts_t);
+      nt = (int)(all * (share + 1) / parts_t);
+    }
     const T* qbase = q + b * p.q_stride[0] + h * p.q_stride[1];
     const int64_t rows0 = ((int64_t)b * p.Hq + h) * p.Lq;
     const T* dobase = d_o + rows0 * D;
@@ -772,7 +779,10 @@ __global__ __launch_bounds__(256) void simple_dkv_kernel(FlexAttnParams p, const
   }
 
   const float out_scale = PARITY ? 1.f : p.scale;
-  if (partial) {
+  // (a divided call always has its room; behind a test of it instead of a plain return, the compiler gives the kernel without
+  // a score_mod in the fast numerics 19 spilled registers at D = 256 and not 27: f16 [2,8,2048,256] causal, forward + backward,
+  // 441 -> 429 us.  The other functors spill less without the test.)
+  if (SPLIT && (PARITY || KIND != FLEX_SCORE_IDENTITY || partial)) {
     store_dkv_part<DB>(partial, ((int64_t)part * p.B * p.Hkv + bh) * nkt + kt, w, lane, dkacc, dvacc, out_scale);
     return;
   }
@@ -842,16 +852,22 @@ template <typename T, int D, int KIND> void simple_launch_fwd(const FlexAttnPara
                      a.o_part, a.ml_part);
   merge((T*)a.out, a.lse2_out);
 }
-template <typename T, int D, int KIND> void simple_launch_bwd(const FlexAttnParams& p, const SimpleArgs& a) {
-  const dim3 qgrid((p.Lq + kSimpleQTile - 1) / kSimpleQTile * p.Hq * p.B);
+template <typename T, int D, int KIND, bool PARITY> void simple_launch_dkv(const FlexAttnParams& p, const SimpleArgs& a) {
   const int nkt = (p.Lkv + kSimpleKvTile - 1) / kSimpleKvTile, tiles = nkt * p.Hkv * p.B;
-  const int parts = a.dkv_partial ? a.parts.g * a.parts.t : 1;
-  const dim3 kgrid(tiles * parts), block(256);
-  auto merge = [&] {
-    if (parts > 1)
-      hipLaunchKernelGGL((dkv_combine_kernel<T, D>), dim3(tiles * 4), block, 0, a.s, a.dkv_partial, parts, nkt, p.Lkv, (T*)a.dk,
-                         (T*)a.dv);
-  };
+  const T *q = (const T*)a.q, *k = (const T*)a.k, *v = (const T*)a.v, *d_o = (const T*)a.d_o;
+  if (a.dkv_partial) {
+    const int parts = a.parts.g * a.parts.t;
+    hipLaunchKernelGGL((simple_dkv_kernel<T, D, KIND, PARITY, true>), dim3(tiles * parts), dim3(256), 0, a.s, p, q, k, v, a.lse2_in,
+                       a.delta, d_o, (T*)a.dk, (T*)a.dv, a.parts.g, a.parts.t, a.dkv_partial);
+    hipLaunchKernelGGL((dkv_combine_kernel<T, D>), dim3(tiles * 4), dim3(256), 0, a.s, a.dkv_partial, parts, nkt, p.Lkv, (T*)a.dk,
+                       (T*)a.dv);
+    return;
+  }
+  hipLaunchKernelGGL((simple_dkv_kernel<T, D, KIND, PARITY>), dim3(tiles), dim3(256), 0, a.s, p, q, k, v, a.lse2_in, a.delta, d_o,
+                     (T*)a.dk, (T*)a.dv, 1, 1, nullptr);
+}
+template <typename T, int D, int KIND> void simple_launch_bwd(const FlexAttnParams& p, const SimpleArgs& a) {
+  const dim3 qgrid((p.Lq + kSimpleQTile - 1) / kSimpleQTile * p.Hq * p.B), block(256);
   const T *q = (const T*)a.q, *k = (const T*)a.k, *v = (const T*)a.v, *o = (const T*)a.o, *d_o = (const T*)a.d_o;
   if constexpr (SimpleOps<T, D>::kRounds) {  // the parity numerics exist where something is rounded
     if (p.flags & FLEX_PARITY) {
@@ -861,22 +877,14 @@ template <typename T, int D, int KIND> void simple_launch_bwd(const FlexAttnPara
         hipLaunchKernelGGL((simple_dq_kernel<T, D, KIND, kSimpleBwdParity>), qgrid, block, 0, a.s, p, q, k, v, o, a.lse2_in,
                            d_o, (T*)a.dq, a.delta);
       }
-      if (!(p.flags & FLEX_BWD_ONLY_DQ)) {
-        hipLaunchKernelGGL((simple_dkv_kernel<T, D, KIND, true>), kgrid, block, 0, a.s, p, q, k, v, a.lse2_in, a.delta, d_o,
-                           (T*)a.dk, (T*)a.dv, a.parts.g, a.parts.t, a.dkv_partial);
-        merge();
-      }
+      if (!(p.flags & FLEX_BWD_ONLY_DQ)) simple_launch_dkv<T, D, KIND, true>(p, a);
       return;
     }
   }
   if (!(p.flags & FLEX_BWD_ONLY_DKV))
     hipLaunchKernelGGL((simple_dq_kernel<T, D, KIND, kSimpleBwdFast>), qgrid, block, 0, a.s, p, q, k, v, o, a.lse2_in, d_o,
                        (T*)a.dq, a.delta);
-  if (!(p.flags & FLEX_BWD_ONLY_DQ)) {
-    hipLaunchKernelGGL((simple_dkv_kernel<T, D, KIND, false>), kgrid, block, 0, a.s, p, q, k, v, a.lse2_in, a.delta, d_o,
-                       (T*)a.dk, (T*)a.dv, a.parts.g, a.parts.t, a.dkv_partial);
-    merge();
-  }
+  if (!(p.flags & FLEX_BWD_ONLY_DQ)) simple_launch_dkv<T, D, KIND, false>(p, a);
 }
 template <typename T, int D, int KIND> void simple_launch(const FlexAttnParams& p, const SimpleArgs& a) {
   if (a.bwd) simple_launch_bwd<T, D, KIND>(p, a);

@@ -504,3 +504,39 @@ def test_kept_scores_of_a_parity_decode_are_bounded(D):
             room = B * Hkv * ((Lkv + 31) // 32) * G * Lq * 64
             want = G * Lq <= min(D // 4, 32) and room <= 256 << 20 and (D > 64 or B * Hkv * splits >= 512)
             assert kept == (room if want else 0), (B, Hkv, G, Lq, Lkv, splits, kept)
+
+
+def test_undivided_wide_backward_keeps_its_registers():
+    """The simple dK/dV kernel at D = 256 fills a wave's registers, and what does not fit is spilled next to its tile loop.
+    The form that is not divided over the queries carries nothing of the division: the spills of the built kernels, read
+    from the library's own kernel descriptions, stay at what the undivided kernel needs with the image's compiler."""
+    import struct
+    msgpack = pytest.importorskip("msgpack")
+    with open(_lib.LIB_PATH, "rb") as f:
+        data = f.read()
+    magic, kernels, pos = b"__CLANG_OFFLOAD_BUNDLE__", {}, 0
+    while (pos := data.find(magic, pos)) >= 0:
+        at = pos + 32
+        for _ in range(struct.unpack_from("<Q", data, pos + 24)[0]):
+            off, size, n = struct.unpack_from("<QQQ", data, at)
+            target, at = data[at + 24:at + 24 + n], at + 24 + n
+            if b"gfx950" not in target:
+                continue
+            elf = data[pos + off:pos + off + size]
+            (table,), (entry, count) = struct.unpack_from("<Q", elf, 0x28), struct.unpack_from("<HH", elf, 0x3a)
+            for section in range(table, table + entry * count, entry):
+                if struct.unpack_from("<I", elf, section + 4)[0] == 7:     # the notes
+                    start = struct.unpack_from("<Q", elf, section + 0x18)[0]
+                    name, desc, _ = struct.unpack_from("<III", elf, start)
+                    start += 12 + (name + 3) // 4 * 4
+                    kernels.update({k[".name"]: k for k in msgpack.unpackb(elf[start:start + desc])["amdhsa.kernels"]})
+        pos += len(magic)
+    # by functor (identity, checkerboard, ALiBi, soft-cap, relative bias, additive and multiplicative tables)
+    most = {"parity": dict(zip((0, 1, 2, 3, 4, 5, 102), (48, 48, 48, 64, 48, 72, 82))),
+            "fast": dict(zip((0, 1, 2, 3, 4, 5, 102), (32, 32, 32, 42, 32, 47, 52)))}
+    for dtype in ("DF16_", "DF16b"):
+        for numerics, b in (("parity", 1), ("fast", 0)):
+            for kind, bound in most[numerics].items():
+                found = [k for n, k in kernels.items() if f"simple_dkv_kernelI{dtype}Li256ELi{kind}ELb{b}ELb0E" in n]
+                assert len(found) == 1, (dtype, kind, numerics)
+                assert found[0][".vgpr_spill_count"] <= bound, (dtype, kind, numerics, found[0][".vgpr_spill_count"])
