@@ -62,6 +62,7 @@ bool flex_mfma_fwd_supported(const FlexAttnParams& p) {
 // not split), and nothing at D = 64.
 // any_mask: the most shares any mask gets (a workspace is sized by the shape alone).
 int flex_mfma_fwd_splits(const FlexAttnParams& p, bool any_mask) {
+  if (p.flags & FLEX_NO_SPLIT) return 1;
   const int64_t wgs = (int64_t)((p.Lq + kFwdBM - 1) / kFwdBM) * p.Hq * p.B;
   const int slots = (p.D >= 192 ? 1 : 2) * flex_cu_count();  // 192- and 256-wide heads run one workgroup per compute unit
   const int tiles = (p.Lkv + kFwdBN - 1) / kFwdBN;

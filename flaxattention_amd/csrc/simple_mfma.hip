@@ -84,6 +84,7 @@ static bool short_rows(const FlexAttnParams& p) {
 }
 // any_mask: the most any mask gets (a workspace is sized by the shape alone)
 int flex_simple_fwd_splits(const FlexAttnParams& p, bool any_mask) {
+  if (p.flags & FLEX_NO_SPLIT) return 1;
   return !any_mask && short_rows(p) ? 1 : splits_over_keys(p);
 }
 

@@ -113,10 +113,11 @@ enum FlexFlags {
                             simplification removes the round trips of attention.py:27, 104-105.
                             Exclusive with FLEX_PARITY / FLEX_ROUND_S (it wins); the generic kernels
                             do the same when neither FLEX_STRICT nor FLEX_ROUND_S is set.  */
-  FLEX_NO_SPLIT = 128,   /* flexattn_bwd: one workgroup per key tile always sums all its queries; flexattn_fwd (float32): one
-                            wave always walks all keys of its rows.  Without it a call with few tiles divides
-                            that work (backward: float32 partial sums in the workspace), so that the order of the
-                            sums depends on the number of tiles.  */
+  FLEX_NO_SPLIT = 128,   /* no call is divided for having few tiles: flexattn_fwd walks all keys of a row in one wave, with or
+                            without a workspace, and flexattn_bwd sums all queries of a key tile in one workgroup.
+                            Without it such a call divides that work (partial results in the workspace; float32
+                            forwards also over the waves of a workgroup), so that the order of the sums depends on
+                            the number of tiles.  */
   /* profiling aids for flexattn_bwd: launch only one of the two fused backward
    * kernels.  The dK/dV kernel then reads the delta values a previous complete
    * call left in the same workspace. */

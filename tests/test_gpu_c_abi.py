@@ -200,3 +200,30 @@ def test_threads_on_their_own_streams(dev):
         for a, b in zip(alone[seed], together[seed]):
             for x, y in zip(a, b):
                 assert torch.equal(x, y)
+
+
+@pytest.mark.parametrize("dtype,B,H,Lq,Lkv,D,causal", [
+    (torch.float32, 1, 2, 96, 4096, 64, False), (torch.float32, 1, 2, 128, 4096, 128, True), (torch.float16, 1, 2, 128, 4096, 64, False),
+    (torch.float16, 2, 8, 2048, 2048, 256, True), (torch.bfloat16, 1, 2, 200, 3000, 192, False), (torch.bfloat16, 1, 4, 100, 4096, 128, False)])
+def test_no_split_forward_is_the_same_with_a_workspace(dev, dtype, B, H, Lq, Lkv, D, causal):
+    """FLEX_NO_SPLIT promises that the keys of a call are not divided: a workspace then changes nothing, bit for bit, and none
+    is asked for beyond the log-sum-exp's hand-over."""
+    print("case no split forward", dtype, B, H, Lq, Lkv, D, causal, flush=True)
+    L = _lib.lib()
+    q, k, v = _inputs(dev, B, H, Lq, Lkv, D, dtype)
+    p = _params(q, k, v, q, lo=0 if causal else INT_MIN)
+    p.mask.q_offset = Lkv - Lq
+    parity = dtype == torch.bfloat16
+    p.flags = (1 if dtype != torch.float32 else 0) | (_lib.FLAG_PARITY if parity else 0)
+    room = L.flexattn_fwd_workspace_bytes(p)        # of the same call when it may be divided
+    p.flags |= _lib.FLAG_NO_SPLIT
+    lse_part = (B * H * Lq * 4 + 255) // 256 * 256 if parity else 0
+    assert room > lse_part and L.flexattn_fwd_workspace_bytes(p) == lse_part
+    ws = torch.empty(room, dtype=torch.uint8, device=dev)
+    got = []
+    for w in (None, ws.data_ptr()):
+        o, lse = torch.empty_like(q), torch.empty(B, H, Lq, device=dev)
+        _lib.check(L.flexattn_fwd(p, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(), w, _stream()), "fwd")
+        torch.cuda.synchronize()
+        got.append((o, lse))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
