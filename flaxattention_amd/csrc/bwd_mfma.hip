@@ -83,7 +83,7 @@ size_t flex_dkv_partial_bytes(const FlexAttnParams& p, double slots, double visi
   if (parts > visits) parts = visits;
   // (a call that cannot save 30 us is never divided; even tiles take more rounds than `visits` only beyond the slots)
   if (parts < 2 || (double)visits * visit_us * fmax(1.0, ceil(tiles / slots)) <= 30) return 0;
-  return (size_t)parts * tiles * kListBN * 2 * p.D * sizeof(float);
+  return (size_t)parts * tiles * kListBN * 2 * p.D * sizeof(float) + kPartialAlign;
 }
 
 // two workgroups share a compute unit at D = 64, one has it at D = 128 (and 192 / 256 go to the simple kernel)
@@ -106,8 +106,7 @@ int flex_mfma_bwd(const FlexAttnParams& p, const void* q, const void* k, const v
     return 1;
   }
   const DkvParts n = dkv_parts(p);
-  const size_t delta_bytes = ((size_t)p.B * p.Hq * p.Lq * sizeof(float) + 255) / 256 * 256;
-  const BwdArgs a = {q, k, v, o, d_o, lse2, dq, dk, dv, (float*)workspace, (float*)((char*)workspace + delta_bytes), n.g, n.t, s};
+  const BwdArgs a = {q, k, v, o, d_o, lse2, dq, dk, dv, (float*)workspace, dkv_partial_start(workspace, p), n.g, n.t, s};
   int rc;
   if (p.D >= 192 && !(p.flags & FLEX_BWD_ONLY_DQ)) {
     flex_set_error("fused backward: only the dQ kernel exists for 192- and 256-wide heads");

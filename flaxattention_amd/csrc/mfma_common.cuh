@@ -558,6 +558,14 @@ __device__ __forceinline__ void xcd_tile_map(int wid, int ntile, int nbh, int& r
 // `parts` workgroups share a tile of 128 keys (four waves of 32) and leave float32 partial sums of dK and dV.
 struct DkvParts { int g, t; };   // parts: over the query heads of the group, and over each head's list of query tiles
 
+// where the partial sums start in a backward workspace: behind delta, at the next 16-byte boundary (they are stored as
+// float4, and a caller's workspace need not be aligned to more than a float; the sizes leave room for the gap)
+constexpr size_t kPartialAlign = 16;
+inline float* dkv_partial_start(void* workspace, const FlexAttnParams& p) {
+  const size_t delta_bytes = ((size_t)p.B * p.Hq * p.Lq * sizeof(float) + 255) / 256 * 256;
+  return (float*)(((uintptr_t)workspace + delta_bytes + kPartialAlign - 1) / kPartialAlign * kPartialAlign);
+}
+
 // workgroup id -> (tile's id, part): the parts of a tile stay on one XCD (they read the same K and V) and next to each
 // other in the order
 __device__ __forceinline__ void dkv_part_map(int nbh, int parts, int& wid, int& part) {

@@ -139,7 +139,6 @@ int flex_simple_bwd(const FlexAttnParams& p, const void* q, const void* k, const
   a.q = q; a.k = k; a.v = v; a.o = o; a.d_o = d_o; a.lse2_in = lse2;
   a.dq = dq; a.dk = dk; a.dv = dv; a.delta = (float*)workspace; a.s = s; a.bwd = true;
   a.parts = simple_dkv_parts(p);
-  if (a.parts.g * a.parts.t > 1)
-    a.dkv_partial = (float*)((char*)workspace + ((size_t)p.B * p.Hq * p.Lq * sizeof(float) + 255) / 256 * 256);
+  if (a.parts.g * a.parts.t > 1) a.dkv_partial = dkv_partial_start(workspace, p);
   return dispatch(p, a);
 }

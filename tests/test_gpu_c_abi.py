@@ -227,3 +227,33 @@ def test_no_split_forward_is_the_same_with_a_workspace(dev, dtype, B, H, Lq, Lkv
         torch.cuda.synchronize()
         got.append((o, lse))
     assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+
+
+@pytest.mark.parametrize("dtype,B,H,L,D", [(torch.bfloat16, 1, 4, 2048, 128), (torch.float16, 1, 8, 1024, 256), (torch.float32, 1, 4, 1024, 64)])
+@pytest.mark.parametrize("shift", [0, 4, 12])
+def test_backward_takes_a_workspace_that_is_aligned_to_a_float(dev, dtype, B, H, L, D, shift):
+    """The partial sums of a divided dK/dV call are float4, the workspace may still start at any float: the same bits wherever it
+    lies, and nothing written ahead of it or past its stated size."""
+    print("case workspace alignment", dtype, B, H, L, D, shift, flush=True)
+    lib = _lib.lib()
+    q, k, v = _inputs(dev, B, H, L, L, D, dtype)
+    d_o = _inputs(dev, B, H, L, L, D, dtype)[0].flip(2).contiguous()
+    o, lse = torch.empty_like(q), torch.empty(B, H, L, device=dev)
+    p = _params(q, k, v, o, lo=0)
+    p.flags = 0 if dtype == torch.float32 else 1
+    _lib.check(lib.flexattn_fwd(p, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse.data_ptr(), None, _stream()), "fwd")
+    nbytes = lib.flexattn_bwd_workspace_bytes(p)
+    delta = (B * H * L * 4 + 255) // 256 * 256
+    assert (nbytes - delta) % (128 * 2 * D * 4) == 16       # whole tiles, and the gap up to a 16-byte boundary
+    got = []
+    for at in (0, shift):
+        buf = torch.full((nbytes + 4096,), 0x5A, dtype=torch.uint8, device=dev)
+        assert buf.data_ptr() % 256 == 0
+        grads = [torch.empty_like(t) for t in (q, k, v)]
+        _lib.check(lib.flexattn_bwd(p, *(t.data_ptr() for t in (q, k, v, o, lse, d_o, *grads)), buf.data_ptr() + 256 + at, _stream()), "bwd")
+        torch.cuda.synchronize()
+        ahead, partials, behind = (bool((part == 0x5A).all()) for part in (
+            buf[:256 + at], buf[256 + at + delta:256 + at + nbytes], buf[256 + at + nbytes:]))
+        assert ahead and behind and not partials      # the partial sums are there, and nothing beside the workspace
+        got.append(grads)
+    assert all(torch.equal(a, b) for a, b in zip(*got))
