@@ -65,8 +65,8 @@ EXPORTS = [
     "flexattn_abi_version", "flexattn_last_error", "flexattn_preferred_tiles", "flexattn_kernel_family",
     "flexattn_block_mask_workspace_bytes", "flexattn_block_mask_build", "flexattn_pack_mask", "flexattn_bitmap_fit",
     "flexattn_affine_tables",
-    "flexattn_fwd_workspace_bytes", "flexattn_fwd",
-    "flexattn_bwd_workspace_bytes", "flexattn_bwd",
+    "flexattn_fwd_workspace_bytes", "flexattn_fwd_workspace_needed", "flexattn_fwd",
+    "flexattn_bwd_workspace_bytes", "flexattn_bwd_workspace_needed", "flexattn_bwd",
     "flexattn_decode_workspace_bytes", "flexattn_decode", "flexattn_decode_static",
 ]
 
@@ -107,11 +107,10 @@ def lib() -> C.CDLL:
     L.flexattn_pack_mask.argtypes = [C.c_void_p, C.POINTER(C.c_int64)] + [C.c_int32] * 6 + [C.c_void_p] * 4
     L.flexattn_bitmap_fit.argtypes = [C.c_void_p] + [C.c_int32] * 3 + [C.c_void_p] * 2
     L.flexattn_affine_tables.argtypes = [C.c_void_p, C.c_int64] + [C.c_int32] * 2 + [C.c_void_p] * 5
-    L.flexattn_fwd_workspace_bytes.restype = C.c_size_t
-    L.flexattn_fwd_workspace_bytes.argtypes = [C.POINTER(FlexAttnParams)]
+    for fn in (L.flexattn_fwd_workspace_bytes, L.flexattn_fwd_workspace_needed, L.flexattn_bwd_workspace_bytes,
+               L.flexattn_bwd_workspace_needed):
+        fn.restype, fn.argtypes = C.c_size_t, [C.POINTER(FlexAttnParams)]
     L.flexattn_fwd.argtypes = [C.POINTER(FlexAttnParams)] + [C.c_void_p] * 7
-    L.flexattn_bwd_workspace_bytes.restype = C.c_size_t
-    L.flexattn_bwd_workspace_bytes.argtypes = [C.POINTER(FlexAttnParams)]
     L.flexattn_bwd.argtypes = [C.POINTER(FlexAttnParams)] + [C.c_void_p] * 11
     L.flexattn_decode_workspace_bytes.restype = C.c_size_t
     L.flexattn_decode_workspace_bytes.argtypes = [C.POINTER(FlexAttnParams), C.c_int32]

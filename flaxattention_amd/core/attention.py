@@ -360,7 +360,7 @@ def _run_fwd(plan: _Plan, q, k, v) -> Tuple[Array, Array]:
                     # never needs (it always passes lse2): beyond that part, the bytes are split partials
                     parity = (plan.flags & _lib.FLAG_PARITY) and not (plan.flags & _lib.FLAG_UNROUNDED)
                     lse_part = (plan.B * plan.Hq * plan.Lq * 4 + 255) // 256 * 256 if parity else 0
-                    nbytes = int(L.flexattn_fwd_workspace_bytes(p))
+                    nbytes = int(L.flexattn_fwd_workspace_needed(p))
                     plan.fwd_ws_bytes = nbytes if nbytes > lse_part else 0
                 if plan.fwd_ws_bytes:
                     ws = torch.empty(plan.fwd_ws_bytes, dtype=torch.uint8, device=q.device)
@@ -388,7 +388,7 @@ def _run_bwd(plan: _Plan, q, k, v, o, lse2, d_o, d_lse2=None) -> Tuple[Array, Ar
         p2.d_lse2 = d_lse2.data_ptr()
         p = p2
     with _on_device(q.device):
-        ws = torch.empty(max(L.flexattn_bwd_workspace_bytes(p), 256), dtype=torch.uint8, device=q.device)
+        ws = torch.empty(max(L.flexattn_bwd_workspace_needed(p), 256), dtype=torch.uint8, device=q.device)
         rc = L.flexattn_bwd(p, q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), lse2.data_ptr(), d_o.data_ptr(),
                             dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ws.data_ptr(), _stream(q))
     _lib.check(rc, "flexattn_bwd")

@@ -73,7 +73,16 @@ DkvParts flex_dkv_parts(const FlexAttnParams& p, double slots, double visit_us) 
   }
   return best;
 }
-// Bytes of the partial sums for the most parts any mask and lists can get: a workspace is sized by the shape alone.
+static size_t partial_bytes(const FlexAttnParams& p, int64_t parts) {
+  const int64_t tiles = (int64_t)((p.Lkv + kListBN - 1) / kListBN) * p.Hkv * p.B;
+  return parts < 2 ? 0 : (size_t)parts * tiles * kListBN * 2 * p.D * sizeof(float) + kPartialAlign;
+}
+// bytes of the partial sums of this very call, with its mask and lists
+size_t flex_dkv_partial_bytes_of(const FlexAttnParams& p, double slots, double visit_us) {
+  const DkvParts n = flex_dkv_parts(p, slots, visit_us);
+  return partial_bytes(p, (int64_t)n.g * n.t);
+}
+// and for the most parts any mask and lists can get: a workspace may be sized by the shape alone
 size_t flex_dkv_partial_bytes(const FlexAttnParams& p, double slots, double visit_us) {
   if (p.flags & (FLEX_UNROUNDED | FLEX_NO_SPLIT)) return 0;
   const int64_t tiles = (int64_t)((p.Lkv + kListBN - 1) / kListBN) * p.Hkv * p.B;
@@ -83,7 +92,7 @@ size_t flex_dkv_partial_bytes(const FlexAttnParams& p, double slots, double visi
   if (parts > visits) parts = visits;
   // (a call that cannot save 30 us is never divided; even tiles take more rounds than `visits` only beyond the slots)
   if (parts < 2 || (double)visits * visit_us * fmax(1.0, ceil(tiles / slots)) <= 30) return 0;
-  return (size_t)parts * tiles * kListBN * 2 * p.D * sizeof(float) + kPartialAlign;
+  return partial_bytes(p, parts);
 }
 
 // two workgroups share a compute unit at D = 64, one has it at D = 128 (and 192 / 256 go to the simple kernel)
@@ -94,9 +103,10 @@ static DkvParts dkv_parts(const FlexAttnParams& p) {
   return flex_dkv_parts(p, dkv_slots(p), kVisitUs);
 }
 
-// beside delta, which the caller accounts for: the partial sums of a divided dK/dV call
-size_t flex_mfma_bwd_workspace(const FlexAttnParams& p) {
-  return p.D == 64 || p.D == 128 ? flex_dkv_partial_bytes(p, dkv_slots(p), kVisitUs) : 0;
+// beside delta, which the caller accounts for: the partial sums of a divided dK/dV call (any_mask: of any call of the shape)
+size_t flex_mfma_bwd_workspace(const FlexAttnParams& p, bool any_mask) {
+  if (p.D != 64 && p.D != 128) return 0;
+  return (any_mask ? flex_dkv_partial_bytes : flex_dkv_partial_bytes_of)(p, dkv_slots(p), kVisitUs);
 }
 
 int flex_mfma_bwd(const FlexAttnParams& p, const void* q, const void* k, const void* v, const void* o, const float* lse2,

@@ -48,7 +48,7 @@ int flex_mfma_fwd(const FlexAttnParams& p, const void* q, const void* k, const v
                   void* partials, hipStream_t s);
 bool flex_mfma_bwd_supported(const FlexAttnParams& p);
 bool flex_mfma_dq_wide_supported(const FlexAttnParams& p);
-size_t flex_mfma_bwd_workspace(const FlexAttnParams& p);
+size_t flex_mfma_bwd_workspace(const FlexAttnParams& p, bool any_mask);
 int flex_mfma_bwd(const FlexAttnParams& p, const void* q, const void* k, const void* v, const void* o, const float* lse2,
                   const void* d_o, void* dq, void* dk, void* dv, void* workspace, hipStream_t s);
 bool flex_decode_supported(const FlexAttnParams& p);
@@ -64,7 +64,7 @@ int flex_simple_fwd_splits(const FlexAttnParams& p, bool any_mask);
 size_t flex_simple_fwd_partial_bytes(const FlexAttnParams& p, int splits);
 int flex_simple_fwd(const FlexAttnParams& p, const void* q, const void* k, const void* v, void* o, float* lse2, int splits,
                     void* partials, hipStream_t s);
-size_t flex_simple_bwd_workspace(const FlexAttnParams& p);
+size_t flex_simple_bwd_workspace(const FlexAttnParams& p, bool any_mask);
 int flex_simple_bwd(const FlexAttnParams& p, const void* q, const void* k, const void* v, const void* o, const float* lse2,
                     const void* d_o, void* dq, void* dk, void* dv, void* workspace, hipStream_t s);
 
@@ -148,15 +148,17 @@ static size_t fwd_lse_bytes(const FlexAttnParams* p) {
   return ((p->flags & FLEX_PARITY) && !(p->flags & FLEX_UNROUNDED)) ? lse_bytes(p) : 0;
 }
 
-extern "C" size_t flexattn_fwd_workspace_bytes(const FlexAttnParams* p) {
+static size_t fwd_workspace(const FlexAttnParams* p, bool any_mask) {
   if (!p) return 0;
   size_t n = fwd_lse_bytes(p);
   // the matrix-core forward kernels split the keys of a call with few query tiles over several workgroups, whose
   // partial results live here
-  if (wants_fused(p) && flex_mfma_fwd_supported(*p)) n += flex_mfma_fwd_partial_bytes(*p, flex_mfma_fwd_splits(*p, true));
-  else if (wants_fused(p) && flex_simple_supported(*p, 0)) n += flex_simple_fwd_partial_bytes(*p, flex_simple_fwd_splits(*p, true));
+  if (wants_fused(p) && flex_mfma_fwd_supported(*p)) n += flex_mfma_fwd_partial_bytes(*p, flex_mfma_fwd_splits(*p, any_mask));
+  else if (wants_fused(p) && flex_simple_supported(*p, 0)) n += flex_simple_fwd_partial_bytes(*p, flex_simple_fwd_splits(*p, any_mask));
   return n;
 }
+extern "C" size_t flexattn_fwd_workspace_bytes(const FlexAttnParams* p) { return fwd_workspace(p, true); }
+extern "C" size_t flexattn_fwd_workspace_needed(const FlexAttnParams* p) { return fwd_workspace(p, false); }
 
 extern "C" int flexattn_fwd(const FlexAttnParams* p, const void* q, const void* k, const void* v, void* o, float* lse2,
                             void* workspace, flexattn_stream_t stream) {
@@ -199,13 +201,15 @@ extern "C" int flexattn_fwd(const FlexAttnParams* p, const void* q, const void* 
 
 static size_t delta_bytes(const FlexAttnParams* p) { return ((size_t)p->B * p->Hq * p->Lq * sizeof(float) + 255) / 256 * 256; }
 
-extern "C" size_t flexattn_bwd_workspace_bytes(const FlexAttnParams* p) {
+static size_t bwd_workspace(const FlexAttnParams* p, bool any_mask) {
   if (!p) return 0;
   size_t n = delta_bytes(p);
-  if (wants_fused(p) && flex_simple_supported(*p, 1)) n += flex_simple_bwd_workspace(*p);
-  else if (wants_fused(p) && flex_mfma_bwd_supported(*p)) n += flex_mfma_bwd_workspace(*p);
+  if (wants_fused(p) && flex_simple_supported(*p, 1)) n += flex_simple_bwd_workspace(*p, any_mask);
+  else if (wants_fused(p) && flex_mfma_bwd_supported(*p)) n += flex_mfma_bwd_workspace(*p, any_mask);
   return n;
 }
+extern "C" size_t flexattn_bwd_workspace_bytes(const FlexAttnParams* p) { return bwd_workspace(p, true); }
+extern "C" size_t flexattn_bwd_workspace_needed(const FlexAttnParams* p) { return bwd_workspace(p, false); }
 
 extern "C" int flexattn_bwd(const FlexAttnParams* p, const void* q, const void* k, const void* v, const void* o,
                             const float* lse2, const void* d_o, void* dq, void* dk, void* dv, void* workspace,

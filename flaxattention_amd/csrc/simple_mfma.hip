@@ -7,6 +7,7 @@ void flex_set_error(const char* fmt, ...);
 int flex_cu_count();
 DkvParts flex_dkv_parts(const FlexAttnParams& p, double slots, double visit_us);
 size_t flex_dkv_partial_bytes(const FlexAttnParams& p, double slots, double visit_us);
+size_t flex_dkv_partial_bytes_of(const FlexAttnParams& p, double slots, double visit_us);
 int flex_simple_f32_64(const FlexAttnParams& p, const SimpleArgs& a);
 int flex_simple_f32_128(const FlexAttnParams& p, const SimpleArgs& a);
 int flex_simple_f16_192(const FlexAttnParams& p, const SimpleArgs& a);
@@ -125,8 +126,8 @@ int flex_simple_fwd(const FlexAttnParams& p, const void* q, const void* k, const
 // 13 us at D = 192 / 256 in 16 bits and 18 / 36 us at D = 64 / 128 in float32; one workgroup per compute unit.
 static double simple_visit_us(const FlexAttnParams& p) { return p.dtype != FLEX_F32 ? 13. : p.D == 64 ? 18. : 36.; }
 static DkvParts simple_dkv_parts(const FlexAttnParams& p) { return flex_dkv_parts(p, flex_cu_count(), simple_visit_us(p)); }
-size_t flex_simple_bwd_workspace(const FlexAttnParams& p) {
-  return flex_dkv_partial_bytes(p, flex_cu_count(), simple_visit_us(p));
+size_t flex_simple_bwd_workspace(const FlexAttnParams& p, bool any_mask) {
+  return (any_mask ? flex_dkv_partial_bytes : flex_dkv_partial_bytes_of)(p, flex_cu_count(), simple_visit_us(p));
 }
 
 int flex_simple_bwd(const FlexAttnParams& p, const void* q, const void* k, const void* v, const void* o, const float* lse2,

@@ -244,6 +244,9 @@ int flexattn_affine_tables(const float* values, int64_t maps, int32_t rows, int3
  * with Dv features; lse2: [B,Hq,Lq] fp32 base-2 log-sum-exp (-inf on rows with
  * no visible key), may be NULL.  */
 size_t flexattn_fwd_workspace_bytes(const FlexAttnParams* p);
+/* The part of flexattn_fwd_workspace_bytes (the most any mask of the shape takes) that a call with exactly these
+ * parameters, mask and lists among them, uses: enough for that call.  flexattn_bwd_workspace_needed likewise. */
+size_t flexattn_fwd_workspace_needed(const FlexAttnParams* p);
 int flexattn_fwd(const FlexAttnParams* p, const void* q, const void* k, const void* v,
                  void* o, float* lse2, void* workspace, flexattn_stream_t stream);
 
@@ -253,6 +256,7 @@ int flexattn_fwd(const FlexAttnParams* p, const void* q, const void* k, const vo
  * d_o is a contiguous [B,Hq,Lq,Dv] tensor (the strides in `p` describe q, k,
  * v and o only); dq/dk/dv are contiguous [B,H,L,D] tensors of the input dtype.  */
 size_t flexattn_bwd_workspace_bytes(const FlexAttnParams* p);
+size_t flexattn_bwd_workspace_needed(const FlexAttnParams* p);
 int flexattn_bwd(const FlexAttnParams* p, const void* q, const void* k, const void* v,
                  const void* o, const float* lse2, const void* d_o,
                  void* dq, void* dk, void* dv, void* workspace, flexattn_stream_t stream);

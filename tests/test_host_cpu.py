@@ -540,3 +540,32 @@ def test_undivided_wide_backward_keeps_its_registers():
                 found = [k for n, k in kernels.items() if f"simple_dkv_kernelI{dtype}Li256ELi{kind}ELb{b}ELb0E" in n]
                 assert len(found) == 1, (dtype, kind, numerics)
                 assert found[0][".vgpr_spill_count"] <= bound, (dtype, kind, numerics, found[0][".vgpr_spill_count"])
+
+
+@pytest.mark.parametrize("dtype,D", [(_lib.FLEX_F16, 64), (_lib.FLEX_BF16, 128), (_lib.FLEX_F16, 256), (_lib.FLEX_F32, 64), (_lib.FLEX_F32, 128)])
+def test_a_call_is_told_what_it_uses_of_the_workspace(dtype, D):
+    """The sizes by shape cover every mask of the shape; what one call uses is never more, and nothing beyond delta where it
+    divides nothing: a dense call of a causal-sized shape, short sequences, FLEX_NO_SPLIT."""
+    L = _lib.lib()
+    bands = {"none": (-2**31, 2**31 - 1, -1), "causal": (0, 2**31 - 1, -1), "window": (0, 500, -1), "sink": (0, 500, 3)}
+    shapes = ((1, 8, 2, 2048, 2048), (2, 8, 8, 2048, 2048), (1, 2, 1, 130, 5000), (1, 1, 1, 128, 128), (1, 8, 8, 8192, 8192),
+              (16, 16, 16, 4096, 4096), (1, 32, 8, 4096, 4096), (1, 4, 4, 700, 900))
+    for B, Hq, Hkv, Lq, Lkv in shapes:
+        for name, (lo, hi, sink) in bands.items():
+            p = _lib.FlexAttnParams()
+            p.dtype, p.B, p.Hq, p.Hkv, p.Lq, p.Lkv, p.D, p.Dv = dtype, B, Hq, Hkv, Lq, Lkv, D, D
+            for field, H, n in (("q_stride", Hq, Lq), ("k_stride", Hkv, Lkv), ("v_stride", Hkv, Lkv), ("o_stride", Hq, Lq)):
+                getattr(p, field)[:] = [H * n * D, n * D, D]
+            p.mask.lo, p.mask.hi, p.mask.sink = lo, hi, sink
+            delta = (B * Hq * Lq * 4 + 255) // 256 * 256
+            fwd, bwd = L.flexattn_fwd_workspace_needed(p), L.flexattn_bwd_workspace_needed(p)
+            assert fwd <= L.flexattn_fwd_workspace_bytes(p) and delta <= bwd <= L.flexattn_bwd_workspace_bytes(p)
+            assert bwd == delta or (bwd - delta - 16) % (((Lkv + 127) // 128) * Hkv * B * 128 * 2 * D * 4) == 0
+            if (B, Lq) in ((16, 4096), (1, 128)):
+                assert bwd == delta, (name, B, Lq)
+            # as many query tiles as fit at once: halved under a causal mask only
+            if (B, Lq) == ((2, 2048) if D == 256 else (1, 8192)) and Hq == Hkv:
+                assert (fwd > 0) == (name == "causal" and D >= 128 and dtype != _lib.FLEX_F32), (name, fwd)
+            p.flags = _lib.FLAG_NO_SPLIT
+            assert L.flexattn_bwd_workspace_needed(p) == L.flexattn_bwd_workspace_bytes(p) == delta
+            assert L.flexattn_fwd_workspace_needed(p) == L.flexattn_fwd_workspace_bytes(p) == 0
