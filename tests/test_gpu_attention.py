@@ -1184,7 +1184,8 @@ def test_backward_split_over_the_queries(dev, dtype, B, Hq, Hkv, Lq, Lkv, D, kin
         if split:
             out, lse2 = _run_fwd(plan, qd, kd, vd)
         delta = (B * Hq * Lq * 4 + 255) // 256 * 256
-        assert (_lib.lib().flexattn_bwd_workspace_bytes(plan.params(qd, kd, vd, out)) > delta) == split
+        # (what this very call uses; the size by shape alone would not tell whether it is divided)
+        assert (_lib.lib().flexattn_bwd_workspace_needed(plan.params(qd, kd, vd, out)) > delta) == split
         grads[split] = _run_bwd(plan, qd, kd, vd, out, lse2, dod)
     assert torch.equal(grads[True][0], grads[False][0])
     want = ref_attention_bwd(q, k, v, d_o, None, omask, strict=True)
@@ -1248,7 +1249,9 @@ def test_forward_with_uneven_tiles_is_halved(dev, dtype, B, H, Lq, Lkv, D, halve
     plan = _make_plan(q, k, v, None, bm, None, D ** -0.5, None)
     lse_part = (B * H * Lq * 4 + 255) // 256 * 256 if dtype == torch.bfloat16 else 0
     rows = (B * H * Lq * 2 * (D + 2) * 4 + 255) // 256 * 256
-    assert _lib.lib().flexattn_fwd_workspace_bytes(plan.params(q, k, v, q)) - lse_part == (rows if halved else 0)
+    assert _lib.lib().flexattn_fwd_workspace_needed(plan.params(q, k, v, q)) - lse_part == (rows if halved else 0)
+    dense = _make_plan(q, k, v, None, None, None, D ** -0.5, None)   # even tiles: not halved
+    assert _lib.lib().flexattn_fwd_workspace_needed(dense.params(q, k, v, q)) == lse_part
     a, la = fa.flax_attention(q, k, v, block_mask=bm, return_lse=True)
     b, lb = fa.flax_attention(q, k, v, block_mask=bm, return_lse=True, kernel_options={"split_kv": False})
     assert (la - lb).abs().max().item() <= 1e-5   # float32 sums of up to 8150 terms in another order
