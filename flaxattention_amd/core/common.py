@@ -267,7 +267,7 @@ def affine_score_mod(fn: Callable, B: int, H: int, Lq: int, Lkv: int, device, co
     near = (min(B, 2), H, min(Lq, P), min(Lkv, P + 2))
     if corner is not None and all(have >= want for have, want in zip(corner.shape[1:], near)):
         return _affine_tables(fn, B, H, Lq, Lkv, device, corner[:, :near[0], :near[1], :near[2], :near[3]])
-    s = torch.tensor([-1.75, -0.5, 0.0, 0.625, 2.5], dtype=torch.float32).reshape(5, 1, 1, 1, 1)
+    s = torch.tensor(_CORNER_SCORES, dtype=torch.float32).reshape(5, 1, 1, 1, 1)
     b = torch.arange(min(B, 2), dtype=torch.int32).reshape(1, -1, 1, 1, 1)
     h = torch.arange(H, dtype=torch.int32).reshape(1, 1, H, 1, 1)
     q = torch.arange(min(Lq, P), dtype=torch.int32).reshape(1, 1, 1, -1, 1)
@@ -294,10 +294,10 @@ def _affine_tables(fn: Callable, B: int, H: int, Lq: int, Lkv: int, device, out:
         return None
     name = getattr(fn, "__name__", "affine_score_mod")
     # One call of the callable at all six scores, one kernel that makes the tables and checks them on every position, one
-    # wait -- as long as six planes are small (a corner that does not vary over the batch counts as one that has no batch
-    # extent); larger problems are read off and checked piece by piece below.
-    planes = (1 if bool((out == out[:, :1]).all()) else B) * H * Lq * Lkv
-    if torch.device(device).type == "cuda" and planes <= _SIX_PLANES_ELEMS:
+    # wait -- as long as six planes of what the callable returns are small; larger problems, and those whose planes find no
+    # room, are read off and checked piece by piece below.
+    y = None
+    if torch.device(device).type == "cuda" and _result_positions(fn, B, H, Lq, Lkv, device) <= _SIX_PLANES_ELEMS:
         try:
             y = torch.as_tensor(fn(*_grid5(_TABLE_SCORES, (B, H, Lq, Lkv), device))).to(torch.float32)
             y = y.reshape((1,) * (5 - y.dim()) + tuple(y.shape))
@@ -306,9 +306,12 @@ def _affine_tables(fn: Callable, B: int, H: int, Lq: int, Lkv: int, device, out:
                 y = None
         except Exception:   # (what a callable raises on five-dimensional tensors it may not raise on four)
             y = None
-        if y is not None:
+    if y is not None:
+        try:
             y = torch.broadcast_to(y, (6, *extents, Lkv)).contiguous()
             return _tables_of_planes(fn, name, y, Lq)
+        except torch.OutOfMemoryError:
+            y = None
     # the tables, on the device; a [1,1,1,1] score keeps every extent the callable does not use at 1
     bi = torch.arange(B, dtype=torch.int32, device=device).reshape(B, 1, 1, 1)
     hi = torch.arange(H, dtype=torch.int32, device=device).reshape(1, H, 1, 1)
@@ -355,6 +358,19 @@ def _affine_tables(fn: Callable, B: int, H: int, Lq: int, Lkv: int, device, out:
         spec.add = torch.cat([add[:, :, :, 0].flip(-1), add[:, :, 0, 1:]], dim=-1).contiguous()
         spec.diag_zero = Lq - 1
     return spec
+
+
+def _result_positions(fn: Callable, B: int, H: int, Lq: int, Lkv: int, device) -> int:
+    """Positions of what the callable returns over the whole problem.  Where all of them are too many for one call, its
+    batch and head extents are read off the shape it returns for a single position."""
+    if B * H * Lq * Lkv <= _SIX_PLANES_ELEMS:
+        return B * H * Lq * Lkv
+    try:
+        shape = torch.as_tensor(fn(*_grid5(_TABLE_SCORES, (B, H, 1, 1), device))).shape
+    except Exception:
+        return B * H * Lq * Lkv
+    shape = (1,) * (5 - len(shape)) + tuple(shape)
+    return shape[1] * shape[2] * Lq * Lkv
 
 
 def _tables_of_planes(fn: Callable, name: str, y: torch.Tensor, Lq: int) -> Optional[ScoreMod]:

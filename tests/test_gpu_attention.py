@@ -1235,6 +1235,41 @@ def test_affine_lowering_in_one_call_equals_the_general_path(dev, B, H, Lq, Lkv,
     assert common.affine_score_mod(mods["not finite"], B, H, Lq, Lkv, dev) is None
 
 
+def test_affine_lowering_in_one_call_is_bounded(dev, monkeypatch):
+    """The evaluation at six scores stays within its bound whatever the corner of the index space looks like, and where its
+    planes do not fit the callable is read off piece by piece: the same tables."""
+    from flaxattention_amd.core import common
+    print("case affine bound", flush=True)
+    B, H, Lq, Lkv = 40, 2, 24, 40
+    g = torch.Generator(device=dev).manual_seed(8)
+    late = torch.randn(B, H, Lq, Lkv, generator=g, device=dev)
+    late[:3] = 0                                    # the first sequences agree
+    shared = torch.randn(H, Lq, Lkv, generator=g, device=dev)
+    sizes = []
+
+    def watched(table):
+        def mod(s, b, h, q, kv):
+            y = s + (table[b, h, q, kv] if table.dim() == 4 else table[h, q, kv])
+            sizes.append(y.numel())
+            return y
+        return mod
+    want = [common.affine_score_mod(watched(t), B, H, Lq, Lkv, dev) for t in (late, shared)]
+    assert max(sizes) == 6 * B * H * Lq * Lkv and want[0].add.shape == (B, H, Lq, Lkv) and want[1].add.shape == (1, H, Lq, Lkv)
+    monkeypatch.setattr(common, "_SIX_PLANES_ELEMS", 4 * H * Lq * Lkv)     # four batch elements' worth
+    for table, ref, most in ((late, want[0], B * H * Lq * Lkv), (shared, want[1], 6 * H * Lq * Lkv)):
+        sizes.clear()
+        got = common.affine_score_mod(watched(table), B, H, Lq, Lkv, dev)
+        assert max(sizes) == most, sizes      # (piece by piece: one plane at a time)
+        assert torch.equal(got.add, ref.add) and got.mul is None and ref.mul is None
+    monkeypatch.undo()
+
+    def no_room(*a):
+        raise torch.OutOfMemoryError("planes")
+    monkeypatch.setattr(common, "_tables_of_planes", no_room)
+    got = common.affine_score_mod(watched(late), B, H, Lq, Lkv, dev)
+    assert torch.equal(got.add, want[0].add)
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["f16", "bf16"])
 @pytest.mark.parametrize("B,H,Lq,Lkv,D,halved", [(2, 8, 2001, 2048, 256, True), (3, 5, 2048, 2000, 192, True),
                                                  (1, 8, 7777, 8150, 128, True), (1, 16, 4096, 4096, 64, False)])
