@@ -44,7 +44,8 @@ selects numerics here:
     {"split_kv": bool}    False: the forward kernel never splits a call over the keys
                           (by default it does when the query tiles alone are fewer
                           workgroups than the GPU has compute units), and the backward
-                          never splits a key tile's queries; the result of a
+                          never splits a key tile's queries (by default it does
+                          where key tiles are few or uneven); the result of a
                           (batch, head) pair then does not depend on how many pairs
                           the call has, bit for bit
     {"pad_head_dim": bool}  inputs whose head sizes are not among those of the matrix-core kernels

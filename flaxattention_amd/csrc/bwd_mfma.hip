@@ -40,10 +40,10 @@ bool flex_mfma_bwd_supported(const FlexAttnParams& p) {
 // How many workgroups share a key tile of a dK/dV kernel of which the chip holds `slots` at once: n.g over the query heads
 // of the group times n.t over each head's list of query tiles.  A key tile's workgroup visits up to `visits` query tiles
 // of visit_us each; under a mask the work of the tiles differs (causal: the heaviest is twice the mean), so with no more
-// tiles than slots the heaviest one is the call: bf16 [1,32->8,4096,128] causal, 256 tiles on 256 slots, 637 us against
-// 398 + 14 us in two parts; f16 [2,8,2048,256] causal 214 us against
-// 148 + 27 us.  What adding the partial sums costs: a launch, and their
-// bytes twice (27 us for twice 256 slots at D = 128, about half of it hidden).  Taken where it promises a fifth and 30 us
+// tiles than slots the heaviest one is the call.  dK/dV as calls of their own, merge included, undivided -> in two parts: bf16
+// [1,32->8,4096,128] causal, 256 tiles on 256 slots, 598 -> 346 us; f16 [2,8,2048,256] causal 203 -> 156 us, bf16
+// 262 -> 197 us.  What adding the partial sums costs: a launch, and their bytes twice (at the copy rate 27 us for twice 256
+// slots at D = 128, 54 us at 256; about half of it hidden).  Taken where it promises a fifth and 30 us
 // (less is lost again on the second launch where the host sets the pace: bf16 [1,4,881,64] causal 131 -> 145 us).
 DkvParts flex_dkv_parts(const FlexAttnParams& p, double slots, double visit_us) {
   if (p.flags & (FLEX_UNROUNDED | FLEX_NO_SPLIT)) return {1, 1};
