@@ -1,5 +1,7 @@
 // Simple matrix-core kernels (float32 at D 64 / 128, fp16 / bf16 at D 192 / 256): checks and dispatch.  The kernels
 // are in simple_mfma.cuh, instantiated per (dtype, head size) by simple_mfma_inst.hip.
+#include <cmath>
+
 #include "simple_mfma.cuh"
 
 using namespace flex;
@@ -66,22 +68,37 @@ static int splits_over_keys(const FlexAttnParams& p) {
 }
 // Float32 forwards of few query tiles: 32 rows per workgroup with the key steps divided over its waves
 // (simple_fwd_short_kernel) instead of 128 rows.  Four times the workgroups with a quarter of the chain, so it wins while those
-// fit the chip about twice (causal: while the 128-row ones fit once, their tiles being uneven), and loses beyond, where
-// it only reads K and V four times as often.  us, 128 rows / 32 rows, D = 64 and 128: 8 tiles [1,4,256] causal 27 / 17
-// and 43 / 19; 16 tiles [1,4,512] 48 / 19 and 80 / 31; 128 tiles [4,8,512] dense 48 / 35 and 82 / 63; 192 tiles [8,8,384]
-// causal 38 / 30 and 63 / 53, dense 37 / 40; 256 tiles [8,16,256] causal 28 / 32, [4,8,1024] causal 92 / 73.  Against the split
-// over workgroups below, by their chains: 32 tiles [1,4,1024] 52 / 33, 128 tiles [2,8,1024] causal 60 / 39 but dense
-// 97 / 112 at D = 128.
+// fit the chip about twice, and loses beyond, where it only reads K and V four times as often.  us, 128 rows / 32 rows,
+// D = 64 and 128: 8 tiles [1,4,256] causal 27 / 17 and 43 / 19; 16 tiles [1,4,512] 48 / 19 and 80 / 31; 128 tiles [4,8,512]
+// dense 48 / 35 and 82 / 63; 192 tiles [8,8,384] dense 37 / 40; 256 tiles [8,16,256] causal 28 / 32.
+// More tiles than that only where they are uneven (causal, the heaviest twice the mean) and the mean chain they are cut to
+// outweighs four times the workgroups: 192 tiles [8,8,384] 38 / 30 and 63 / 53, 256 tiles [4,8,1024] 92 / 73 and 157 / 133, [8,8,512]
+// 49 / 46 and 82 / 81, but 240 tiles [1,80,384] 39 / 39 and 64 / 68.  A window's tiles are even: 256 tiles [1,8,4096] window
+// 1000 106 / 130 and 180 / 236, four sinks and window 100 35 / 52 and 55 / 86.
+// Against the split over workgroups above, by their chains: causal 32 tiles [1,4,1024] 52 / 33, 128 tiles [2,8,1024] 60 / 39 and
+// 91 / 68; but 96 tiles [1,6,2048 against 33 keys] at D = 128 17.5 / 20.5; dense 96 tiles [1,6,2048] 97 / 115 and 163 / 221, three packed documents there 53 / 38 and 81 / 64 (as a bitmap, which
+// counts as dense); window 64, 96 tiles [1,3,4096] 23 / 18 and 32 / 24, window 300 35 / 31 and 50 / 52, window 1000 65 / 70 and
+// 102 / 129.
 static bool short_rows(const FlexAttnParams& p) {
   if (p.dtype != FLEX_F32 || (p.flags & FLEX_NO_SPLIT)) return false;
   const int64_t wgs = (int64_t)((p.Lq + kSimpleQTile - 1) / kSimpleQTile) * p.Hq * p.B;
   const int cus = flex_cu_count(), steps = (p.Lkv + kSimpleStep - 1) / kSimpleStep, splits = splits_over_keys(p);
+  const bool window = p.mask.kind == FLEX_MASK_BAND && p.mask.hi != INT32_MAX;
   const bool causal = p.mask.kind == FLEX_MASK_BAND && p.mask.lo != INT32_MIN && p.Lq > p.Lkv / 2;
-  if (wgs > cus / 2) return causal && wgs <= cus && steps >= 12;
-  if (splits == 1) return true;
-  double rounds = 4. * wgs / cus * (causal ? 0.5 : 1.);
-  if (rounds < 1) rounds = 1;
-  return 1.1 * rounds * steps / 4 <= (double)steps / splits;
+  const double fill = (double)wgs / cus;
+  if (wgs > cus / 2) return causal && !window && wgs <= cus && steps >= 12 && steps * (1 - 0.5 * fill) > 7.5 * fill;
+  if (causal && !window && splits > 1) return 1.1 * fmax(1, 2 * fill) * steps / 4 <= (double)steps / splits;
+  // even tiles, and calls of so few keys that the split above leaves them whole: the steps a 128-row tile lists (a bitmap may
+  // list all of them) against the visits of a wave of 32 rows, in as many rounds as four times the workgroups take; a visit
+  // costs more than a step of the tile does
+  double listed = steps, mine = steps;
+  if (window && splits > 1) {
+    const double width = p.mask.lo == INT32_MIN ? p.Lkv : fmin(p.Lkv, (double)p.mask.hi - p.mask.lo);
+    const bool sinks = p.mask.sink >= 0;
+    listed = fmin(steps, (width + 128) / 32 + 1 + 2 * sinks);
+    mine = fmin(steps, (width + 32) / 32 + 1 + sinks);
+  }
+  return ceil(4 * fill) * ceil(mine / 4) * (p.D == 64 ? 1.25 : 1.4) <= listed / splits + 0.5;
 }
 // any_mask: the most any mask gets (a workspace is sized by the shape alone)
 int flex_simple_fwd_splits(const FlexAttnParams& p, bool any_mask) {

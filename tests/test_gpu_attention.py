@@ -1321,6 +1321,25 @@ def test_short_float32_forward(dev, B, Hq, Hkv, Lq, Lkv, D, kind):
         assert max_abs(lse.cpu()[~dead], want_lse[~dead]) <= 1e-4
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("H,Lq,Lkv,kind,short", [(8, 4096, 4096, "window", False), (16, 2048, 2048, "sink", False), (80, 384, 384, "causal", False),
+                                                 (6, 2048, 33, "none", False), (32, 1024, 1024, "causal", True), (6, 2048, 2048, "causal", True)])
+def test_float32_forward_of_even_tiles_keeps_its_rows(dev, H, Lq, Lkv, kind, short, D):
+    """Float32 calls whose tiles fill the compute units evenly (windows), or have few keys, are not cut into workgroups of 32 rows:
+    the bits of the undivided call; uneven ones are, and their float32 sums only run in another order."""
+    print("case f32 rows", H, Lq, Lkv, kind, D, flush=True)
+    q, k, v = (t.to(dev) for t in seeded_qkv(1, H, H, Lq, Lkv, D, torch.float32))
+    mask = {"window": generate_sliding_window(1000), "sink": generate_attention_sink(100, 3), "causal": causal_mask, "none": None}[kind]
+    bm = fa.create_block_mask(mask, None, None, Lq, Lkv, device=dev) if mask is not None else None
+    a, la = fa.flax_attention(q, k, v, block_mask=bm, return_lse=True)
+    b, lb = fa.flax_attention(q, k, v, block_mask=bm, return_lse=True, kernel_options={"split_kv": False})
+    if D == 64 and Lkv == 33:
+        short = True   # two steps of 32 keys: the shorter one of the two at D = 64
+    assert (torch.equal(a, b) and torch.equal(la, lb)) != short
+    # up to 2048 terms in another order: a few units of 2^-24
+    assert rel_l2(a.cpu(), b.cpu()) <= 2e-6 and (la - lb).abs().max().item() <= 1e-5
+
+
 @pytest.mark.parametrize("gain", [0.5, 1.0, 3.0, 12.0])
 @pytest.mark.parametrize("D,cap", [(64, 50.0), (128, 50.0), (128, 7.0), (256, 20.0)])
 def test_softcap_against_64_bits(dev, D, cap, gain):

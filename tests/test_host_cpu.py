@@ -569,3 +569,19 @@ def test_a_call_is_told_what_it_uses_of_the_workspace(dtype, D):
             p.flags = _lib.FLAG_NO_SPLIT
             assert L.flexattn_bwd_workspace_needed(p) == L.flexattn_bwd_workspace_bytes(p) == delta
             assert L.flexattn_fwd_workspace_needed(p) == L.flexattn_fwd_workspace_bytes(p) == 0
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_float32_forward_divides_the_keys_where_tiles_are_even(D):
+    """Float32 forwards of 96 query tiles: under a causal mask the 32-row kernel takes them (no partial results), dense calls
+    and wide windows are split over the keys in two (half a wave of 32-row workgroups would run in a round of its own)."""
+    L = _lib.lib()
+    for hi, sink, lo, divided in ((2**31 - 1, -1, 0, False), (2**31 - 1, -1, -2**31, True), (1000, -1, 0, True), (1000, 3, 0, True),
+                                  (64, -1, 0, False)):
+        p = _lib.FlexAttnParams()
+        p.dtype, p.B, p.Hq, p.Hkv, p.Lq, p.Lkv, p.D, p.Dv = _lib.FLEX_F32, 1, 3, 3, 4096, 4096, D, D
+        for name in ("q_stride", "k_stride", "v_stride", "o_stride"):
+            getattr(p, name)[:] = [3 * 4096 * D, 4096 * D, D]
+        p.mask.lo, p.mask.hi, p.mask.sink = lo, hi, sink
+        want = (3 * 4096 * 2 * (D + 2) * 4 + 255) // 256 * 256 if divided else 0
+        assert L.flexattn_fwd_workspace_needed(p) == want, (lo, hi, sink)
