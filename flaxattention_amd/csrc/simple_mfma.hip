@@ -74,7 +74,8 @@ static int splits_over_keys(const FlexAttnParams& p) {
 // More tiles than that only where they are uneven (causal, the heaviest twice the mean) and the mean chain they are cut to
 // outweighs four times the workgroups: 192 tiles [8,8,384] 38 / 30 and 63 / 53, 256 tiles [4,8,1024] 92 / 73 and 157 / 133, [8,8,512]
 // 49 / 46 and 82 / 81, but 240 tiles [1,80,384] 39 / 39 and 64 / 68.  A window's tiles are even: 256 tiles [1,8,4096] window
-// 1000 106 / 130 and 180 / 236, four sinks and window 100 35 / 52 and 55 / 86.
+// 1000 106 / 130 and 180 / 236, four sinks and window 100 35 / 52 and 55 / 86; 192 tiles [1,12,2048] window 300 47 / 43 and
+// 76 / 72, window 64 24 / 22 and 38 / 34, sinks and window 100 34 / 37 and 54 / 60.
 // Against the split over workgroups above, by their chains: causal 32 tiles [1,4,1024] 52 / 33, 128 tiles [2,8,1024] 60 / 39 and
 // 91 / 68; but 96 tiles [1,6,2048 against 33 keys] at D = 128 17.5 / 20.5; dense 96 tiles [1,6,2048] 97 / 115 and 163 / 221, three packed documents there 53 / 38 and 81 / 64 (as a bitmap, which
 // counts as dense); window 64, 96 tiles [1,3,4096] 23 / 18 and 32 / 24, window 300 35 / 31 and 50 / 52, window 1000 65 / 70 and
@@ -86,19 +87,22 @@ static bool short_rows(const FlexAttnParams& p) {
   const bool window = p.mask.kind == FLEX_MASK_BAND && p.mask.hi != INT32_MAX;
   const bool causal = p.mask.kind == FLEX_MASK_BAND && p.mask.lo != INT32_MIN && p.Lq > p.Lkv / 2;
   const double fill = (double)wgs / cus;
-  if (wgs > cus / 2) return causal && !window && wgs <= cus && steps >= 12 && steps * (1 - 0.5 * fill) > 7.5 * fill;
+  if (causal && !window && wgs > cus / 2) return wgs <= cus && steps >= 12 && steps * (1 - 0.5 * fill) > 7.5 * fill;
   if (causal && !window && splits > 1) return 1.1 * fmax(1, 2 * fill) * steps / 4 <= (double)steps / splits;
   // even tiles, and calls of so few keys that the split above leaves them whole: the steps a 128-row tile lists (a bitmap may
   // list all of them) against the visits of a wave of 32 rows, in as many rounds as four times the workgroups take; a visit
   // costs more than a step of the tile does
+  const double visit = p.D == 64 ? 1.25 : 1.4;
   double listed = steps, mine = steps;
-  if (window && splits > 1) {
+  if (window && (splits > 1 || wgs > cus / 2)) {
     const double width = p.mask.lo == INT32_MIN ? p.Lkv : fmin(p.Lkv, (double)p.mask.hi - p.mask.lo);
     const bool sinks = p.mask.sink >= 0;
     listed = fmin(steps, (width + 128) / 32 + 1 + 2 * sinks);
     mine = fmin(steps, (width + 32) / 32 + 1 + sinks);
   }
-  return ceil(4 * fill) * ceil(mine / 4) * (p.D == 64 ? 1.25 : 1.4) <= listed / splits + 0.5;
+  if (wgs > cus / 2)   // (a wave's share of a window with sinks is uneven: the sinks' step comes on top of it)
+    return causal && fill <= 0.75 && p.mask.sink < 0 && ceil(4 * fill) * (ceil(mine / 4) * visit + 0.65) <= listed;
+  return ceil(4 * fill) * ceil(mine / 4) * visit <= listed / splits + 0.5;
 }
 // any_mask: the most any mask gets (a workspace is sized by the shape alone)
 int flex_simple_fwd_splits(const FlexAttnParams& p, bool any_mask) {
