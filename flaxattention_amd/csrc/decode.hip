@@ -80,15 +80,16 @@ size_t flex_decode_workspace(const FlexAttnParams& p, int splits) {
 // K: at most half of that (columns <= D / 4).  Cold KV caches, bf16, us with K read twice / scores kept:
 //   [16,8,6016,128]  1 column 104.5 / 81.9, 4: 104.8 / 85.9, 8: 104.9 / 90.0, 16: 105.8 / 98.2, 32: 106.5 / 105.9
 //   [1,8,32768,128]  1 column 48.9 / 43.1, 32: 49.8 / 48.1;   [16,8,6016,256]  1 column 207 / 149, 32: 213 / 189
-//   [64,8,8192,64]   1 column 274 / 202, 8: 275 / 238, 16: 279 / 263 -- two workgroups per compute unit, but with one
-//   [16,8,6016,64]   1 column 58.4 / 63.2, 16: 58.5 / 66.3;   [32,8,8192,64]  143 / 145, 16 columns 143 / 158
+//   [64,8,8192,64]   1 column 274 / 202, 8: 275 / 238, 16: 279 / 263;   [17,8,6016,64]  71.6 / 65.7, 72.0 / 69.9, 72.2 / 73.5
+// -- calls in which compute units have a second workgroup; with at most one each
+//   [16,8,6016,64]   1 column 58.8 / 63.0, 16: 59.0 / 66.1;   [32,8,2048,64] 1 column 44.9 / 47.8
 // At D = 64 a step of one operand is 4 KB a wave, and one workgroup per compute unit has too few of them in flight.
 // The room is bounded, so that a cache that nearly fills the card still fits: beyond kMaxKeptBytes K is read twice.
 constexpr size_t kMaxKeptBytes = (size_t)256 << 20;
 size_t flex_decode_kept_bytes(const FlexAttnParams& p, int splits) {
   const int64_t ncols = (int64_t)(p.Hq / p.Hkv) * p.Lq, heads = (int64_t)p.B * p.Hkv;
   if (!(p.flags & FLEX_PARITY) || ncols > p.D / 4 || ncols > 32) return 0;
-  if (p.D == 64 && heads * splits < 2 * flex_cu_count()) return 0;
+  if (p.D == 64 && heads * splits <= flex_cu_count()) return 0;
   const size_t bytes = (size_t)heads * ((p.Lkv + kStep - 1) / kStep) * ncols * kStep * 2;
   return bytes <= kMaxKeptBytes ? bytes : 0;
 }
