@@ -779,10 +779,11 @@ __global__ __launch_bounds__(256) void simple_dkv_kernel(FlexAttnParams p, const
   }
 
   const float out_scale = PARITY ? 1.f : p.scale;
-  // (a divided call always has its room; behind a test of it instead of a plain return, the compiler gives the kernel without
-  // a score_mod in the fast numerics 19 spilled registers at D = 256 and not 27: f16 [2,8,2048,256] causal, forward + backward,
-  // 441 -> 429 us.  The other functors spill less without the test.)
-  if (SPLIT && (PARITY || KIND != FLEX_SCORE_IDENTITY || partial)) {
+  // (a divided call always has its room; behind a test of it instead of a plain return, the compiler's allocation for the
+  // kernels without a score_mod is the faster one at D = 256: f16 [2,8,2048,256] causal, forward + backward, 441 -> 429 us, bf16
+  // [1,16->4,4096,256] causal 1437 -> 1414, dense 2419 -> 2365.  The other functors are faster without the test: f16 soft-cap
+  // 485 -> 480, bf16 checkerboard 612 -> 604.)
+  if (SPLIT && (KIND != FLEX_SCORE_IDENTITY || partial)) {
     store_dkv_part<DB>(partial, ((int64_t)part * p.B * p.Hkv + bh) * nkt + kt, w, lane, dkacc, dvacc, out_scale);
     return;
   }
