@@ -465,6 +465,14 @@ template <typename T> __device__ __forceinline__ void round_pair(float& a, float
   a = (float)h[0];
   b = (float)h[1];
 }
+// bfloat16: one conversion per value, packed with a zero below it, IS the rounded value as fp32 (a bfloat16 is the high
+// half of an fp32).  A packed conversion of the pair has to be taken apart again by a shift and an AND; a conversion or a
+// shift keeps the SIMD for four cycles, an AND for two, so that a pair costs 8 cycles instead of 10.  bf16 [8,8,2048,64]
+// ALiBi causal forward + backward 337.6 -> 325.0 us, [1,32->8,4096,128] causal 995 -> 981 us.
+template <> __device__ __forceinline__ void round_pair<bf16>(float& a, float& b) {
+  a = __uint_as_float(__builtin_bit_cast(unsigned, round_pack<bf16>(0.f, a)));
+  b = __uint_as_float(__builtin_bit_cast(unsigned, round_pack<bf16>(0.f, b)));
+}
 // three-input max without the NaN-quieting canonicalisation the compiler adds to fmaxf
 __device__ __forceinline__ float max3(float a, float b, float c) {
   float r;
