@@ -112,6 +112,10 @@ __global__ __launch_bounds__(256, ((D == 128 && MODE == kBwdFast) || D >= 192) ?
   float drow = 0.f;  // kBwdDelta: this lane's share of sum_j P_ij round(dP_ij)
   float lse = lse2[row_id];
   if (lse == -INFINITY) lse = INFINITY;  // row without visible keys: P = 0
+  // The parity numerics scale dS = P o (dP - delta) before it is rounded.  The factor's magnitude joins the exponent of P,
+  // its sign the result: as a product of its own, with a scalar operand (4 cycles instead of 2), it was 64 of 500 vector
+  // cycles per 32x32 block.
+  if constexpr (MODE == kBwdParity) lse -= log2f(fabsf(p.scale));
 
   const FlexTileLists& tl = p.tiles_bwd;
   const int32_t* full_idx = nullptr;
@@ -300,8 +304,6 @@ __global__ __launch_bounds__(256, ((D == 128 && MODE == kBwdFast) || D >= 192) ?
             d0 = fast_exp2(sacc[r]) * (a0 - delta);
             d1 = fast_exp2(sacc[r + 1]) * (a1 - delta);
             if (!Score2<KIND>::kGradOne) { d0 *= gacc[r]; d1 *= gacc[r + 1]; }
-            d0 *= p.scale;  // before dS is rounded, as the dense path has it
-            d1 *= p.scale;
           } else {
             d0 = fast_exp2(sacc[r]) * dpacc[r];
             d1 = fast_exp2(sacc[r + 1]) * dpacc[r + 1];
@@ -342,7 +344,7 @@ __global__ __launch_bounds__(256, ((D == 128 && MODE == kBwdFast) || D >= 192) ?
     return;
   }
   // fast numerics: the scale factor of dS = P o (dP - delta) o g * scale is applied once here
-  const float out_scale = MODE == kBwdParity ? 1.f : p.scale;
+  const float out_scale = MODE == kBwdParity ? (p.scale < 0.f ? -1.f : 1.f) : p.scale;
   if (q_row < p.Lq) {
     T* op = dq + row_id * D + 4 * g;
 #pragma unroll
@@ -445,6 +447,9 @@ __global__ __launch_bounds__(DkvShape<D>::kThreads, D == 64 ? 2 : 1) void bwd_dk
 
   const FlexTileLists& tl = p.tiles_bwd;
   Score2<KIND> sm;
+  // parity numerics: dS = P o (scale * dP - scale * delta), one fused multiply-add per entry.  In a vector register where
+  // one is to spare: an operand from a scalar register makes it 4 cycles instead of 2.
+  const float scale = D == 64 ? p.scale : vector_value(p.scale);
   float key_grad = 1.f;  // derivative of a score_mod that depends on the key only: applied to dK at the end
 
   for (int gi = SPLIT ? part % parts_g : 0; gi < G; gi += SPLIT ? parts_g : 1) {
@@ -516,7 +521,7 @@ __global__ __launch_bounds__(DkvShape<D>::kThreads, D == 64 ? 2 : 1) void bwd_dk
       float* lw = reinterpret_cast<float*>(Ow + BM * ROWE);
       if (tid < BM) {
         lw[tid] = lreg;        // rows past Lq carry lse = +inf: P = 0, whatever the clamped loads hold
-        lw[BM + tid] = -dreg;  // the dP accumulator starts from -delta
+        lw[BM + tid] = PARITY ? -dreg * p.scale : -dreg;  // the dP accumulator starts from -delta; parity: the scaled delta
       }
     };
     __syncthreads();  // the stages may still be in use by the previous head of the group
@@ -565,7 +570,7 @@ __global__ __launch_bounds__(DkvShape<D>::kThreads, D == 64 ? 2 : 1) void bwd_dk
       float16_t sacc, dpacc;
       const int ql = qrow_w + 4 * g;  // local row of register 0
       sm.tileT(q0 + ql, kv_col);      // a table-reading score_mod fetches its entries under the products
-      float16_t ndel;  // -delta of the block's rows (parity numerics: subtracted after dP is rounded)
+      float16_t ndel;  // -delta * scale of the block's rows (parity numerics: joins dP * scale after dP is rounded)
 #pragma unroll
       for (int rr = 0; rr < 4; rr++) {
         const float4_t d4 = *reinterpret_cast<const float4_t*>(del_s + ql + 8 * rr);
@@ -633,14 +638,13 @@ __global__ __launch_bounds__(DkvShape<D>::kThreads, D == 64 ? 2 : 1) void bwd_dk
           if constexpr (PARITY) {
             float a0 = dpacc[r], a1 = dpacc[r + 1];
             round_pair<T>(a0, a1);
-            d0 = p0 * (a0 + ndel[r]);
-            d1 = p1 * (a1 + ndel[r + 1]);
+            d0 = p0 * fmaf(a0, scale, ndel[r]);
+            d1 = p1 * fmaf(a1, scale, ndel[r + 1]);
           } else {
             d0 = p0 * dpacc[r];
             d1 = p1 * dpacc[r + 1];
           }
           if (!Score2<KIND>::kGradOne) { d0 *= gacc[r]; d1 *= gacc[r + 1]; }
-          if constexpr (PARITY) { d0 *= p.scale; d1 *= p.scale; }
           if constexpr (HILO) {
             split_pack<T>(p0, p1, pp[e], pl[e]);
             split_pack<T>(d0, d1, dd[e], dl[e]);
