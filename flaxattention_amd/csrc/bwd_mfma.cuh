@@ -77,7 +77,7 @@ __global__ __launch_bounds__(256, ((D == 128 && MODE == kBwdFast) || D >= 192) ?
   const int i32 = lane & 31, g = lane >> 5, i16 = lane & 15;
   const int nqt = (p.Lq + BM - 1) / BM;
   int rank, bh;
-  xcd_tile_map(blockIdx.x, nqt, p.Hq * p.B, rank, bh);
+  xcd_tile_map<((D == 128 && MODE == kBwdFast) || D >= 192) ? 1 : 2>(blockIdx.x, nqt, p.Hq * p.B, rank, bh);
   const int qt = nqt - 1 - rank;
   const int h = bh % p.Hq, b = bh / p.Hq, hk = h / (p.Hq / p.Hkv);
   const int q_row = qt * BM + w * 32 + i32;
@@ -409,7 +409,7 @@ __global__ __launch_bounds__(DkvShape<D>::kThreads, D == 64 ? 2 : 1) void bwd_dk
   int kt, bh;  // early key tiles see the most queries under causal masks
   int wid = blockIdx.x, part = 0;
   if constexpr (SPLIT) dkv_part_map(p.Hkv * p.B, parts_g * parts_t, wid, part);
-  xcd_tile_map(wid, nkt, p.Hkv * p.B, kt, bh);
+  xcd_tile_map<(D == 64 && !SPLIT) ? 2 : 1>(wid, nkt, p.Hkv * p.B, kt, bh);
   const int hk = bh % p.Hkv, b = bh / p.Hkv, G = p.Hq / p.Hkv;
   const int kv_col = kt * BN + wk * 32 + i32;
   const int kv_ld = min(kv_col, p.Lkv - 1);

@@ -77,7 +77,7 @@ __global__ __launch_bounds__(256, D >= 192 ? 1 : 2) void fwd_mfma_kernel(FlexAtt
   const int i32 = lane & 31, g = lane >> 5, i16 = lane & 15;
   const int nqt = (p.Lq + BM - 1) / BM;
   int rank, bh;
-  xcd_tile_map(blockIdx.x, nqt, p.Hq * p.B, rank, bh);
+  xcd_tile_map<D >= 192 ? 1 : PASS == kFwdLse ? 4 : D == 64 ? 3 : 2>(blockIdx.x, nqt, p.Hq * p.B, rank, bh);
   const int qt = nqt - 1 - rank;  // late query tiles see the most keys under causal masks
   const int h = bh % p.Hq, b = bh / p.Hq, hk = h / (p.Hq / p.Hkv);
 
@@ -489,7 +489,7 @@ __global__ __launch_bounds__(256, 2) void fwd_pipe_kernel(FlexAttnParams p, cons
   const int i32 = lane & 31, g = lane >> 5, i16 = lane & 15;
   const int nqt = (p.Lq + BM - 1) / BM;
   int rank, bh;
-  xcd_tile_map(blockIdx.x, nqt, p.Hq * p.B, rank, bh);
+  xcd_tile_map<1>(blockIdx.x, nqt, p.Hq * p.B, rank, bh);
   const int qt = nqt - 1 - rank;
   const int h = bh % p.Hq, b = bh / p.Hq, hk = h / (p.Hq / p.Hkv);
   const int q_row0 = qt * BM + w * (32 * RQ) + i32;

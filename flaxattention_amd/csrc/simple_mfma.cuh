@@ -229,7 +229,7 @@ __global__ __launch_bounds__(256) void simple_fwd_kernel(FlexAttnParams p, const
   const int i32 = lane & 31, g = lane >> 5;
   const int nqt = (p.Lq + kSimpleQTile - 1) / kSimpleQTile;
   int rank, bh;
-  xcd_tile_map(blockIdx.x, nqt, p.Hq * p.B, rank, bh);
+  xcd_tile_map<1>(blockIdx.x, nqt, p.Hq * p.B, rank, bh);
   const int qt = nqt - 1 - rank;  // late query tiles see the most keys under causal masks
   const int h = bh % p.Hq, b = bh / p.Hq, hk = h / (p.Hq / p.Hkv);
   const int q_row = qt * kSimpleQTile + w * 32 + i32;
@@ -383,7 +383,7 @@ __global__ __launch_bounds__(256) void simple_fwd_short_kernel(FlexAttnParams p,
   const int i32 = lane & 31, g = lane >> 5;
   const int nqt = (p.Lq + 31) / 32;
   int rank, bh;
-  xcd_tile_map(blockIdx.x, nqt, p.Hq * p.B, rank, bh);
+  xcd_tile_map<1>(blockIdx.x, nqt, p.Hq * p.B, rank, bh);
   const int qt = nqt - 1 - rank;  // late query rows see the most keys under causal masks
   const int h = bh % p.Hq, b = bh / p.Hq, hk = h / (p.Hq / p.Hkv);
   const int q_row = qt * 32 + i32;
@@ -527,7 +527,7 @@ __global__ __launch_bounds__(256) void simple_dq_kernel(FlexAttnParams p, const 
   const int i32 = lane & 31, g = lane >> 5;
   const int nqt = (p.Lq + kSimpleQTile - 1) / kSimpleQTile;
   int rank, bh;
-  xcd_tile_map(blockIdx.x, nqt, p.Hq * p.B, rank, bh);
+  xcd_tile_map<1>(blockIdx.x, nqt, p.Hq * p.B, rank, bh);
   const int qt = nqt - 1 - rank;
   const int h = bh % p.Hq, b = bh / p.Hq, hk = h / (p.Hq / p.Hkv);
   const int q_row = qt * kSimpleQTile + w * 32 + i32;
@@ -666,7 +666,7 @@ __global__ __launch_bounds__(256) void simple_dkv_kernel(FlexAttnParams p, const
   int kt, bh;  // early key tiles see the most queries under causal masks
   int wid = blockIdx.x, part = 0;
   if constexpr (SPLIT) dkv_part_map(p.Hkv * p.B, parts_g * parts_t, wid, part);
-  xcd_tile_map(wid, nkt, p.Hkv * p.B, kt, bh);
+  xcd_tile_map<1>(wid, nkt, p.Hkv * p.B, kt, bh);
   const int hk = bh % p.Hkv, b = bh / p.Hkv, G = p.Hq / p.Hkv;
   const int kv_col = kt * kSimpleKvTile + w * 32 + i32;
   const int kv_ld = min(kv_col, p.Lkv - 1);

@@ -1385,3 +1385,23 @@ def test_softcap_rows_do_not_depend_on_what_they_cannot_see(dev, dtype, numerics
     want = v.double().cumsum(2) / torch.arange(1, L + 1, device=dev, dtype=torch.float64).reshape(-1, 1)
     assert ((zero.double() - want).norm() / want.norm()).item() <= 1.5 * torch.finfo(dtype).eps
     assert (lse0[0, 0].double() - torch.arange(1, L + 1, device=dev, dtype=torch.float64).log()).abs().max().item() <= 1e-5
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("H,L", [(5, 13200), (8, 8200), (16, 4096)])
+def test_every_tile_is_visited_whatever_the_workgroup_order(dev, H, L, D):
+    """Workgroups of the second (fourth) round over the compute units run backwards through the tiles; a head by itself has too
+    few tiles for a second round.  The kernels are the same either way, so the results are, bit for bit."""
+    print("case workgroup order", H, L, D, flush=True)
+    q, k, v = (t.to(dev) for t in seeded_qkv(1, H, H, L, L, D, torch.bfloat16))
+    bm = fa.create_block_mask(generate_sliding_window(200), None, None, L, L, device=dev)
+    opts = {"split_kv": False}
+
+    def step(*qkv):
+        qkv = [t.detach().contiguous().requires_grad_(True) for t in qkv]
+        out = fa.flax_attention(*qkv, block_mask=bm, kernel_options=opts)
+        return (out, *torch.autograd.grad(out, qkv, torch.ones_like(out)))
+    whole = step(q, k, v)
+    for h in (0, H // 2, H - 1):
+        for a, b in zip(whole, step(*(t[:, h:h + 1] for t in (q, k, v)))):
+            assert torch.equal(a[:, h:h + 1], b)
