@@ -586,6 +586,20 @@ __device__ __forceinline__ void xcd_tile_map(int wid, int ntile, int nbh, int& r
   }
 }
 
+// N matrix steps with operands from LDS, each read AHEAD steps before its use.  Left alone the compiler reads an operand,
+// waits for it and uses it, one after the other, wherever registers are short -- with one wave per SIMD nothing covers
+// the 100 cycles of each read.  The fences keep its scheduler from undoing the order.
+template <int N, int AHEAD, typename Slot, typename Read, typename Use>
+__device__ __forceinline__ void read_ahead(Read read, Use use) {
+  Slot ring[AHEAD + 1];
+#pragma unroll
+  for (int s = 0; s < N + AHEAD; s++) {
+    if (s < N) read(s, ring[s % (AHEAD + 1)]);
+    __builtin_amdgcn_sched_barrier(0);
+    if (s >= AHEAD) use(s - AHEAD, ring[(s - AHEAD) % (AHEAD + 1)]);
+  }
+}
+
 // ---- dK/dV calls divided over the queries ----
 // `parts` workgroups share a tile of 128 keys (four waves of 32) and leave float32 partial sums of dK and dV.
 struct DkvParts { int g, t; };   // parts: over the query heads of the group, and over each head's list of query tiles
