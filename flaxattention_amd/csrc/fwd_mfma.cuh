@@ -51,8 +51,7 @@ __global__ __launch_bounds__(256, D >= 192 ? 1 : 2) void fwd_mfma_kernel(FlexAtt
                                                            float* __restrict__ o_part, float* __restrict__ ml_part) {
   // Split-KV: with gridDim.y > 1 workgroup (x, y) visits share y of its query tile's key tiles and leaves an
   // unnormalised partial (O, m, l) per row in o_part / ml_part, in the layout decode_combine_kernel merges (kFwdLse:
-  // only (m, l); kFwdNorm: the partial outputs add up, written with m = 0 and l = 1 for share 0, l = 0 for the
-  // others).  For calls whose query tiles alone would leave most compute units without a workgroup.
+  // only (m, l), which kFwdNorm merges for its rows; the partial outputs of kFwdNorm add up).  For calls whose query tiles alone would leave most compute units without a workgroup.
   typedef typename Frag<T>::vec8 vec8;
   typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
   constexpr int RQ = 1, BM = kFwdBM, BN = kFwdBN;
@@ -199,7 +198,33 @@ __global__ __launch_bounds__(256, D >= 192 ? 1 : 2) void fwd_mfma_kernel(FlexAtt
     if constexpr (PASS == kFwdNorm) {
       // the row's log-sum-exp from the first pass takes the place of the running reference maximum and never
       // moves; a row without visible keys (-inf) gets +inf, so that every P is 0
-      const float l2 = lse2[((int64_t)b * p.Hq + h) * p.Lq + min(q_row0 + 32 * a, p.Lq - 1)];
+      const int q_ld = min(q_row0 + 32 * a, p.Lq - 1);
+      const int64_t row = ((int64_t)b * p.Hq + h) * p.Lq + q_ld;
+      float l2;
+      if (nsplit == 1) {
+        l2 = lse2[row];
+      } else {
+        // the first pass left (m, l) of every share: every workgroup merges those of its own rows, the first share writes the
+        // result out (the merge in a launch of its own: bf16 [1,32->8,512 of 16384,128] 252.7 us, here 249.4)
+        const float2* ml = reinterpret_cast<const float2*>(ml_part) + row;
+        const int64_t rows = (int64_t)p.B * p.Hq * p.Lq;
+        float m = -INFINITY, l = 0.f;
+        for (int s0 = 0; s0 < nsplit; s0 += 4) {
+          float2 part[4];   // four shares' loads in flight together
+#pragma unroll
+          for (int u = 0; u < 4; u++) part[u] = ml[min(s0 + u, nsplit - 1) * rows];
+          float m_new = m;
+#pragma unroll
+          for (int u = 0; u < 4; u++) m_new = fmaxf(m_new, part[u].x);
+          if (m_new == -INFINITY) continue;
+          l *= fast_exp2(m - m_new);
+#pragma unroll
+          for (int u = 0; u < 4; u++) l += s0 + u < nsplit ? fast_exp2(part[u].x - m_new) * part[u].y : 0.f;
+          m = m_new;
+        }
+        l2 = l > 0.f ? m + log2f(l) : -INFINITY;
+        if (split == 0 && g == 0 && q_row0 + 32 * a < p.Lq) lse2[row] = l2;
+      }
       m_run[a] = l2 == -INFINITY ? INFINITY : l2;
     }
 #pragma unroll
@@ -420,9 +445,9 @@ __global__ __launch_bounds__(256, D >= 192 ? 1 : 2) void fwd_mfma_kernel(FlexAtt
       // partial result of this share; a row that saw nothing here must not hold the merge's reference up: m = -inf
       if (q_row < p.Lq) {
         const int64_t at = ((int64_t)split * p.B * p.Hq + (int64_t)b * p.Hq + h) * p.Lq + q_row;
-        if (g == 0) {
-          ml_part[at * 2] = PASS == kFwdNorm ? 0.f : (l_tot > 0.f ? m_run[a] : -INFINITY);
-          ml_part[at * 2 + 1] = PASS == kFwdNorm ? (split == 0 ? 1.f : 0.f) : l_tot;
+        if (PASS != kFwdNorm && g == 0) {
+          ml_part[at * 2] = l_tot > 0.f ? m_run[a] : -INFINITY;
+          ml_part[at * 2 + 1] = l_tot;
         }
         if constexpr (PASS != kFwdLse) {
           float* op = o_part + at * D + 4 * g;
@@ -825,18 +850,18 @@ struct FwdArgs {
   float *o_part, *ml_part;
 };
 
-// one pass of the list-driven kernel; over split key ranges it is followed by the merge of the partials (one wave per
-// row), which writes `o` (unless null) and `lse2` (unless null)
+// one pass of the list-driven kernel; over split key ranges it is followed by the merge of the partial outputs (one wave
+// per row)
 template <typename T, int D, int KIND, bool RS, bool BITS, int PASS>
 static void launch_list_kernel(const FlexAttnParams& p, const FwdArgs& a) {
   const int splits = a.splits > 1 ? a.splits : 1;
   dim3 grid((p.Lq + kFwdBM - 1) / kFwdBM * p.Hq * p.B, splits);
   hipLaunchKernelGGL((fwd_mfma_kernel<T, D, KIND, RS, BITS, PASS>), grid, dim3(256), 0, a.s, p, (const T*)a.q, (const T*)a.k,
                      (const T*)a.v, (T*)a.o, a.lse2, a.o_part, a.ml_part);
-  if (splits > 1) {
+  if (splits > 1 && PASS != kFwdLse) {   // (the second pass merges the log-sum-exps of the first itself)
     const int64_t rows = (int64_t)p.B * p.Hq * p.Lq;
-    hipLaunchKernelGGL((decode_combine_kernel<T, D>), dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, a.s, p, a.o_part, a.ml_part,
-                       splits, PASS == kFwdLse ? (T*)nullptr : (T*)a.o, PASS == kFwdNorm ? (float*)nullptr : a.lse2);
+    hipLaunchKernelGGL((decode_combine_kernel<T, D>), dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, a.s, p, a.o_part,
+                       PASS == kFwdNorm ? nullptr : a.ml_part, splits, (T*)a.o, PASS == kFwdNorm ? nullptr : a.lse2);
   }
 }
 
