@@ -234,3 +234,18 @@ def test_band_fit_of_packed_bitmaps(dev, Q, KV):
     assert same and torch.equal(dense(got), m)
     g = torch.Generator().manual_seed(Q)
     assert _fit_bitmaps(pack_bits(torch.rand(Q, KV, generator=g) < 0.5)[None].to(dev)) == (True, None)
+
+
+@pytest.mark.parametrize("bs", [32, 64, 128, (64, 96), (96, 32), (160, 128), (48, 80)], ids=str)
+@pytest.mark.parametrize("B,H,Q,KV", [(2, 1, 700, 700), (1, 3, 130, 1000), (2, 2, 33, 31)])
+def test_lists_of_bitmaps_at_any_block_size(dev, B, H, Q, KV, bs):
+    """Tiles made of whole 32 x 32 blocks are told by the blocks' classes, others by counting bits; empty, full and mixed tiles,
+    maps that differ by batch and head, lengths that end inside a tile."""
+    print("case bitmap lists", B, H, Q, KV, bs, flush=True)
+    gen = torch.Generator().manual_seed(Q + KV)
+    doc = torch.randint(0, 3, (B, H, 64), generator=gen).repeat_interleave(29, dim=2)   # 29 positions a piece
+
+    def mask(b, h, q, kv):
+        table = doc.to(q.device)   # (positions past the lengths are padding: a captured table is read at the last one there)
+        return table[b, h, q.clamp(max=Q - 1)] >= table[b, h, kv.clamp(max=KV - 1)]
+    check(fa.create_block_mask(mask, B, H, Q, KV, BLOCK_SIZE=bs, device=dev), ref_create_block_mask(mask, B, H, Q, KV, BLOCK_SIZE=bs))
