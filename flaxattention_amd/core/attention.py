@@ -65,7 +65,8 @@ import torch
 from .. import _lib
 from .blockmask import BlockMask, _create_empty_block_mask
 from .common import (IDENTITY, MaskMod, ScoreMod, ScoreModNotLowered, _identity, _mask_mod_signature,
-                     _score_mod_signature, resolve_mask_mod, resolve_score_mod)
+                     _score_mod_signature, resolve_mask_mod, resolve_score_mod,
+                     _on_device, _stream)
 
 Array = torch.Tensor
 
@@ -292,33 +293,6 @@ def _holder_for(mask: MaskMod) -> BlockMask:
                                      torch.zeros([1, 1, 1, 1], dtype=torch.int32, device=dev), mask_mod=mask)
         _holders[key] = h
     return h
-
-
-def _stream(t) -> int:
-    """Raw handle of torch's current stream on the tensor's device (the private accessor skips the Stream object
-    that torch.cuda.current_stream builds on every call)."""
-    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
-    if raw is not None:
-        return raw(t.device.index if t.device.index is not None else torch.cuda.current_device())
-    return torch.cuda.current_stream(t.device).cuda_stream
-
-
-class _on_device:
-    """torch.cuda.device(dev) only when dev is not already current (entering the context costs ~10 us of host time)."""
-    __slots__ = ("ctx",)
-
-    def __init__(self, dev):
-        idx = dev.index
-        self.ctx = None if idx is None or idx == torch.cuda.current_device() else torch.cuda.device(dev)
-
-    def __enter__(self):
-        if self.ctx is not None:
-            self.ctx.__enter__()
-
-    def __exit__(self, *exc):
-        if self.ctx is not None:
-            self.ctx.__exit__(*exc)
-        return False
 
 
 def _run_fwd(plan: _Plan, q, k, v) -> Tuple[Array, Array]:

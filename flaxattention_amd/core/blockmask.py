@@ -27,7 +27,7 @@ import torch
 
 from .. import _lib
 from .common import (INT_MAX, INT_MIN, MaskMod, _get_mod_type, _ModificationType, _mask_mod_signature,
-                     _score_mod_signature, band_and, band_or, dense_mask_on_device, resolve_mask_mod)
+                     _score_mod_signature, band_and, band_or, dense_mask_on_device, resolve_mask_mod, _on_device, _stream)
 
 Array = torch.Tensor
 
@@ -282,17 +282,15 @@ def build_lists(spec: MaskMod, B: int, H: int, nq: int, nkv: int, q_block: int, 
     )
     ws = torch.empty(L.flexattn_block_mask_workspace_bytes(B, H, nq, nkv), dtype=torch.uint8, device=device)
     m = spec.c_struct()
-    with torch.cuda.device(device):
-        stream = torch.cuda.current_stream(device).cuda_stream
+    with _on_device(ws.device):
         rc = L.flexattn_block_mask_build(
             m, B, H, nq, nkv, q_block, kv_block,
             out["kv_num_blocks"].data_ptr(), out["kv_indices"].data_ptr(),
             out["full_kv_num_blocks"].data_ptr(), out["full_kv_indices"].data_ptr(),
             out["q_num_blocks"].data_ptr(), out["q_indices"].data_ptr(),
             out["full_q_num_blocks"].data_ptr(), out["full_q_indices"].data_ptr(),
-            ws.data_ptr(), stream)
+            ws.data_ptr(), _stream(ws))
     _lib.check(rc, "flexattn_block_mask_build")
-    ws.record_stream(torch.cuda.current_stream(device))
     out.update(q_block=q_block, kv_block=kv_block, n_q_blocks=nq, n_kv_blocks=nkv, B=B, H=H, spec=spec)
     return out
 

@@ -23,6 +23,36 @@ import torch
 
 from .. import _lib
 
+
+def _stream(t) -> int:
+    """Raw handle of torch's current stream on the tensor's device (the private accessor skips the Stream object
+    that torch.cuda.current_stream builds on every call)."""
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is not None:
+        return raw(t.device.index if t.device.index is not None else torch.cuda.current_device())
+    return torch.cuda.current_stream(t.device).cuda_stream
+
+
+class _on_device:
+    """torch.cuda.device(dev) only when dev is not already current (entering the context costs ~10 us of host time)."""
+    __slots__ = ("ctx",)
+
+    def __init__(self, dev):
+        if dev.type != "cuda":
+            raise ValueError(f"Expected a cuda device, but got: {dev}")
+        idx = dev.index
+        self.ctx = None if idx is None or idx == torch.cuda.current_device() else torch.cuda.device(dev)
+
+    def __enter__(self):
+        if self.ctx is not None:
+            self.ctx.__enter__()
+
+    def __exit__(self, *exc):
+        if self.ctx is not None:
+            self.ctx.__exit__(*exc)
+        return False
+
+
 Array = torch.Tensor
 _score_mod_signature = Callable[[Array, Array, Array, Array, Array], Array]
 _mask_mod_signature = Callable[[Array, Array, Array, Array], Array]
@@ -380,10 +410,10 @@ def _tables_of_planes(fn: Callable, name: str, y: torch.Tensor, Lq: int) -> Opti
     add, mul = torch.empty_like(y[0]), torch.empty_like(y[0])
     diag = torch.empty((b, h, rows + Lkv - 1), dtype=torch.float32, device=y.device) if rows == Lq > 1 and Lkv > 1 else None
     flags = torch.zeros(4, dtype=torch.int32, device=y.device)
-    with torch.cuda.device(y.device):
+    with _on_device(y.device):
         rc = _lib.lib().flexattn_affine_tables(y.data_ptr(), b * h, rows, Lkv, add.data_ptr(), mul.data_ptr(),
                                                diag.data_ptr() if diag is not None else None, flags.data_ptr(),
-                                               torch.cuda.current_stream(y.device).cuda_stream)
+                                               _stream(y))
     _lib.check(rc, "flexattn_affine_tables")
     bad, adds, scales, bends = flags.tolist()
     if bad:
@@ -878,11 +908,11 @@ def _pack_slab(m: torch.Tensor, q0: int, at: int, bits: torch.Tensor, bits_t: Op
     nb, nh, rows, KVp = m.shape
     Qp = bits.shape[1]
     if m.is_cuda:
-        with torch.cuda.device(m.device):
+        with _on_device(m.device):
             rc = _lib.lib().flexattn_pack_mask(
                 m.data_ptr(), (ctypes.c_int64 * 4)(*m.stride()), nb, nh, q0, rows, Qp, KVp, bits[at].data_ptr(),
                 bits_t[at].data_ptr() if bits_t is not None else None, blk[at].data_ptr(),
-                torch.cuda.current_stream(m.device).cuda_stream)
+                _stream(m))
         _lib.check(rc, "flexattn_pack_mask")
         return
     m = m.reshape(nb * nh, rows, KVp)
@@ -897,9 +927,9 @@ def _fit_bitmaps(bits: torch.Tensor) -> Tuple[bool, Optional[MaskMod]]:
     n, Qp, W = bits.shape
     if bits.is_cuda:
         fit = torch.empty(6, dtype=torch.int32, device=bits.device)
-        with torch.cuda.device(bits.device):
+        with _on_device(bits.device):
             rc = _lib.lib().flexattn_bitmap_fit(bits.data_ptr(), n, Qp, W * 32, fit.data_ptr(),
-                                                torch.cuda.current_stream(bits.device).cuda_stream)
+                                                _stream(bits))
         _lib.check(rc, "flexattn_bitmap_fit")
         lo, differs, d, kv, bad_sink, bad_plain = fit.tolist()
         if differs:
