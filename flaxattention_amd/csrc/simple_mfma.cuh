@@ -108,7 +108,7 @@ template <typename T, int D> struct SimpleOps16 {
     return acc;
   }
   // (both products: operands two steps ahead.  dK/dV of f16 [2,8,2048,256] causal, in two parts with their merge, 158 -> 147 us,
-  // bf16 parity 215 -> 198, D = 192 109 -> 98)
+  // bf16 parity 215 -> 198, 179 with round_block's packed pairs, D = 192 109 -> 98)
   static __device__ __forceinline__ float16_t row_product(const T* tile, int i32, int g, const Resident& r, float16_t acc) {
     const T* row = tile + i32 * ROWE + 8 * g;
     read_ahead<D / 16, 2, vec8>(
@@ -140,7 +140,7 @@ template <typename T, int D> struct SimpleOps16 {
         [&](int j, const vec8& a) __attribute__((always_inline)) { acc[j % DB] = Frag<T>::mfma(a, b[j / DB], acc[j % DB]); });
   }
   // (pairs packed and taken apart again, not round_pair: with bfloat16's conversion of single values the undivided dK/dV kernel
-  // at D = 256 spills 49 registers instead of 41, the divided one 85 instead of 77: bf16 [2,8,2048,256] causal 198 -> 178 us)
+  // at D = 256 spills 49 registers instead of 41, the divided one 85 instead of 77: bf16 [2,8,2048,256] causal 198 -> 179 us)
   static __device__ __forceinline__ void round_block(float16_t& x) {
 #pragma unroll
     for (int r = 0; r < 16; r += 2) {
