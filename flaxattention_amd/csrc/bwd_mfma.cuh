@@ -224,6 +224,13 @@ __global__ __launch_bounds__(256, ((D == 128 && MODE == kBwdFast) || D >= 192) ?
   // fast numerics: dP starts at -delta, so the accumulator comes out as dP - delta; the parity numerics
   // round dP first
   const float neg_delta = (MODE == kBwdFast || MODE == kBwdHiLo) ? -delta : 0.f;
+  // The parity kernel at D = 128 spills: by packed pairs it keeps 16 .. 68 registers in scratch (identity .. tables), by
+  // bfloat16's conversion of single values up to 10 more: bf16 [2,8,2048,128] causal 90 us against 72, ALiBi 131 : 123
+  // (a checkerboard's kernel spills 18 and takes the same time either way)
+  auto round = [](float& a, float& b) __attribute__((always_inline)) {
+    if constexpr (D == 128 && MODE == kBwdParity) round_pair_packed<T>(a, b);
+    else round_pair<T>(a, b);
+  };
   // one tile out of the stage named by `stage` (= it & 1)
   auto tile_step = [&](auto stage, int it) {
     constexpr int ST = decltype(stage)::value;
@@ -281,7 +288,7 @@ __global__ __launch_bounds__(256, ((D == 128 && MODE == kBwdFast) || D >= 192) ?
 #pragma unroll
       for (int r = 0; r < 16; r += 2) {
         float s0 = sacc[r], s1 = sacc[r + 1];
-        if (ROUND_S) round_pair<T>(s0, s1);
+        if (ROUND_S) round(s0, s1);
         sacc[r] = sm.apply_sub(s0, acc_row(r), lse);
         sacc[r + 1] = sm.apply_sub(s1, acc_row(r + 1), lse);
         if (!Score2<KIND>::kGradOne) {
@@ -316,7 +323,7 @@ __global__ __launch_bounds__(256, ((D == 128 && MODE == kBwdFast) || D >= 192) ?
           float d0, d1;
           if constexpr (MODE == kBwdParity) {
             float a0 = dpacc[r], a1 = dpacc[r + 1];
-            round_pair<T>(a0, a1);
+            round(a0, a1);
             d0 = fast_exp2(sacc[r]) * (a0 - delta);
             d1 = fast_exp2(sacc[r + 1]) * (a1 - delta);
             if (!Score2<KIND>::kGradOne) { d0 *= gacc[r]; d1 *= gacc[r + 1]; }

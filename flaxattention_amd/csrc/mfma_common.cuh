@@ -468,15 +468,18 @@ __device__ __forceinline__ void split_pack(float a, float b, typename Pair<T>::v
   hi = round_pack<T>(a, b);
   lo = Pair<T>::pack(a - (float)hi[0], b - (float)hi[1]);
 }
-template <typename T> __device__ __forceinline__ void round_pair(float& a, float& b) {
+// Two values rounded through T by one packed conversion.
+template <typename T> __device__ __forceinline__ void round_pair_packed(float& a, float& b) {
   typename Pair<T>::v2 h = round_pack<T>(a, b);
   a = (float)h[0];
   b = (float)h[1];
 }
+template <typename T> __device__ __forceinline__ void round_pair(float& a, float& b) { round_pair_packed<T>(a, b); }
 // bfloat16: one conversion per value, packed with a zero below it, IS the rounded value as fp32 (a bfloat16 is the high
 // half of an fp32).  A packed conversion of the pair has to be taken apart again by a shift and an AND; a conversion or a
 // shift keeps the SIMD for four cycles, an AND for two, so that a pair costs 8 cycles instead of 10.  bf16 [8,8,2048,64]
-// ALiBi causal forward + backward 337.6 -> 325.0 us, [1,32->8,4096,128] causal 995 -> 981 us.
+// ALiBi causal forward + backward 337.6 -> 325.0 us, [1,32->8,4096,128] causal 995 -> 981 us.  Not for kernels that spill: the
+// two values live longer than the packed one (same bits either way; those take round_pair_packed).
 template <> __device__ __forceinline__ void round_pair<bf16>(float& a, float& b) {
   a = __uint_as_float(__builtin_bit_cast(unsigned, round_pack<bf16>(0.f, a)));
   b = __uint_as_float(__builtin_bit_cast(unsigned, round_pack<bf16>(0.f, b)));

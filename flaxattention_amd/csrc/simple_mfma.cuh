@@ -139,14 +139,15 @@ template <typename T, int D> struct SimpleOps16 {
         },
         [&](int j, const vec8& a) __attribute__((always_inline)) { acc[j % DB] = Frag<T>::mfma(a, b[j / DB], acc[j % DB]); });
   }
-  // (pairs packed and taken apart again, not round_pair: with bfloat16's conversion of single values the undivided dK/dV kernel
-  // at D = 256 spills 49 registers instead of 41, the divided one 85 instead of 77: bf16 [2,8,2048,256] causal 198 -> 179 us)
+  // (by packed pairs: with bfloat16's conversion of single values the undivided dK/dV kernel at D = 256 spills 49 registers
+  // instead of 41, the divided one 85 instead of 77: bf16 [2,8,2048,256] causal 198 -> 179 us)
   static __device__ __forceinline__ void round_block(float16_t& x) {
 #pragma unroll
     for (int r = 0; r < 16; r += 2) {
-      const typename Pair<T>::v2 h = round_pack<T>(x[r], x[r + 1]);
-      x[r] = (float)h[0];
-      x[r + 1] = (float)h[1];
+      float a = x[r], b = x[r + 1];
+      round_pair_packed<T>(a, b);
+      x[r] = a;
+      x[r + 1] = b;
     }
   }
   static __device__ __forceinline__ void store4(T* p, float a, float b, float c, float d) {

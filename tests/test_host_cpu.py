@@ -506,10 +506,8 @@ def test_kept_scores_of_a_parity_decode_are_bounded(D):
             assert kept == (room if want else 0), (B, Hkv, G, Lq, Lkv, splits, kept)
 
 
-def test_undivided_wide_backward_keeps_its_registers():
-    """The simple dK/dV kernel at D = 256 fills a wave's registers, and what does not fit is spilled next to its tile loop.
-    The form that is not divided over the queries carries nothing of the division: the spills of the built kernels, read
-    from the library's own kernel descriptions, stay at what the undivided kernel needs with the image's compiler."""
+def _built_kernels():
+    """The kernel descriptions of the built library, by name."""
     import struct
     msgpack = pytest.importorskip("msgpack")
     with open(_lib.LIB_PATH, "rb") as f:
@@ -531,6 +529,14 @@ def test_undivided_wide_backward_keeps_its_registers():
                     start += 12 + (name + 3) // 4 * 4
                     kernels.update({k[".name"]: k for k in msgpack.unpackb(elf[start:start + desc])["amdhsa.kernels"]})
         pos += len(magic)
+    return kernels
+
+
+def test_undivided_wide_backward_keeps_its_registers():
+    """The simple dK/dV kernel at D = 256 fills a wave's registers, and what does not fit is spilled next to its tile loop.
+    The form that is not divided over the queries carries nothing of the division: the spills of the built kernels, read
+    from the library's own kernel descriptions, stay at what the undivided kernel needs with the image's compiler."""
+    kernels = _built_kernels()
     # by functor (identity, checkerboard, ALiBi, soft-cap, relative bias, additive and multiplicative tables)
     most = {"parity": dict(zip((0, 1, 2, 3, 4, 5, 102), (48, 48, 48, 64, 48, 72, 82))),
             "fast": dict(zip((0, 1, 2, 3, 4, 5, 102), (32, 32, 32, 42, 32, 47, 52)))}
@@ -540,6 +546,19 @@ def test_undivided_wide_backward_keeps_its_registers():
                 found = [k for n, k in kernels.items() if f"simple_dkv_kernelI{dtype}Li256ELi{kind}ELb{b}ELb0E" in n]
                 assert len(found) == 1, (dtype, kind, numerics)
                 assert found[0][".vgpr_spill_count"] <= bound, (dtype, kind, numerics, found[0][".vgpr_spill_count"])
+
+
+@pytest.mark.parametrize("dtype", ["DF16_", "DF16b"], ids=["f16", "bf16"])
+def test_narrow_dq_kernels_keep_their_registers(dtype):
+    """The dQ kernel of the parity numerics at D = 128 spills as it is; how it rounds and orders its products must not add to that
+    (the conversion of single bfloat16 values took 10 registers more, and up to a fifth of the kernel's time)."""
+    kernels = _built_kernels()
+    most = {2: dict(zip((0, 1, 2, 3, 4, 5, 102), (16, 18, 42, 48, 42, 52, 68)))}   # by mode, then by functor
+    for mode, bounds in most.items():
+        for kind, bound in bounds.items():
+            found = [k for n, k in kernels.items() if f"bwd_dq_kernelI{dtype}Li128ELi{kind}ELb{int(mode == 2)}ELb1ELi{mode}E" in n]
+            assert len(found) == 1, (kind, mode)
+            assert found[0][".vgpr_spill_count"] <= bound + 4, (kind, mode, found[0][".vgpr_spill_count"])
 
 
 @pytest.mark.parametrize("dtype,D", [(_lib.FLEX_F16, 64), (_lib.FLEX_BF16, 128), (_lib.FLEX_F16, 256), (_lib.FLEX_F32, 64), (_lib.FLEX_F32, 128)])
