@@ -77,7 +77,9 @@ __global__ __launch_bounds__(256, ((D == 128 && MODE == kBwdFast) || D >= 192) ?
   const int i32 = lane & 31, g = lane >> 5, i16 = lane & 15;
   const int nqt = (p.Lq + BM - 1) / BM;
   int rank, bh;
-  xcd_tile_map<((D == 128 && MODE == kBwdFast) || D >= 192) ? 1 : 2>(blockIdx.x, nqt, p.Hq * p.B, rank, bh);
+  // (one workgroup has the compute unit in the fast kernel at D = 128 and in the wide ones; the unrounded dQ at D = 128 is
+  // slower with its second round turned: [8,8,2048,128] causal 174 against 172 us, ALiBi 194 : 190, f16 soft-cap 227 : 223)
+  xcd_tile_map<(D == 128 && (MODE == kBwdFast || MODE == kBwdHiLo)) || D >= 192 ? 1 : 2>(blockIdx.x, nqt, p.Hq * p.B, rank, bh);
   const int qt = nqt - 1 - rank;
   const int h = bh % p.Hq, b = bh / p.Hq, hk = h / (p.Hq / p.Hkv);
   const int q_row = qt * BM + w * 32 + i32;

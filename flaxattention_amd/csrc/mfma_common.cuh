@@ -561,29 +561,30 @@ template <int D> __device__ __forceinline__ constexpr int lds_swz(int r) {
 // under causal-like masks the long workgroups start first and the short ones fill
 // the tail.  `rank` counts tiles from the heaviest (0) to the lightest (ntile-1).
 //
-// RESIDENT: workgroups of the kernel that a compute unit holds at once.  An XCD fills its 32 compute units round by
-// round, so with heavy-first ids a compute unit that starts with the heaviest tile of the first round also gets the
-// heaviest of the second.  The odd ones of the first RESIDENT rounds run backwards instead: every compute unit starts
-// with the same amount of work, and the later rounds, dealt as workgroups end, no longer have to make up for it (the first
-// of two workgroups on a compute unit runs 1.5 times as fast as the second, so they did not: with 2 x 2 workgroups of a
-// causal problem the sums came out 32 .. 36 tiles where 34 is the mean).  Causal, bf16 [8,8,2048,64] log-sum-exp pass
-// 42.5 -> 41.0 us, row sweep 61.4 -> 58.7, dQ 77 -> 74.5; [1,32->8,4096,128] log-sum-exp 98 -> 95, second pass 150 -> 147,
-// row sweep 152 -> 149.  A mask that gives every tile the same work is not affected.
-template <int RESIDENT>
+// ROUNDS: an XCD fills its 32 compute units round by round, so with heavy-first ids a compute unit that starts with the
+// heaviest tile of the first round also gets the heaviest of the second.  Of the first ROUNDS rounds the odd ones run
+// backwards instead (1: none does, 2: the second, 4: the second and the fourth): every compute unit starts with the same
+// amount of work, and the later rounds, dealt as workgroups end, no longer have to make up for it (the first of two
+// workgroups on a compute unit runs 1.5 times as fast as the second, so they did not: with 2 x 2 workgroups of a causal
+// problem the sums came out 32 .. 36 tiles where 34 is the mean).  Causal, bf16 [8,8,2048,64] log-sum-exp pass 42.5 -> 41.0 us,
+// row sweep 61.4 -> 58.7, dQ 77 -> 74.5; [1,32->8,4096,128] log-sum-exp 98 -> 95, second pass 150 -> 147, row sweep 152 -> 149.
+// Each kernel takes the number that was the fastest of those tried on it, at most the workgroups that a compute unit holds
+// of it; two kernels of the unrounded numerics are faster without (at their callers).  A mask that gives every tile the
+// same work is not affected.
+template <int ROUNDS>
 __device__ __forceinline__ void xcd_tile_map(int wid, int ntile, int nbh, int& rank, int& bh) {
   constexpr int kXcd = 8, kCus = 32;
-  const int xcd = wid % kXcd;
-  int local = wid / kXcd;
-  if constexpr (RESIDENT > 1) {
-    const int round = local / kCus;
-    if (round < RESIDENT && (round & 1) && (round + 1) * kCus * kXcd <= ntile * nbh) local = (2 * round + 1) * kCus - 1 - local;
+  if constexpr (ROUNDS > 1) {
+    const int xcd = wid % kXcd, local = wid / kXcd, round = local / kCus;
+    if (round < ROUNDS && (round & 1) && (round + 1) * kCus * kXcd <= ntile * nbh)
+      wid = ((2 * round + 1) * kCus - 1 - local) * kXcd + xcd;
   }
   if (nbh % kXcd == 0) {
     const int per = nbh / kXcd;           // heads per XCD
+    const int xcd = wid % kXcd, local = wid / kXcd;
     rank = local / per;
     bh = xcd * per + local % per;
   } else {
-    wid = local * kXcd + xcd;
     rank = wid / nbh;
     bh = wid % nbh;
   }

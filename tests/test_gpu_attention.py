@@ -1388,10 +1388,11 @@ def test_softcap_rows_do_not_depend_on_what_they_cannot_see(dev, dtype, numerics
 
 
 @pytest.mark.parametrize("D", [64, 128])
-@pytest.mark.parametrize("H,L", [(5, 13200), (8, 8200), (16, 4096)])
+@pytest.mark.parametrize("H,L", [(5, 13200), (8, 8200), (16, 4096), (5, 26300), (8, 16400)])
 def test_every_tile_is_visited_whatever_the_workgroup_order(dev, H, L, D):
-    """Workgroups of the second (fourth) round over the compute units run backwards through the tiles; a head by itself has too
-    few tiles for a second round.  The kernels are the same either way, so the results are, bit for bit."""
+    """Workgroups of the second round over the compute units (256 tiles), in the log-sum-exp pass also those of the fourth (1024
+    tiles: the last two lengths), run backwards through the tiles; a head by itself has too few tiles for a second round.
+    The kernels are the same either way, so the results are, bit for bit."""
     print("case workgroup order", H, L, D, flush=True)
     q, k, v = (t.to(dev) for t in seeded_qkv(1, H, H, L, L, D, torch.bfloat16))
     bm = fa.create_block_mask(generate_sliding_window(200), None, None, L, L, device=dev)
