@@ -116,7 +116,8 @@ __global__ __launch_bounds__(256, ((D == 128 && MODE == kBwdFast) || D >= 192) ?
   if (lse == -INFINITY) lse = INFINITY;  // row without visible keys: P = 0
   // The parity numerics scale dS = P o (dP - delta) before it is rounded.  The factor's magnitude joins the exponent of P,
   // its sign the result: as a product of its own, with a scalar operand (4 cycles instead of 2), it was 64 of 500 vector
-  // cycles per 32x32 block.
+  // cycles per 32x32 block.  A scale of 0 makes the exponent -inf and dS 0.  Where the logarithm is no multiple of 1/2 it and
+  // the difference round: dS carries about 1e-7 relative instead of 0.5e-7 into its own rounding, 5e-4 or 4e-3.
   if constexpr (MODE == kBwdParity) lse -= log2f(fabsf(p.scale));
 
   const FlexTileLists& tl = p.tiles_bwd;
@@ -488,8 +489,12 @@ __global__ __launch_bounds__(DkvShape<D>::kThreads, D == 64 ? 2 : 1) void bwd_dk
   const FlexTileLists& tl = p.tiles_bwd;
   Score2<KIND> sm;
   // parity numerics: dS = P o (scale * dP - scale * delta), one fused multiply-add per entry.  In a vector register where
-  // one is to spare: an operand from a scalar register makes it 4 cycles instead of 2.
-  const float scale = D == 64 ? p.scale : vector_value(p.scale);
+  // one is to spare: an operand from a scalar register makes it 4 cycles instead of 2.  (Held in one by the kernels that have
+  // no use for it, it cost the unrounded soft-cap at D = 128 four per cent: f16 [8,8,2048,128] causal 275 against 265 us.)
+  // Rounding: scale * delta is rounded once more than in P o (dP - delta) * scale, where scale is no power of two, by up to half
+  // a unit of a delta that is a float32 sum and so no more exact itself: a row with one visible key, dS = 0, leaves a residue
+  // of the same size either way (bf16 D = 128, scale 0.1: largest |dK| 1.1e-5 both; scale 1.7: 3.3e-4 and 3.2e-4).
+  const float scale = PARITY && D != 64 ? vector_value(p.scale) : p.scale;
   float key_grad = 1.f;  // derivative of a score_mod that depends on the key only: applied to dK at the end
 
   for (int gi = SPLIT ? part % parts_g : 0; gi < G; gi += SPLIT ? parts_g : 1) {
