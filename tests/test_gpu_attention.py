@@ -1406,3 +1406,38 @@ def test_every_tile_is_visited_whatever_the_workgroup_order(dev, H, L, D):
     for h in (0, H // 2, H - 1):
         for a, b in zip(whole, step(*(t[:, h:h + 1] for t in (q, k, v)))):
             assert torch.equal(a[:, h:h + 1], b)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("scale", [-0.1, 0.0, 0.05, 1.7])
+@pytest.mark.parametrize("D,Hq,Hkv,Lq,Lkv", [(64, 4, 2, 300, 333), (128, 3, 3, 130, 260), (128, 16, 4, 2048, 2048), (192, 2, 1, 129, 200)])
+def test_parity_backward_at_any_scale(dev, dtype, scale, D, Hq, Hkv, Lq, Lkv):
+    """The parity numerics apply the scale before dS is rounded, inside the kernels: negative, zero, above one and no power of
+    two, under score_mods with and without a derivative of their own, with rows that see no key; one call has its dK/dV divided
+    over the queries.  A scale of zero leaves no gradient of q and k at all."""
+    print("case scale", dtype, scale, D, Lq, flush=True)
+    q, k, v = seeded_qkv(1, Hq, Hkv, Lq, Lkv, D, dtype)
+    # scores and gradients at the largest scale as large as the default scale makes them of normal inputs (1.7 * 0.05 is about
+    # 1 / sqrt(128), 1.7 / 16 about the same): the tolerances are made for the rounding of those
+    q = (0.05 * q.float()).to(dtype)
+    d_o = (torch.randn(q.shape, generator=torch.Generator().manual_seed(3)) / 16).to(dtype)
+    mods = ((None, None), (generate_alibi_bias(Hq, -1.0), o_alibi_config(Hq)), (generate_tanh_softcap(3.0), o_tanh_softcap(3.0)),
+            (checkerboard, o_checkerboard))
+    for score, oscore in mods[:2] if Lq > 1000 else mods:
+        qd, kd, vd = (t.to(dev).requires_grad_(True) for t in (q, k, v))
+        bm = fa.create_block_mask(offset_causal_mask(-2), None, None, Lq, Lkv, device=dev)
+        out = fa.flax_attention(qd, kd, vd, score_mod=score, block_mask=bm, scale=scale, enable_gqa=Hq != Hkv,
+                                kernel_options={"numerics": "parity"})
+        got = (out, *torch.autograd.grad(out, (qd, kd, vd), d_o.to(dev)))
+        want = (ref_attention(q, k, v, oscore, o_offset_causal(-2), scale=scale),
+                *ref_attention_bwd(q, k, v, d_o, oscore, o_offset_causal(-2), scale=scale))
+        for what, a, b in zip(("O", "dQ", "dK", "dV"), got, want):
+            if scale == 0.0 and what in ("O", "dV"):
+                # a row's n probabilities are all 1 / n: where that lies within float32's error of the middle between two
+                # values of the dtype, all of them may round the other way, by one unit of at most eps
+                assert rel_l2(a.detach().cpu(), b) <= torch.finfo(dtype).eps, what
+            else:
+                close(a, b, dtype, what, scale_maxabs=True)
+        if scale == 0.0:
+            assert not got[1].any() and not got[2].any()
+        assert not got[1][:, :, :2].any()   # the rows without a key
