@@ -63,7 +63,7 @@ class FlexAttnParams(C.Structure):
 
 EXPORTS = [
     "flexattn_abi_version", "flexattn_last_error", "flexattn_preferred_tiles", "flexattn_kernel_family",
-    "flexattn_block_mask_workspace_bytes", "flexattn_block_mask_build", "flexattn_pack_mask", "flexattn_bitmap_fit",
+    "flexattn_block_mask_workspace_bytes", "flexattn_block_mask_workspace_needed", "flexattn_block_mask_build", "flexattn_pack_mask", "flexattn_bitmap_fit",
     "flexattn_affine_tables",
     "flexattn_fwd_workspace_bytes", "flexattn_fwd_workspace_needed", "flexattn_fwd",
     "flexattn_bwd_workspace_bytes", "flexattn_bwd_workspace_needed", "flexattn_bwd",
@@ -102,6 +102,8 @@ def lib() -> C.CDLL:
     L.flexattn_kernel_family.argtypes = [C.POINTER(FlexAttnParams), C.c_int32]
     L.flexattn_block_mask_workspace_bytes.restype = C.c_size_t
     L.flexattn_block_mask_workspace_bytes.argtypes = [C.c_int32] * 4
+    L.flexattn_block_mask_workspace_needed.restype = C.c_size_t
+    L.flexattn_block_mask_workspace_needed.argtypes = [C.POINTER(FlexMask)] + [C.c_int32] * 6
     L.flexattn_block_mask_build.argtypes = ([C.POINTER(FlexMask)] + [C.c_int32] * 6 +
                                             [C.c_void_p] * 8 + [C.c_void_p, C.c_void_p])
     L.flexattn_pack_mask.argtypes = [C.c_void_p, C.POINTER(C.c_int64)] + [C.c_int32] * 6 + [C.c_void_p] * 4

@@ -280,8 +280,8 @@ def build_lists(spec: MaskMod, B: int, H: int, nq: int, nkv: int, q_block: int, 
         q_num_blocks=torch.empty((B, H, nkv), **i32), q_indices=torch.empty((B, H, nkv, nq), **i32),
         full_q_num_blocks=torch.empty((B, H, nkv), **i32), full_q_indices=torch.empty((B, H, nkv, nq), **i32),
     )
-    ws = torch.empty(L.flexattn_block_mask_workspace_bytes(B, H, nq, nkv), dtype=torch.uint8, device=device)
     m = spec.c_struct()
+    ws = torch.empty(max(L.flexattn_block_mask_workspace_needed(m, B, H, nq, nkv, q_block, kv_block), 256), dtype=torch.uint8, device=device)
     with _on_device(ws.device):
         rc = L.flexattn_block_mask_build(
             m, B, H, nq, nkv, q_block, kv_block,

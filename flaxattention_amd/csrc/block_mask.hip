@@ -15,8 +15,8 @@ namespace flex {
 
 constexpr int kClassifyThreads = 256;
 
-// Bitmaps whose tiles are not made of classified blocks.  One workgroup per tile.  flags: [B*H, nq, nkv] int8 for partial
-// and full.
+// Bitmaps whose classes the ordering kernel does not work out itself (tile_source).  One workgroup per tile.  flags:
+// [B*H, nq, nkv] int8 for partial and full.
 __global__ __launch_bounds__(kClassifyThreads) void classify_tiles_kernel(
     FlexMask mask, int H, int nq, int nkv, int qb, int kvb, int8_t* __restrict__ partial,
     int8_t* __restrict__ full) {
@@ -60,10 +60,20 @@ __global__ __launch_bounds__(kClassifyThreads) void classify_tiles_kernel(
 //   kBand    with d = q + q_offset - kv a key is visible iff d >= lo && (d <= hi || kv <= sink): a tile is full iff its first row
 //            sees its last key and its last row's gap (sink, q + q_offset - hi) misses it, and empty iff every row ends ahead
 //            of the tile or has the gap over all of it
-//   kClasses a bitmap that carries the classes of its 32 x 32 blocks, tiles made of whole blocks
+//   kClasses a bitmap that carries the classes of its 32 x 32 blocks, tiles made of a few whole blocks
 // Lists of a band of 512 rows against 16384 keys in tiles of 128 x 128: classify + order 4.7 + 4.6 us, in one launch 4.6; documents
 // [2,3000 x 3000] 6.2 + 2.8 -> 7.0.  bf16 [1,32->8,512 of 16384,128] forward with a fresh mask (two sets of lists): 249.4 -> 244.3.
 enum { kFlags = 0, kBand = 1, kClasses = 2 };
+// A lane reads a tile's block classes one after the other, twice a list (to count, to write) and for every (b, h): so only where a
+// tile has at most 16 of them, and where a map that all (b, h) share is not gone through more than 16 times over.  Lists of
+// documents [2,3072,3072], flags / classes: 8 blocks a tile 6.8 / 5.1 us, 16 6.5 / 5.5, 32 6.5 / 9.6, 64 6.8 / 12.1, 1024
+// 33.6 / 97.4; of one shared map [2048,2048] at 128 x 128 for 16 (b, h) 6.8 / 5.6, for 64 6.8 / 8.5, for 256 7.7 / 22.6.
+static int tile_source(const FlexMask& mask, int B, int H, int qb, int kvb) {
+  if (mask.kind == FLEX_MASK_BAND) return kBand;
+  const bool shared = mask.bits_stride_b == 0 && mask.bits_stride_h == 0;
+  const bool few = qb % 32 == 0 && kvb % 32 == 0 && (long long)(qb / 32) * (kvb / 32) <= 16 && (!shared || (long long)B * H <= 16);
+  return mask.blk && few ? kClasses : kFlags;
+}
 struct TileSource {
   FlexMask mask;
   int qb, kvb, H;
@@ -276,6 +286,10 @@ extern "C" size_t flexattn_block_mask_workspace_bytes(int32_t B, int32_t H, int3
   size_t n = (size_t)B * H * nq * nkv;
   return 2 * ((n + 255) / 256 * 256);
 }
+extern "C" size_t flexattn_block_mask_workspace_needed(const FlexMask* mask, int32_t B, int32_t H, int32_t nq, int32_t nkv, int32_t qb,
+                                                       int32_t kvb) {
+  return mask && tile_source(*mask, B, H, qb, kvb) == kFlags ? flexattn_block_mask_workspace_bytes(B, H, nq, nkv) : 0;
+}
 
 void flex_set_error(const char* fmt, ...);
 
@@ -300,9 +314,7 @@ extern "C" int flexattn_block_mask_build(const FlexMask* mask, int32_t B, int32_
   size_t n = (size_t)B * H * nq * nkv;
   int8_t* partial = (int8_t*)workspace;
   int8_t* full = partial + (n + 255) / 256 * 256;
-  // where a tile's class takes a few operations the ordering kernel works it out itself
-  const bool blocks = mask->kind == FLEX_MASK_BITS && mask->blk && qb % 32 == 0 && kvb % 32 == 0;
-  const int source = mask->kind == FLEX_MASK_BAND ? kBand : blocks ? kClasses : kFlags;
+  const int source = tile_source(*mask, B, H, qb, kvb);
   // (a bitmap broadcast over batch and head does not look at (b, h): its tiles are classified once and every (b, h) orders
   // the same flags)
   const bool uniform = mask->bits_stride_b == 0 && mask->bits_stride_h == 0;

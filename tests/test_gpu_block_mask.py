@@ -236,10 +236,10 @@ def test_band_fit_of_packed_bitmaps(dev, Q, KV):
     assert _fit_bitmaps(pack_bits(torch.rand(Q, KV, generator=g) < 0.5)[None].to(dev)) == (True, None)
 
 
-@pytest.mark.parametrize("bs", [32, 64, 128, (64, 96), (96, 32), (160, 128), (48, 80)], ids=str)
+@pytest.mark.parametrize("bs", [32, 64, 128, (64, 96), (96, 32), (160, 128), (48, 80), 256, (512, 32), (32, 512), (64, 1024)], ids=str)
 @pytest.mark.parametrize("B,H,Q,KV", [(2, 1, 700, 700), (1, 3, 130, 1000), (2, 2, 33, 31)])
 def test_lists_of_bitmaps_at_any_block_size(dev, B, H, Q, KV, bs):
-    """Tiles made of whole 32 x 32 blocks are told by the blocks' classes, others by counting bits; empty, full and mixed tiles,
+    """Tiles made of up to 16 whole 32 x 32 blocks are told by the blocks' classes, others by counting bits; empty, full and mixed tiles,
     maps that differ by batch and head, lengths that end inside a tile."""
     print("case bitmap lists", B, H, Q, KV, bs, flush=True)
     gen = torch.Generator().manual_seed(Q + KV)
@@ -249,3 +249,16 @@ def test_lists_of_bitmaps_at_any_block_size(dev, B, H, Q, KV, bs):
         table = doc.to(q.device)   # (positions past the lengths are padding: a captured table is read at the last one there)
         return table[b, h, q.clamp(max=Q - 1)] >= table[b, h, kv.clamp(max=KV - 1)]
     check(fa.create_block_mask(mask, B, H, Q, KV, BLOCK_SIZE=bs, device=dev), ref_create_block_mask(mask, B, H, Q, KV, BLOCK_SIZE=bs))
+
+
+@pytest.mark.parametrize("B,H", [(1, 1), (2, 8), (3, 6), (4, 16)])
+@pytest.mark.parametrize("bs", [64, 128, 256])
+def test_lists_of_a_map_that_all_heads_share(dev, B, H, bs):
+    """One bitmap for every (batch, head): up to 16 of them read its classes themselves, more order flags that were made once."""
+    print("case shared map", B, H, bs, flush=True)
+    ids = torch.randint(0, 3, (40,), generator=torch.Generator().manual_seed(bs)).repeat_interleave(29)
+
+    def mask(b, h, q, kv):
+        table = ids.to(q.device)
+        return table[q.clamp(max=999)] >= table[kv.clamp(max=899)]   # (past the lengths: padding, read at the last position)
+    check(fa.create_block_mask(mask, B, H, 1000, 900, BLOCK_SIZE=bs, device=dev), ref_create_block_mask(mask, B, H, 1000, 900, BLOCK_SIZE=bs))

@@ -606,3 +606,26 @@ def test_float32_forward_divides_the_keys_where_tiles_are_even(D):
         p.mask.lo, p.mask.hi, p.mask.sink = lo, hi, sink
         want = (3 * 4096 * 2 * (D + 2) * 4 + 255) // 256 * 256 if divided else 0
         assert L.flexattn_fwd_workspace_needed(p) == want, (lo, hi, sink)
+
+
+def test_block_lists_classify_in_the_ordering_launch_only_where_tiles_are_small():
+    """Bands, and bitmaps with block classes whose tiles hold at most 16 blocks, need no room for flags; larger tiles, tiles that cut
+    blocks, bitmaps without classes and a map shared by many (batch, head) are classified once, with a workgroup a tile."""
+    L = _lib.lib()
+    need = L.flexattn_block_mask_workspace_needed
+
+    def mask(kind=_lib.MASK_BITS, blk=True, stride_b=4096):
+        m = _lib.FlexMask()
+        m.kind, m.hi, m.bits = kind, 2**31 - 1, 4096      # (only whether the arrays are there is looked at)
+        m.blk = 4096 if blk else None
+        m.bits_stride_b = m.blk_stride_b = stride_b
+        return m
+    for qb, kvb, few in ((32, 32, True), (128, 64, True), (128, 128, True), (512, 32, True), (32, 512, True), (160, 128, False), (256, 128, False),
+                         (256, 256, False), (1024, 1024, False), (8192, 8192, False), (48, 64, False), (64, 80, False), (31, 33, False)):
+        size = L.flexattn_block_mask_workspace_bytes(2, 3, 4, 5)
+        assert need(mask(), 2, 3, 4, 5, qb, kvb) == (0 if few else size), (qb, kvb)
+        assert need(mask(blk=False), 2, 3, 4, 5, qb, kvb) == size
+        assert need(mask(_lib.MASK_BAND), 2, 3, 4, 5, qb, kvb) == 0
+    for B, H, few in ((1, 1, True), (2, 8, True), (1, 17, False), (4, 16, False)):
+        assert need(mask(stride_b=0), B, H, 4, 5, 128, 128) == (0 if few else L.flexattn_block_mask_workspace_bytes(B, H, 4, 5))
+        assert need(mask(), B, H, 4, 5, 128, 128) == 0
