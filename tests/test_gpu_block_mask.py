@@ -133,7 +133,7 @@ def test_from_kv_blocks_transposes(dev):
 
 @pytest.mark.parametrize("seed", range(12))
 def test_band_closed_form_matches_brute_force(dev, seed):
-    """Band masks are classified per tile from a closed-form row count; the oracle evaluates every
+    """Band masks are classified per tile from its corners; the oracle evaluates every
     (q, kv) pair.  Random band parameters, including unbounded sides, sinks and offsets."""
     import random
     from flaxattention_amd.core.common import INT_MAX
@@ -262,3 +262,18 @@ def test_lists_of_a_map_that_all_heads_share(dev, B, H, bs):
         table = ids.to(q.device)
         return table[q.clamp(max=999)] >= table[kv.clamp(max=899)]   # (past the lengths: padding, read at the last position)
     check(fa.create_block_mask(mask, B, H, 1000, 900, BLOCK_SIZE=bs, device=dev), ref_create_block_mask(mask, B, H, 1000, 900, BLOCK_SIZE=bs))
+
+
+@pytest.mark.parametrize("bs", [32, 128, (48, 80), (128, 1), (1, 64)], ids=str)
+@pytest.mark.parametrize("lo,hi,sink,off", [(5, 4, -1, 0), (5, 4, 70, 0), (5, 4, 79, 3), (0, -1, 127, 0), (2**31 - 1, 2**31 - 1, -1, 0), (-300, -90, -1, 0),
+                                            (-300, -90, 31, -7), (INT_MIN, -1, 40, 0), (0, 0, -1, 0), (INT_MIN, 2**31 - 1, -1, 0), (0, 63, 1000, 50)])
+def test_band_edges_against_brute_force(dev, lo, hi, sink, off, bs):
+    """Empty bands with and without sinks (inside a tile, on its last key), bands ahead of the diagonal, unbounded sides, a band of
+    one key, tiles of one row or one key."""
+    print("case band edges", lo, hi, sink, off, bs, flush=True)
+
+    def omask(b, h, q_idx, kv_idx):
+        d = q_idx + off - kv_idx
+        return (d >= lo) & ((d <= hi) | (kv_idx <= sink))
+    check(fa.create_block_mask(MaskMod(lo, hi, sink, off, name="band"), 1, 1, 200, 330, BLOCK_SIZE=bs, device=dev),
+          ref_create_block_mask(omask, 1, 1, 200, 330, BLOCK_SIZE=bs))
