@@ -445,19 +445,16 @@ __global__ __launch_bounds__(256) void decode_combine_kernel(FlexAttnParams p, c
   // the kernel is a chain of memory latencies (its data was written by other XCDs and comes from HBM), and this
   // way there is one of them instead of two
   float v0[8][D / 64];
-  if (o) {
 #pragma unroll
-    for (int u = 0; u < 8; u++)
+  for (int u = 0; u < 8; u++)
 #pragma unroll
-      for (int a = 0; a < D / 64; a++) v0[u][a] = (u < splits) ? o_part[(u * rows + row) * D + lane + 64 * a] : 0.f;
-  }
+    for (int a = 0; a < D / 64; a++) v0[u][a] = (u < splits) ? o_part[(u * rows + row) * D + lane + 64 * a] : 0.f;
   float m = ms;
   for (int off = 32; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
   const float sc = (ms == -INFINITY) ? 0.f : fast_exp2(ms - m);
   float l = sc * ls;
   for (int off = 32; off > 0; off >>= 1) l += __shfl_xor(l, off, 64);
   if (lse2 && lane == 0) lse2[row] = l > 0.f ? m + log2f(l) : -INFINITY;
-  if (!o) return;  // first pass of the parity numerics: only the merged log-sum-exp
   float acc[D / 64];
 #pragma unroll
   for (int a = 0; a < D / 64; a++) acc[a] = 0.f;

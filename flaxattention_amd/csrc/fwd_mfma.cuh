@@ -42,6 +42,34 @@ constexpr int kPipeBM = 256;  // query rows of a workgroup of the pipelined dens
 //                instructions per fragment) and the row sum adds the unrounded exponentials: the "unrounded"
 //                numerics, launched with ROUND_S = false
 enum { kFwdOnePass = 0, kFwdLse = 1, kFwdNorm = 2, kFwdHiLo = 3 };
+
+// Base-2 log-sum-exp of a row of which n shares left (m, l) at ml[s * rows], -inf if none saw a key.  Each half of a wave
+// holds the row and takes every second share, N of them in flight together: the loads are what it waits for, and with a
+// maximum between every four of them a call of 64 shares waited sixteen times.  bf16 forwards against the end of a cache, the
+// merge as a launch of its own / four shares at a time / here: 64 shares [1,8,128 of 32768,64] 44.2 / 51.3 / 44.8 us, D = 128
+// 60.4 / 67.9 / 60.9; 32 shares [1,8,256 of 16384,64] 40.6 / 42.3 / 39.6; 8 shares [1,16,512 of 8192,64] 62.3 / 60.4 / 59.7;
+// 4 shares [1,32,512 of 16384,128] 285.7 / 283.0 / 285.0 (a launch's host time not counted)
+template <int N>
+__device__ __forceinline__ float merged_lse(const float2* ml, int64_t rows, int n, int g) {
+  float m = -INFINITY, l = 0.f;
+  for (int s0 = 0; s0 < n; s0 += 2 * N) {
+    float2 part[N];
+#pragma unroll
+    for (int u = 0; u < N; u++) part[u] = ml[min(s0 + 2 * u + g, n - 1) * rows];
+    float m_new = m;
+#pragma unroll
+    for (int u = 0; u < N; u++) m_new = fmaxf(m_new, part[u].x);
+    if (m_new == -INFINITY) continue;
+    l *= fast_exp2(m - m_new);
+#pragma unroll
+    for (int u = 0; u < N; u++) l += s0 + 2 * u + g < n ? fast_exp2(part[u].x - m_new) * part[u].y : 0.f;
+    m = m_new;
+  }
+  const float top = xhalf_max(m);
+  l = xhalf_sum(m == -INFINITY ? 0.f : l * fast_exp2(m - top));
+  return l > 0.f ? top + log2f(l) : -INFINITY;
+}
+
 // D = 256: one wave per SIMD (Q fragments, K fragments and the accumulator are 64 + 64 + 128 registers, the V
 // fragments another 64 that are fetched late) and the two stages are 128 KB.
 template <typename T, int D, int KIND, bool ROUND_S, bool BITS, int PASS = kFwdOnePass>
@@ -51,7 +79,8 @@ __global__ __launch_bounds__(256, D >= 192 ? 1 : 2) void fwd_mfma_kernel(FlexAtt
                                                            float* __restrict__ o_part, float* __restrict__ ml_part) {
   // Split-KV: with gridDim.y > 1 workgroup (x, y) visits share y of its query tile's key tiles and leaves an
   // unnormalised partial (O, m, l) per row in o_part / ml_part, in the layout decode_combine_kernel merges (kFwdLse:
-  // only (m, l), which kFwdNorm merges for its rows; the partial outputs of kFwdNorm add up).  For calls whose query tiles alone would leave most compute units without a workgroup.
+  // only (m, l), which kFwdNorm merges for its rows; the partial outputs of kFwdNorm add up).  For calls whose query tiles
+  // alone would leave most compute units without a workgroup.
   typedef typename Frag<T>::vec8 vec8;
   typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
   constexpr int RQ = 1, BM = kFwdBM, BN = kFwdBN;
@@ -207,24 +236,10 @@ __global__ __launch_bounds__(256, D >= 192 ? 1 : 2) void fwd_mfma_kernel(FlexAtt
         l2 = lse2[row];
       } else {
         // the first pass left (m, l) of every share: every workgroup merges those of its own rows, the first share writes the
-        // result out (the merge in a launch of its own: bf16 [1,32->8,512 of 16384,128] 252.7 us, here 249.4)
+        // result out
         const float2* ml = reinterpret_cast<const float2*>(ml_part) + row;
         const int64_t rows = (int64_t)p.B * p.Hq * p.Lq;
-        float m = -INFINITY, l = 0.f;
-        for (int s0 = 0; s0 < nsplit; s0 += 4) {
-          float2 part[4];   // four shares' loads in flight together
-#pragma unroll
-          for (int u = 0; u < 4; u++) part[u] = ml[min(s0 + u, nsplit - 1) * rows];
-          float m_new = m;
-#pragma unroll
-          for (int u = 0; u < 4; u++) m_new = fmaxf(m_new, part[u].x);
-          if (m_new == -INFINITY) continue;
-          l *= fast_exp2(m - m_new);
-#pragma unroll
-          for (int u = 0; u < 4; u++) l += s0 + u < nsplit ? fast_exp2(part[u].x - m_new) * part[u].y : 0.f;
-          m = m_new;
-        }
-        l2 = l > 0.f ? m + log2f(l) : -INFINITY;
+        l2 = nsplit <= 8 ? merged_lse<4>(ml, rows, nsplit, g) : merged_lse<16>(ml, rows, nsplit, g);
         if (split == 0 && g == 0 && q_row0 + 32 * a < p.Lq) lse2[row] = l2;
       }
       m_run[a] = l2 == -INFINITY ? INFINITY : l2;

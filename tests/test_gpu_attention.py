@@ -295,6 +295,23 @@ def test_forward_split_over_keys(dev, name, dtype, D, B, Hq, Hkv, Lq, opts):
     assert nbytes >= 2 * B * Hq * Lq * (D + 2) * 4
 
 
+@pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 64), (torch.float16, 128), (torch.bfloat16, 256)], ids=str)
+@pytest.mark.parametrize("Lkv,shares", [(2600, 5), (4300, 8), (4700, 9), (9000, 17), (17000, 33), (33000, 64)])
+def test_parity_forward_over_many_shares(dev, dtype, D, Lkv, shares):
+    """The second pass of a parity forward merges the log-sum-exps of any number of shares: rows that see almost all keys, rows
+    that see only the first few (most shares empty, another number of them for every query tile), rows that see none."""
+    from flaxattention_amd import _lib
+    from flaxattention_amd.core.attention import _make_plan
+    print("case many shares", dtype, D, Lkv, flush=True)
+    Lq, H = 130, 2
+    opts = {"numerics": "parity", "decode": False}
+    for off in (Lkv - Lq - 2, 700, -2):
+        run(dev, dtype, 1, H, H, Lq, Lkv, D, mask=offset_causal_mask(off), omask=o_offset_causal(off), strict=False, opts=opts, grad=False)
+    q, k, v = (t.to(dev) for t in seeded_qkv(1, H, H, Lq, Lkv, D, dtype))
+    nbytes = _lib.lib().flexattn_fwd_workspace_needed(_make_plan(q, k, v, None, None, None, 1.0, opts).params(q, k, v, torch.empty_like(q)))
+    assert nbytes // (H * Lq * (D + 2) * 4) == shares
+
+
 def test_forward_split_unrounded_equals_unsplit(dev):
     """The "unrounded" numerics over split key ranges against the same call without a workspace (one pass over all
     keys), through the C ABI; a causal bitmap-free band mask with tile lists."""
