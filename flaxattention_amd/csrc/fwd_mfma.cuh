@@ -86,6 +86,7 @@ __global__ __launch_bounds__(256, D >= 192 ? 1 : 2) void fwd_mfma_kernel(FlexAtt
   constexpr int RQ = 1, BM = kFwdBM, BN = kFwdBN;
   constexpr int DS = D / 16;     // k-steps of the Q.K^T product
   constexpr int DB = D / 32;     // 32-row blocks of O^T
+  constexpr bool kRowsAhead = D >= 192 && !(D == 192 && KIND == FLEX_SCORE_AFFINE && PASS == kFwdHiLo);   // K rows by read_ahead
   constexpr int CPR = D / 8;     // 16-byte chunks per row
   // a wave fills 16 rows (one swizzle period) of a tile: 16 * CPR chunks, 64 per fetch instruction, laid down one after
   // the other; at D = 192 an instruction ends in the middle of a row
@@ -294,7 +295,7 @@ __global__ __launch_bounds__(256, D >= 192 ? 1 : 2) void fwd_mfma_kernel(FlexAtt
       vec8 kfr[DS], vfr[2][DB];
       {
         const T* kp = Ks + (nb * 32 + i32) * D;
-        if constexpr (D < 192) {
+        if constexpr (!kRowsAhead) {
 #pragma unroll
           for (int s = 0; s < DS; s++) kfr[s] = *reinterpret_cast<const vec8*>(kp + (((2 * s) ^ kz) * 8));
         }
@@ -316,9 +317,11 @@ __global__ __launch_bounds__(256, D >= 192 ? 1 : 2) void fwd_mfma_kernel(FlexAtt
       for (int a = 0; a < RQ; a++)
 #pragma unroll
         for (int r = 0; r < 16; r++) sacc[a][r] = 0.f;
-      if constexpr (D >= 192) {
+      if constexpr (kRowsAhead) {
         // one wave per SIMD: K rows four steps, below V columns four steps ahead of their products.  [2,8,2048,256] causal,
-        // undivided: f16 121 -> 104 us, bf16 parity 59 -> 54 and 91 -> 82; D = 192 f16 96 -> 83
+        // undivided: f16 121 -> 104 us, bf16 parity 59 -> 54 and 91 -> 82; D = 192 f16 96 -> 83.  (Not the K rows under an
+        // additive table of the unrounded numerics at D = 192, whose loads they then hold up: f16 [4,8,2048,192] 399 us with
+        // neither, 408 with both, 390 with the V columns alone; causal 220 / 225 / 212)
         const T* kp = Ks + (nb * 32 + i32) * D;
         read_ahead<DS, 4, vec8>(
             [&](int s, vec8& r) __attribute__((always_inline)) { r = *reinterpret_cast<const vec8*>(kp + (((2 * s) ^ kz) * 8)); },
