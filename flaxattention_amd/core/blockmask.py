@@ -27,7 +27,7 @@ import torch
 
 from .. import _lib
 from .common import (INT_MAX, INT_MIN, MaskMod, _get_mod_type, _ModificationType, _mask_mod_signature,
-                     _score_mod_signature, band_and, band_or, dense_mask_on_device, resolve_mask_mod, _on_device, _stream)
+                     _score_mod_signature, band_and, band_or, dense_mask_on_device, resolve_mask_mod, _on_cuda_device, _stream)
 
 Array = torch.Tensor
 
@@ -282,7 +282,7 @@ def build_lists(spec: MaskMod, B: int, H: int, nq: int, nkv: int, q_block: int, 
     )
     m = spec.c_struct()
     ws = torch.empty(max(L.flexattn_block_mask_workspace_needed(m, B, H, nq, nkv, q_block, kv_block), 256), dtype=torch.uint8, device=device)
-    with _on_device(ws.device):
+    with _on_cuda_device(ws.device):
         rc = L.flexattn_block_mask_build(
             m, B, H, nq, nkv, q_block, kv_block,
             out["kv_num_blocks"].data_ptr(), out["kv_indices"].data_ptr(),

@@ -33,13 +33,18 @@ def _stream(t) -> int:
     return torch.cuda.current_stream(t.device).cuda_stream
 
 
+def _on_cuda_device(dev):
+    """_on_device where no front end has looked at the device yet; another than a GPU is refused as torch.cuda.device does."""
+    if dev.type != "cuda":
+        raise ValueError(f"Expected a cuda device, but got: {dev}")
+    return _on_device(dev)
+
+
 class _on_device:
-    """torch.cuda.device(dev) only when dev is not already current (entering the context costs ~10 us of host time)."""
+    """torch.cuda.device(dev) only when dev, a GPU, is not already current (entering the context costs ~10 us of host time)."""
     __slots__ = ("ctx",)
 
     def __init__(self, dev):
-        if dev.type != "cuda":
-            raise ValueError(f"Expected a cuda device, but got: {dev}")
         idx = dev.index
         self.ctx = None if idx is None or idx == torch.cuda.current_device() else torch.cuda.device(dev)
 
@@ -410,7 +415,7 @@ def _tables_of_planes(fn: Callable, name: str, y: torch.Tensor, Lq: int) -> Opti
     add, mul = torch.empty_like(y[0]), torch.empty_like(y[0])
     diag = torch.empty((b, h, rows + Lkv - 1), dtype=torch.float32, device=y.device) if rows == Lq > 1 and Lkv > 1 else None
     flags = torch.zeros(4, dtype=torch.int32, device=y.device)
-    with _on_device(y.device):
+    with _on_cuda_device(y.device):
         rc = _lib.lib().flexattn_affine_tables(y.data_ptr(), b * h, rows, Lkv, add.data_ptr(), mul.data_ptr(),
                                                diag.data_ptr() if diag is not None else None, flags.data_ptr(),
                                                _stream(y))

@@ -629,3 +629,15 @@ def test_block_lists_classify_in_the_ordering_launch_only_where_tiles_are_small(
     for B, H, few in ((1, 1, True), (2, 8, True), (1, 17, False), (4, 16, False)):
         assert need(mask(stride_b=0), B, H, 4, 5, 128, 128) == (0 if few else L.flexattn_block_mask_workspace_bytes(B, H, 4, 5))
         assert need(mask(), B, H, 4, 5, 128, 128) == 0
+
+
+def test_block_lists_are_refused_off_the_gpu_and_attention_asks_once():
+    """Building lists on a CPU device raises what torch.cuda.device raises; the context that the attention calls enter does not look
+    at the device's type again, which their front end has refused already."""
+    from flaxattention_amd.core import blockmask, common
+    with pytest.raises(ValueError, match="Expected a cuda device"):
+        blockmask.build_lists(common.MaskMod(0, 2**31 - 1, -1), 1, 1, 2, 2, 128, 128, torch.device("cpu"))
+    assert common._on_device(torch.device("cpu")).ctx is None
+    with pytest.raises(_lib.FlexAttnError, match="HIP device only"):
+        x = torch.zeros(1, 1, 8, 64)
+        fa.flax_attention(x, x, x)
