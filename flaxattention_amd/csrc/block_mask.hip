@@ -16,7 +16,7 @@ namespace flex {
 constexpr int kClassifyThreads = 256;
 
 // Bitmaps whose classes the ordering kernel does not work out itself (tile_source).  One workgroup per tile.  flags:
-// [B*H, nq, nkv] int8 for partial and full.
+// [B*H, nq, nkv] int8 for partial and full (one set where the map is the same for all (b, h)).
 __global__ __launch_bounds__(kClassifyThreads) void classify_tiles_kernel(
     FlexMask mask, int H, int nq, int nkv, int qb, int kvb, int8_t* __restrict__ partial,
     int8_t* __restrict__ full) {
@@ -68,8 +68,12 @@ enum { kFlags = 0, kBand = 1, kClasses = 2 };
 // tile has at most 16 of them, and where a map that all (b, h) share is not gone through more than 16 times over.  Lists of
 // documents [2,3072,3072], flags / classes: 8 blocks a tile 6.8 / 5.1 us, 16 6.5 / 5.5, 32 6.5 / 9.6, 64 6.8 / 12.1, 1024
 // 33.6 / 97.4; of one shared map [2048,2048] at 128 x 128 for 16 (b, h) 6.8 / 5.6, for 64 6.8 / 8.5, for 256 7.7 / 22.6.
+// A band costs a lane some thirty operations a tile, for every (b, h): above 256 of them flags are made once, a thread per tile.
+// Causal lists, flags / corners: 256 (b, h) of [8192 x 8192] in 64 x 64 51.4 / 53.1 us, in 128 x 128 19.2 / 20.9, of [32768 x 32768] in
+// 128 x 128 171.5 / 155, small grids 10.5 / 7.9; 512 (b, h) of [2048 x 2048] in 64 x 64 16.6 / 20.7, of [8192 x 8192] in 128 x 128
+// 32.0 / 38.0, in 256 x 256 16.2 / 20.1 (flags by a workgroup a tile, as before the corners: 16.9, 33.6 and 16.6).
 static int tile_source(const FlexMask& mask, int B, int H, int qb, int kvb) {
-  if (mask.kind == FLEX_MASK_BAND) return kBand;
+  if (mask.kind == FLEX_MASK_BAND) return (long long)B * H <= 256 ? kBand : kFlags;
   const bool shared = mask.bits_stride_b == 0 && mask.bits_stride_h == 0;
   const bool few = qb % 32 == 0 && kvb % 32 == 0 && (long long)(qb / 32) * (kvb / 32) <= 16 && (!shared || (long long)B * H <= 16);
   return mask.blk && few ? kClasses : kFlags;
@@ -99,6 +103,16 @@ struct TileSource {
     return all ? 1 : none ? 2 : 0;
   }
 };
+
+// The flags of a band that many (b, h) order: a thread per tile, one set for all of them.
+__global__ __launch_bounds__(kClassifyThreads) void classify_band_kernel(TileSource src, int nq, int nkv, int8_t* __restrict__ partial,
+                                                                         int8_t* __restrict__ full) {
+  const long long at = (long long)blockIdx.x * kClassifyThreads + threadIdx.x;
+  if (at >= (long long)nq * nkv) return;
+  const int c = src.band((int)(at / nkv), (int)(at % nkv));
+  partial[at] = c == 0;
+  full[at] = c == 1;
+}
 
 // The four ordered lists of a block mask (partial / full, by query block / by key block) come from one
 // launch: blockIdx.y names the list.
@@ -315,10 +329,14 @@ extern "C" int flexattn_block_mask_build(const FlexMask* mask, int32_t B, int32_
   int8_t* partial = (int8_t*)workspace;
   int8_t* full = partial + (n + 255) / 256 * 256;
   const int source = tile_source(*mask, B, H, qb, kvb);
-  // (a bitmap broadcast over batch and head does not look at (b, h): its tiles are classified once and every (b, h) orders
-  // the same flags)
-  const bool uniform = mask->bits_stride_b == 0 && mask->bits_stride_h == 0;
-  if (source == kFlags)
+  // (a band, or a bitmap broadcast over batch and head, does not look at (b, h): its tiles are classified once and every
+  // (b, h) orders the same flags)
+  const bool uniform = mask->kind == FLEX_MASK_BAND || (mask->bits_stride_b == 0 && mask->bits_stride_h == 0);
+  const TileSource src = {*mask, qb, kvb, H};
+  if (source == kFlags && mask->kind == FLEX_MASK_BAND)
+    hipLaunchKernelGGL(classify_band_kernel, dim3((unsigned)(((long long)nq * nkv + kClassifyThreads - 1) / kClassifyThreads)),
+                       dim3(kClassifyThreads), 0, stream, src, nq, nkv, partial, full);
+  else if (source == kFlags)
     hipLaunchKernelGGL(classify_tiles_kernel, dim3(nkv, nq, uniform ? 1 : B * H), dim3(kClassifyThreads), 0, stream, *mask, H, nq,
                        nkv, qb, kvb, partial, full);
   const long long mat = uniform ? 0 : (long long)nq * nkv;
@@ -339,7 +357,6 @@ extern "C" int flexattn_block_mask_build(const FlexMask* mask, int32_t B, int32_
     const int waves = 4;
     const long long most_rows = (long long)B * H * (by_q ? (by_kv ? (nq > nkv ? nq : nkv) : nkv) : nq);
     const dim3 grid((unsigned)((most_rows + waves - 1) / waves), 4);
-    const TileSource src = {*mask, qb, kvb, H};
     if (source == kBand) hipLaunchKernelGGL(order_rows_kernel<kBand>, grid, dim3(64 * waves), 0, stream, jobs, src, mat, (long long)B * H);
     else if (source == kClasses) hipLaunchKernelGGL(order_rows_kernel<kClasses>, grid, dim3(64 * waves), 0, stream, jobs, src, mat, (long long)B * H);
     else hipLaunchKernelGGL(order_rows_kernel<kFlags>, grid, dim3(64 * waves), 0, stream, jobs, src, mat, (long long)B * H);

@@ -199,7 +199,7 @@ int flexattn_preferred_tiles(int32_t dtype, int32_t D, int32_t Dv, int32_t Lq, i
  * int32: counts [B,H,nq], indices [B,H,nq,nkv]; q_* are [B,H,nkv] and
  * [B,H,nkv,nq].  Any output pointer may be NULL.  `workspace` holds
  * flexattn_block_mask_workspace_bytes() bytes; flexattn_block_mask_workspace_needed() is what this very call uses of
- * them, 0 for bands and for bitmaps whose tiles are few 32x32 blocks each (the pointer must not be NULL all the same).  Those
+ * them, 0 for most bands and for bitmaps whose tiles are few 32x32 blocks each (the pointer must not be NULL all the same).  Those
  * bitmaps are classified from `blk` instead of `bits`, which must describe the same mask.  */
 size_t flexattn_block_mask_workspace_bytes(int32_t B, int32_t H, int32_t n_q_blocks, int32_t n_kv_blocks);
 size_t flexattn_block_mask_workspace_needed(const FlexMask* mask, int32_t B, int32_t H, int32_t n_q_blocks, int32_t n_kv_blocks,

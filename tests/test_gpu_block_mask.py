@@ -5,7 +5,7 @@ import torch
 
 import flaxattention_amd as fa
 from flaxattention_amd.masks import causal_mask, generate_attention_sink, generate_sliding_window, offset_causal_mask
-from flaxattention_amd.core.common import MaskMod, INT_MIN
+from flaxattention_amd.core.common import MaskMod, INT_MAX, INT_MIN
 from oracle import (o_attention_sink, o_causal_mask, o_full_masked, o_noop_mask, o_offset_causal, o_sink_window_lt,
                     o_sliding_window, ref_create_block_mask)
 
@@ -262,6 +262,26 @@ def test_lists_of_a_map_that_all_heads_share(dev, B, H, bs):
         table = ids.to(q.device)
         return table[q.clamp(max=999)] >= table[kv.clamp(max=899)]   # (past the lengths: padding, read at the last position)
     check(fa.create_block_mask(mask, B, H, 1000, 900, BLOCK_SIZE=bs, device=dev), ref_create_block_mask(mask, B, H, 1000, 900, BLOCK_SIZE=bs))
+
+
+@pytest.mark.parametrize("B,H", [(16, 16), (1, 257), (16, 32)])
+@pytest.mark.parametrize("lo,hi,sink,off", [(0, INT_MAX, -1, 0), (0, 60, 40, 3), (5, 4, 70, 0), (-300, -90, -1, 0)])
+@pytest.mark.parametrize("bs", [32, (48, 80)], ids=str)
+def test_lists_of_a_band_that_many_heads_share(dev, B, H, lo, hi, sink, off, bs):
+    """A band for more than 256 (batch, head): flags made once by a thread a tile, the same lists for all as for a single one."""
+    print("case shared band", B, H, lo, hi, sink, off, bs, flush=True)
+    mask = MaskMod(lo, hi, sink, off, name="band")
+    one = fa.create_block_mask(mask, 1, 1, 600, 700, BLOCK_SIZE=bs, device=dev)
+    all_heads = fa.create_block_mask(mask, B, H, 600, 700, BLOCK_SIZE=bs, device=dev)
+
+    def omask(b, h, q_idx, kv_idx):
+        d = q_idx + off - kv_idx
+        return (d >= lo) & ((d <= hi) | (kv_idx <= sink))
+    check(one, ref_create_block_mask(omask, 1, 1, 600, 700, BLOCK_SIZE=bs))
+    for name in ("kv_num_blocks", "kv_indices", "full_kv_num_blocks", "full_kv_indices", "q_num_blocks", "q_indices",
+                 "full_q_num_blocks", "full_q_indices"):
+        a, b = getattr(all_heads, name), getattr(one, name)
+        assert torch.equal(a, b.expand_as(a)), name
 
 
 @pytest.mark.parametrize("bs", [32, 128, (48, 80), (128, 1), (1, 64)], ids=str)

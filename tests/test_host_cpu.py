@@ -610,7 +610,8 @@ def test_float32_forward_divides_the_keys_where_tiles_are_even(D):
 
 def test_block_lists_classify_in_the_ordering_launch_only_where_tiles_are_small():
     """Bands, and bitmaps with block classes whose tiles hold at most 16 blocks, need no room for flags; larger tiles, tiles that cut
-    blocks, bitmaps without classes and a map shared by many (batch, head) are classified once, with a workgroup a tile."""
+    blocks, bitmaps without classes and a map shared by many (batch, head) are classified once, with a workgroup a tile.  A band
+    for more than 256 (batch, head) is classified once too."""
     L = _lib.lib()
     need = L.flexattn_block_mask_workspace_needed
 
@@ -629,6 +630,8 @@ def test_block_lists_classify_in_the_ordering_launch_only_where_tiles_are_small(
     for B, H, few in ((1, 1, True), (2, 8, True), (1, 17, False), (4, 16, False)):
         assert need(mask(stride_b=0), B, H, 4, 5, 128, 128) == (0 if few else L.flexattn_block_mask_workspace_bytes(B, H, 4, 5))
         assert need(mask(), B, H, 4, 5, 128, 128) == 0
+    for B, H, few in ((1, 256, True), (16, 16, True), (1, 257, False), (16, 32, False)):
+        assert need(mask(_lib.MASK_BAND), B, H, 4, 5, 128, 128) == (0 if few else L.flexattn_block_mask_workspace_bytes(B, H, 4, 5))
 
 
 def test_block_lists_are_refused_off_the_gpu_and_attention_asks_once():
