@@ -118,7 +118,11 @@ __global__ __launch_bounds__(256, ((D == 128 && MODE == kBwdFast) || D >= 192) ?
   // its sign the result: as a product of its own, with a scalar operand (4 cycles instead of 2), it was 64 of 500 vector
   // cycles per 32x32 block.  A scale of 0 makes the exponent -inf and dS 0.  Where the logarithm is no multiple of 1/2 it and
   // the difference round: dS carries about 1e-7 relative instead of 0.5e-7 into its own rounding, 5e-4 or 4e-3.
-  if constexpr (MODE == kBwdParity) lse -= log2f(fabsf(p.scale));
+  // (Not in the identity kernel of float16 at D = 128: without the products the compiler puts its reads closer to their uses,
+  // 129 waits instead of 108, and with one workgroup on a compute unit nothing covers them: [2,8,2048,128] causal dQ 80.7 us
+  // against 76.7, the backward 204.5 : 200.2; its other score_mods take the same time either way, bfloat16 207 : 211 us)
+  constexpr bool kScaleInExponent = MODE == kBwdParity && !(D == 128 && KIND == FLEX_SCORE_IDENTITY && __is_same(T, f16));
+  if constexpr (kScaleInExponent) lse -= log2f(fabsf(p.scale));
 
   const FlexTileLists& tl = p.tiles_bwd;
   const int32_t* full_idx = nullptr;
@@ -330,6 +334,7 @@ __global__ __launch_bounds__(256, ((D == 128 && MODE == kBwdFast) || D >= 192) ?
             d0 = fast_exp2(sacc[r]) * (a0 - delta);
             d1 = fast_exp2(sacc[r + 1]) * (a1 - delta);
             if (!Score2<KIND>::kGradOne) { d0 *= gacc[r]; d1 *= gacc[r + 1]; }
+            if constexpr (!kScaleInExponent) { d0 *= p.scale; d1 *= p.scale; }
           } else {
             d0 = fast_exp2(sacc[r]) * dpacc[r];
             d1 = fast_exp2(sacc[r + 1]) * dpacc[r + 1];
@@ -385,7 +390,7 @@ __global__ __launch_bounds__(256, ((D == 128 && MODE == kBwdFast) || D >= 192) ?
     return;
   }
   // fast numerics: the scale factor of dS = P o (dP - delta) o g * scale is applied once here
-  const float out_scale = MODE == kBwdParity ? (p.scale < 0.f ? -1.f : 1.f) : p.scale;
+  const float out_scale = kScaleInExponent ? (p.scale < 0.f ? -1.f : 1.f) : MODE == kBwdParity ? 1.f : p.scale;
   if (q_row < p.Lq) {
     T* op = dq + row_id * D + 4 * g;
 #pragma unroll
