@@ -107,8 +107,10 @@ __global__ __launch_bounds__(256, D >= 192 ? 1 : 2) void fwd_mfma_kernel(FlexAtt
   const int nqt = (p.Lq + BM - 1) / BM;
   int rank, bh;
   // (the unrounded forward at D = 64 is slower with its second round turned: f16 [8,8,2048,64] causal 68.2 against 67.5 us, with
-  // an additive table 274.8 : 268.9)
-  xcd_tile_map<D >= 192 || (D == 64 && PASS == kFwdHiLo) ? 1 : PASS == kFwdLse ? 4 : 2>(blockIdx.x, nqt, p.Hq * p.B, rank, bh);
+  // an additive table 274.8 : 268.9; under a multiplicative and an additive table only calls with tile lists turn theirs: [4,8,2048,64]
+  // without a mask 696 against 680 us, parity 1404 : 1373, D = 128 1432 : 1392, causal 283 against 381 in plain order)
+  xcd_tile_map<D >= 192 || (D == 64 && PASS == kFwdHiLo) ? 1 : PASS == kFwdLse ? 4 : 2>(
+      blockIdx.x, nqt, p.Hq * p.B, rank, bh, KIND != kScoreAffineMul || p.tiles.kv_num);
   const int qt = nqt - 1 - rank;  // late query tiles see the most keys under causal masks
   const int h = bh % p.Hq, b = bh / p.Hq, hk = h / (p.Hq / p.Hkv);
 

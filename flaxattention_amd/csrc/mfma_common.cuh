@@ -569,14 +569,14 @@ template <int D> __device__ __forceinline__ constexpr int lds_swz(int r) {
 // problem the sums came out 32 .. 36 tiles where 34 is the mean).  Causal, bf16 [8,8,2048,64] log-sum-exp pass 42.5 -> 41.0 us,
 // row sweep 61.4 -> 58.7, dQ 77 -> 74.5; [1,32->8,4096,128] log-sum-exp 98 -> 95, second pass 150 -> 147, row sweep 152 -> 149.
 // Each kernel takes the number that was the fastest of those tried on it, at most the workgroups that a compute unit holds
-// of it; two kernels of the unrounded numerics are faster without (at their callers).  A mask that gives every tile the
-// same work is not affected.
+// of it; two kernels of the unrounded numerics are faster without (at their callers).  Tiles of the same work gain
+// nothing, and where a call streams tables past the caches they lose: the caller says by `turn` whether to.
 template <int ROUNDS>
-__device__ __forceinline__ void xcd_tile_map(int wid, int ntile, int nbh, int& rank, int& bh) {
+__device__ __forceinline__ void xcd_tile_map(int wid, int ntile, int nbh, int& rank, int& bh, bool turn = true) {
   constexpr int kXcd = 8, kCus = 32;
   if constexpr (ROUNDS > 1) {
     const int xcd = wid % kXcd, local = wid / kXcd, round = local / kCus;
-    if (round < ROUNDS && (round & 1) && (round + 1) * kCus * kXcd <= ntile * nbh)
+    if (turn && round < ROUNDS && (round & 1) && (round + 1) * kCus * kXcd <= ntile * nbh)
       wid = ((2 * round + 1) * kCus - 1 - local) * kXcd + xcd;
   }
   if (nbh % kXcd == 0) {

@@ -1425,6 +1425,28 @@ def test_every_tile_is_visited_whatever_the_workgroup_order(dev, H, L, D):
             assert torch.equal(a[:, h:h + 1], b)
 
 
+@pytest.mark.parametrize("numerics", ["parity", "fast"])
+@pytest.mark.parametrize("listed", [False, True], ids=["unmasked", "window"])
+@pytest.mark.parametrize("D", [64, 128])
+def test_table_calls_visit_every_tile_with_and_without_lists(dev, D, listed, numerics):
+    """Under a multiplicative table only calls with tile lists turn the second round of workgroups (544 tiles here; the fourth round
+    of the log-sum-exp pass needs 1024: 1088 at the larger head count); a head by itself has no second round."""
+    from flaxattention_amd import _lib
+    from flaxattention_amd.core.common import ScoreMod
+    for H in (32, 64):
+        print("case table order", D, listed, numerics, H, flush=True)
+        L = 2100
+        q, k, v = (t.to(dev) for t in seeded_qkv(1, H, H, L, L, D, torch.bfloat16))
+        table = torch.randn(1, 1, L, L, generator=torch.Generator().manual_seed(5)).to(dev)
+        mod = ScoreMod(_lib.SCORE_AFFINE, name="tables", mul=1 + table / 8, add=table)
+        bm = fa.create_block_mask(generate_sliding_window(300), None, None, L, L, device=dev) if listed else None
+        opts = {"split_kv": False, "numerics": numerics}
+        whole = fa.flax_attention(q, k, v, score_mod=mod, block_mask=bm, kernel_options=opts)
+        for h in (0, H // 2, H - 1):
+            one = fa.flax_attention(*(t[:, h:h + 1].contiguous() for t in (q, k, v)), score_mod=mod, block_mask=bm, kernel_options=opts)
+            assert torch.equal(whole[:, h:h + 1], one)
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["f16", "bf16"])
 @pytest.mark.parametrize("scale", [-0.1, 0.0, 0.05, 1.7])
 @pytest.mark.parametrize("D,Hq,Hkv,Lq,Lkv", [(64, 4, 2, 300, 333), (128, 3, 3, 130, 260), (128, 16, 4, 2048, 2048), (192, 2, 1, 129, 200)])
