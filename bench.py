@@ -51,11 +51,11 @@ PEAK_HBM_GBPS = 8000.0
 # cannot outlive the code it describes.
 TRAFFIC_SOURCE = "profiles/hbm_traffic_config2_and_decode_pmc.md"
 TRAFFIC_KERNEL_FILES = ("fwd_mfma.cuh", "bwd_mfma.cuh", "mfma_common.cuh")
-TRAFFIC_KERNEL_SHA = "79abf2207f8abdd7"
+TRAFFIC_KERNEL_SHA = "b8c19459fb0663cd"
 MEASURED_TRAFFIC_BYTES = {
     ("config2", "fwd_pipe_kernel"): 67966566,
-    ("config2", "bwd_dq_kernel"): 135914291,
-    ("config2", "bwd_dkv_kernel"): 137351373,
+    ("config2", "bwd_dq_kernel"): 136035533,
+    ("config2", "bwd_dkv_kernel"): 137456742,
 }
 
 
